@@ -390,10 +390,22 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     // the row kernels' static LDS (bin walk table) comes on top of the row
     const size_t rb = (size_t)(fftc::padded_size(rpw * g.nf1) + fftc::twiddle_entries(g.nf1)) * cs;
     const size_t cb = (size_t)(fftc::padded_size(cpw * g.nf2) + fftc::twiddle_entries(g.nf2)) * cs;
-    // a row part of a row split kRowSplit ways (256 threads at most)
-    const size_t rbp = (size_t)(fftc::padded_size(g.nf1 / kRowSplit) + fftc::twiddle_entries(g.nf1)) * cs;
+    // A row part of a row split `split` ways (256 threads at most): FP32 rows
+    // of 8192 in two parts of 4096, the length of the register-resident
+    // plane-loop row kernels, all others kRowSplit ways.  Halves against whole
+    // rows: 4 channels of 4096^2 (90 planes, ~80 record visits per row and
+    // plane) 5.1 against 8.1 ms per launch (ms2dirty), a dirty2ms call 115
+    // against 153 ms.  Each part adds its own share of every visit to the
+    // record's accumulator, so dirty2ms keeps dense rows whole: the one plane of
+    // a 20M-point 2-D transform (15,000 visits per row) took 6.8 ms in halves
+    // against 3.4; equal near 1,000 visits.  ms2dirty has halves ahead there
+    // too (5.8 against 7.3 ms: integer LDS atomics).
+    const double visits = (double)nrow_valid * g.kw * g.kww / ((double)g.P * g.nf2);
+    const bool halves = !dbl && g.nf1 == 8192 && !tn.compact && (!tn.to_vis || visits <= 1024);
+    const int split = halves ? 2 : kRowSplit;
+    const size_t rbp = (size_t)(fftc::padded_size(g.nf1 / split) + fftc::twiddle_entries(g.nf1)) * cs;
     const bool row_whole = rb + 2048 <= lds_max && rpw * g.nf1 / 16 <= max_threads;
-    const bool row_split = rpw == 1 && g.nf1 >= 4096 && g.nf1 / kRowSplit <= 16 * 256 && rbp + 2048 <= lds_max / 2;
+    const bool row_split = rpw == 1 && g.nf1 >= 4096 && g.nf1 / split <= 16 * 256 && rbp + 2048 <= lds_max / 2;
     const bool col_whole = cb <= lds_max && cpw * g.nf2 / 16 <= max_threads;
     // columns of 16384 held in registers (FP64: exchanged through LDS one
     // component at a time; FP32: the first and last stages in registers)
@@ -423,11 +435,11 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
           break;
         }
       }
-      // rows too long for two workgroups per CU run split kRowSplit ways
-      if (!row_whole || (rpw == 1 && rb + 2048 > lds_max / 2 && g.nf1 >= 4096)) {
-        g.rsplit = kRowSplit;
+      // rows too long for two workgroups per CU run split, and FP32 rows of 8192
+      if (!row_whole || (rpw == 1 && rb + 2048 > lds_max / 2 && g.nf1 >= 4096) || (halves && row_split)) {
+        g.rsplit = split;
         g.nslot = g.nf1 / 2;
-        g.slot_lg = 31 - __builtin_clz(g.nf1 / (2 * kRowSplit));
+        g.slot_lg = 31 - __builtin_clz(g.nf1 / (2 * split));
         g.lds_rowp_bytes = (int)rbp;
       }
       g.nct = (g.nslot + kTile - 1) / kTile;
@@ -496,7 +508,7 @@ int device_lds_bytes() {
 
 
 // Phase 1 (one wait): w range and unflagged count of every problem, then their geometries.
-int plan_all(const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int dev, std::vector<ChanPlan> &cps) {
+int plan_all(bool to_image, const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int dev, std::vector<ChanPlan> &cps) {
   std::vector<int> nbm(n), base(n + 1, 0);
   for (int i = 0; i < n; ++i) {
     nbm[i] = pbs[i].nrow > 0 ? std::min(nblocks(pbs[i].nrow), 1024) : 0;
@@ -521,6 +533,7 @@ int plan_all(const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int 
   CURIG_HIP(hipStreamSynchronize(st));
   Tuning tn = tune ? *tune : Tuning();
   if (tn.lds_bytes <= 0) tn.lds_bytes = device_lds_bytes();
+  tn.to_vis = to_image ? 0 : 1;
   cps.assign(n, ChanPlan());
   for (int i = 0; i < n; ++i) {
     double wmin = INFINITY, wmax = -INFINITY;
@@ -680,9 +693,11 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image,
     CURIG_TRY(twiddles<T>(dev, g0, st, t1, t2));
     b.tw1 = t1;
     b.tw2 = t2;
-    CURIG_TRY(allow_spread_rows<T>(g0));
-    CURIG_TRY(allow_row_interp<T>(g0));
-    CURIG_TRY(allow_cols<T>(g0));
+    // channels may differ in how their rows are split
+    for (const ChanPlan &cp : cps) {
+      CURIG_TRY(to_image ? allow_spread_rows<T>(cp.g) : allow_row_interp<T>(cp.g));
+      CURIG_TRY(allow_cols<T>(cp.g));
+    }
   } else {
     // create every FFT plan the batches will use (full and tail batches, split
     // into chunks of at most kMaxFftElems elements) and size the work buffer
@@ -945,7 +960,7 @@ template <typename T>
 int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int graph_mode,
                Stats *sts, int dev) {
   std::vector<ChanPlan> cps;
-  CURIG_TRY(plan_all(pbs, n, st, tune, dev, cps));
+  CURIG_TRY(plan_all(to_image, pbs, n, st, tune, dev, cps));
   Bufs b;
   if (g_arena) {
     // no-allocation call: the LDS FFT path only (rocFFT plans allocate), and
@@ -1093,8 +1108,10 @@ int ms2dirty_device_noalloc(const Problem &pb, hipStream_t st, const Tuning *tun
   ar.base = base;
   ar.cap = kScratchBytes;
   g_arena = &ar;
-  const int ier = pb.dbl ? run_locked<double>(true, &pb, 1, st, tune, 0, nullptr, dev)
-                         : run_locked<float>(true, &pb, 1, st, tune, 0, nullptr, dev);
+  Tuning tn = tune ? *tune : Tuning();
+  tn.compact = 1;  // the layouts with the smallest working set
+  const int ier = pb.dbl ? run_locked<double>(true, &pb, 1, st, &tn, 0, nullptr, dev)
+                         : run_locked<float>(true, &pb, 1, st, &tn, 0, nullptr, dev);
   g_arena = nullptr;
   const int ierm = ws_mark(dev, st);
   return ier != kOk ? ier : ierm;

@@ -3,6 +3,8 @@
 // (kern_lds_{spread,interp,cols}_{f32,f64}.hip), each of which instantiates
 // its launchers.
 #pragma once
+#include <type_traits>
+
 #include "dev_common.h"
 #include "trig.h"
 
@@ -1652,17 +1654,28 @@ template <typename T> inline bool whole_row_planes(const Geom &g) {
   return g.rsplit == 0 && g.rpw == 1 && g.nf1 == 4096;
 }
 
+// f(std::integral_constant<int, S>) for the splits a plan chooses: kRowSplit,
+// and 2 for FP32 rows of 8192
+template <typename T, typename F> inline void with_split(int S, F f) {
+  if constexpr (sizeof(T) == 4 && kRowSplit != 2) {
+    if (S == 2) return f(std::integral_constant<int, 2>());
+  }
+  f(std::integral_constant<int, kRowSplit>());
+}
+
 // ms2dirty, one batch on the LDS path: spread + row FFT -> H (column-tiled)
 template <typename T>
 void lds_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const Geom &g, int p0, int nb, cpx<T> *H,
                      const cpx<T> *tw1, hipStream_t st) {
-  if (g.rsplit == kRowSplit) {
-    const int nt = g.nf1 / (16 * kRowSplit), grd = kRowSplit * g.nf2;
+  if (g.rsplit > 1) {
+    const int nt = g.nf1 / (16 * g.rsplit), grd = g.rsplit * g.nf2;
     const int lb = g.lds_rowp_bytes;
-    if (g.kw <= 8)
-      spread_row_part_planes_kernel<T, 16, 8, kRowSplit><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
-    else
-      spread_row_part_planes_kernel<T, 16, 16, kRowSplit><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
+    with_split<T>(g.rsplit, [&](auto S) {
+      if (g.kw <= 8)
+        spread_row_part_planes_kernel<T, 16, 8, S.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
+      else
+        spread_row_part_planes_kernel<T, 16, 16, S.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
+    });
     return;
   }
   if (whole_row_planes<T>(g)) {
@@ -1691,10 +1704,14 @@ int allow_spread_rows(const Geom &g) {
     CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 8, 1>, lb)));
     CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 16, 1>, lb)));
   }
-  if (g.rsplit == kRowSplit) {
+  if (g.rsplit > 1) {
     const int lb = g.lds_rowp_bytes;
-    CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 8, kRowSplit>, lb)));
-    CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 16, kRowSplit>, lb)));
+    int ier = kOk;
+    with_split<T>(g.rsplit, [&](auto S) {
+      ier = allow_lds(spread_row_part_planes_kernel<T, 16, 8, S.value>, lb);
+      if (ier == kOk) ier = allow_lds(spread_row_part_planes_kernel<T, 16, 16, S.value>, lb);
+    });
+    CURIG_TRY(ier);
   }
   return kOk;
 }
@@ -1702,7 +1719,7 @@ int allow_spread_rows(const Geom &g) {
 // rows (rsplit 0) or row parts (rsplit kRowSplit) of 4096 points (FP64:
 // 173 VGPRs at the two workgroups per CU that its LDS allows)
 template <typename T> inline bool interp_planes(const Geom &g) {
-  return (g.rsplit == 0 && g.rpw == 1 && g.nf1 == 4096) || (g.rsplit == kRowSplit && g.nf1 / kRowSplit == 4096);
+  return (g.rsplit == 0 && g.rpw == 1 && g.nf1 == 4096) || (g.rsplit > 1 && g.nf1 / g.rsplit == 4096);
 }
 
 // dirty2ms, one batch on the LDS path: inverse row FFT fused with the interpolation
@@ -1711,24 +1728,24 @@ void lds_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx
                     const cpx<T> *tw1, const Geom &g, int p0, int nb, hipStream_t st) {
   if (interp_planes<T>(g)) {
     // rows or row parts of 4096: one workgroup per (row, part) walks the batch's planes
-    const int S = g.rsplit == kRowSplit ? kRowSplit : 1;
-    const int lb = S == 1 ? g.lds_row_bytes : g.lds_rowp_bytes, grd = S * g.nf2;
-    if (S == 1) {
+    const bool s1 = g.rsplit <= 1;
+    const int lb = s1 ? g.lds_row_bytes : g.lds_rowp_bytes, grd = (s1 ? 1 : g.rsplit) * g.nf2;
+    auto go = [&](auto S) {
       if (g.kw <= 8)
-        row_ifft_interp_part_planes_kernel<T, 8, 1><<<grd, 256, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, nb, -1);
+        row_ifft_interp_part_planes_kernel<T, 8, S.value><<<grd, 256, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, nb,
+                                                                              -1);
       else
-        row_ifft_interp_part_planes_kernel<T, 16, 1><<<grd, 256, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, nb, -1);
-    } else {
-      if (g.kw <= 8)
-        row_ifft_interp_part_planes_kernel<T, 8, kRowSplit><<<grd, 256, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, nb,
-                                                                                -1);
-      else
-        row_ifft_interp_part_planes_kernel<T, 16, kRowSplit><<<grd, 256, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0,
-                                                                                 nb, -1);
-    }
+        row_ifft_interp_part_planes_kernel<T, 16, S.value><<<grd, 256, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, nb,
+                                                                               -1);
+    };
+    if (s1)
+      go(std::integral_constant<int, 1>());
+    else
+      with_split<T>(g.rsplit, go);
     return;
   }
-  if (g.rsplit == kRowSplit) {
+  if (g.rsplit > 1) {
+    // parts of other lengths (FP64 rows of 8192): kRowSplit ways
     const dim3 grd(kRowSplit * g.nf2, nb);
     const int nt = g.nf1 / (16 * kRowSplit), lb = g.lds_rowp_bytes;
     if (g.kw <= 8)
@@ -1749,17 +1766,22 @@ template <typename T>
 int allow_row_interp(const Geom &g) {
   CURIG_TRY(allow_lds(row_ifft_interp_kernel<T, 16, 8>, g.lds_row_bytes));
   CURIG_TRY(allow_lds(row_ifft_interp_kernel<T, 16, 16>, g.lds_row_bytes));
-  if (g.rsplit == kRowSplit) {
+  if (interp_planes<T>(g)) {
+    const bool s1 = g.rsplit <= 1;
+    const int lb = s1 ? g.lds_row_bytes : g.lds_rowp_bytes;
+    int ier = kOk;
+    auto go = [&](auto S) {
+      ier = allow_lds(row_ifft_interp_part_planes_kernel<T, 8, S.value>, lb);
+      if (ier == kOk) ier = allow_lds(row_ifft_interp_part_planes_kernel<T, 16, S.value>, lb);
+    };
+    if (s1)
+      go(std::integral_constant<int, 1>());
+    else
+      with_split<T>(g.rsplit, go);
+    CURIG_TRY(ier);
+  } else if (g.rsplit > 1) {
     CURIG_TRY((allow_lds(row_ifft_interp_part_kernel<T, 16, 8, kRowSplit>, g.lds_rowp_bytes)));
     CURIG_TRY((allow_lds(row_ifft_interp_part_kernel<T, 16, 16, kRowSplit>, g.lds_rowp_bytes)));
-  }
-  if (interp_planes<T>(g)) {
-    const bool s1 = g.rsplit != kRowSplit;
-    const int lb = s1 ? g.lds_row_bytes : g.lds_rowp_bytes;
-    CURIG_TRY((allow_lds(row_ifft_interp_part_planes_kernel<T, 8, 1>, lb)));
-    CURIG_TRY((allow_lds(row_ifft_interp_part_planes_kernel<T, 16, 1>, lb)));
-    CURIG_TRY((allow_lds(row_ifft_interp_part_planes_kernel<T, 8, kRowSplit>, lb)));
-    CURIG_TRY((allow_lds(row_ifft_interp_part_planes_kernel<T, 16, kRowSplit>, lb)));
   }
   return kOk;
 }
