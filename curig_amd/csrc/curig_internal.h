@@ -99,16 +99,17 @@ struct Geom {
   int rpw;            // grid rows per workgroup in the row pass (rpw * nf1 = 16 * threads)
   int cpw;            // grid columns per workgroup in the column pass (cpw * nf2 = 16 * threads)
   int cpw_inv;        // the same for the dirty2ms column pass (whole column tiles where they fit)
-  int lds_coli_bytes; // its LDS
+  int pch_fwd, pch_inv;  // planes per workgroup of the column passes (>= Pb: one workgroup walks the whole batch)
+  int nacc;           // ms2dirty accumulators: one per plane chunk of a batch, summed by the epilogue
   int nct;            // column tiles of a plane's row-transformed layout (nslot / kTile, rounded up)
   int tstride;        // elements from one column tile to the next: nf2 * kTile + a pad
   int nslot;          // column slots of that layout: N1, or nf1 / 2 with split rows
   int slot_lg;        // split rows: log2 of the slots per row part (nf1 / (2 rsplit))
   int lds_row_bytes;  // dynamic LDS of the row-pass workgroup
-  int lds_col_bytes;  // dynamic LDS of the column-pass workgroup
+  int lds_col_bytes;  // dynamic LDS of the workgroup of a 16384-point column
   int rsplit;         // > 1: rows run as rsplit workgroups of nf1 / rsplit (too long for two per CU)
   int lds_rowp_bytes; // dynamic LDS of a row-part workgroup
-  int colreg;         // 1: FP64 columns of 16384, held in registers by 1024 threads (one column slot each)
+  int colreg;         // 1: columns of 16384, held in registers by 1024 threads (one column slot each)
 };
 
 // Column-tile width of the intermediate planes (LDS path, both directions):
@@ -119,6 +120,7 @@ struct Geom {
 #define CURIG_TILE_LOG2 2
 #endif
 constexpr int kTileLog2 = CURIG_TILE_LOG2;
+static_assert(kTileLog2 >= 1 && kTileLog2 <= 2, "2 or 4 columns: the column kernels step rows by multiples of 4");
 // Bytes between consecutive column tiles beyond their nf2 * kTile elements.
 // Without it the tiles of a plane sit 2^k bytes apart and the kTile-column
 // chunks that one row writes (or reads) all fall into the same memory channel.

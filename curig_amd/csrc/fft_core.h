@@ -121,6 +121,29 @@ template <typename T, int R> FC_HD void dft_small(cpx<T> *v, int sign) {
   for (int i = 0; i < R; ++i) v[i] = a[i];
 }
 
+// dft_small<16> after its first radix-2 level: v[r] and v[r + 8] (r < 8) hold
+// x[r] + x[r + 8] and x[r] - x[r + 8]
+template <typename T> FC_HD void dft16_from_pairs(cpx<T> *v, int sign) {
+  cpx<T> a[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) a[bitrev(i, 4)] = v[i];
+#pragma unroll
+  for (int len = 4; len <= 16; len <<= 1) {
+#pragma unroll
+    for (int st = 0; st < 16; st += len) {
+#pragma unroll
+      for (int j = 0; j < len / 2; ++j) {
+        const int t = j * (16 / len);
+        cpx<T> u = a[st + j], w = rot16(a[st + j + len / 2], t, sign);
+        a[st + j] = add(u, w);
+        a[st + j + len / 2] = sub(u, w);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = a[i];
+}
+
 struct Layout {
   int n;            // sequence length (power of 2)
   int count;        // independent sequences
@@ -229,6 +252,10 @@ FC_HD int twiddle_split(int n) {
   return (m + 1) / 2;
 }
 FC_HD int twiddle_entries(int n) { return (n >> twiddle_split(n)) + (1 << twiddle_split(n)); }
+
+// the same as constant expressions
+FC_HD constexpr int twiddle_split_c(int n, int m = 0) { return (1 << m) < n ? twiddle_split_c(n, m + 1) : (m + 1) / 2; }
+FC_HD constexpr int twiddle_entries_c(int n) { return (n >> twiddle_split_c(n)) + (1 << twiddle_split_c(n)); }
 
 // Radices used for a length-n transform: maxr, maxr, ..., then the remainder.
 FC_HD int stage_radix(int n, int Ns, int maxr = 16) { return (Ns * maxr <= n) ? maxr : n / Ns; }

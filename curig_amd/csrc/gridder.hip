@@ -280,12 +280,48 @@ int check_args(const Problem &pb) {
 
 }  // namespace
 
-// FP32 columns of 16384 run the register-resident column kernels as FP64 does
-// (1: yes; 0: the LDS column kernels)
-#ifndef CURIG_COLREG_FP32
-#define CURIG_COLREG_FP32 1
-#endif
-inline bool col_reg_fp32() { return CURIG_COLREG_FP32 != 0; }
+// Columns and planes per workgroup of the column passes.
+static void plan_columns(Geom &g, size_t cs, size_t lds_max, bool compact) {
+  g.pch_fwd = g.pch_inv = g.Pb;
+  if (g.colreg) {
+    g.cpw = g.cpw_inv = 1;
+    // the inverse pass in short launches' worth of planes: its workgroups, one
+    // column each, share lines of H in fours, and the further they drift apart
+    // over the planes the more partial lines the L2 writes back (8192^2, 32
+    // planes: 19.9 ms walking all planes, 17.7, 13.9 and 16.1 ms in chunks of 8,
+    // 4 and 2; a chunk's setup costs about one plane)
+    g.pch_inv = std::min(4, g.Pb);
+    g.lds_col_bytes = (int)colreg_lds_bytes(cs);
+    return;
+  }
+  const int G = g.nf2 / 16;  // threads per column
+  // 256 threads, or fewer (one wavefront at least) while that leaves fewer than
+  // kFill workgroups
+  constexpr int kFill = 1024;
+  int c = std::max(1, 256 / G);
+  while (c > 1 && (c / 2) * G >= 64 && (g.nslot + c - 1) / c < kFill) c /= 2;
+  g.cpw = g.cpw_inv = c;
+  if (cs == 16 && g.nf2 == 4096) g.cpw = 2;
+  // the dirty2ms column pass writes H: workgroups of fewer than kTile columns
+  // leave each chunk to several workgroups, which reach a plane at different
+  // times, and the L2 then writes the chunk's lines back more than once (2.4x
+  // the bytes at 4096^2); with whole tiles, else half tiles, a workgroup's
+  // lanes write whole chunks or halves (1.0x)
+  const int top = cs == 8 ? 1024 : 512;
+  for (int t = kTile; t >= 2 && g.cpw_inv < t; t /= 2)
+    if (t * G <= std::min(top, std::max(256, 4 * G)) && (size_t)t * (g.nf2 + g.nf2 / 16 + 16) * cs + 9216 <= lds_max)
+      g.cpw_inv = t;
+  // Few columns leave the chip idle: the batch's planes are then walked by
+  // several workgroups (a 256^2 image, 16 planes of 512: 128 workgroups of one
+  // wavefront for all planes), each ms2dirty chunk with its own accumulator.
+  auto chunk = [&](int groups) {
+    const int n = std::min((kFill + groups - 1) / groups, 8);
+    return std::max(std::min(2, g.Pb), (g.Pb + n - 1) / n);
+  };
+  g.pch_inv = chunk((g.nslot + g.cpw_inv - 1) / g.cpw_inv);
+  if (!compact) g.pch_fwd = chunk((g.nslot + g.cpw - 1) / g.cpw);
+  g.nacc = (g.Pb + g.pch_fwd - 1) / g.pch_fwd;
+}
 
 int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, double eps, double sigma, int sign,
                   double wmin_m, double wmax_m, bool dbl, const Tuning *tune, Geom *gp, KernelOpts *kop,
@@ -378,7 +414,8 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   // workgroup's LDS, with the image at most half the grid on each axis
   g.fft_lds = 0;
   g.rpw = g.cpw = g.nct = g.tstride = g.nslot = g.slot_lg = g.lds_row_bytes = g.lds_col_bytes = g.rsplit =
-      g.lds_rowp_bytes = g.colreg = g.cpw_inv = g.lds_coli_bytes = 0;
+      g.lds_rowp_bytes = g.colreg = g.cpw_inv = g.pch_fwd = g.pch_inv = 0;
+  g.nacc = 1;
   auto pow2 = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
   const size_t cs = dbl ? 16 : 8;
   const size_t lds_max = tn.lds_bytes > 0 ? (size_t)tn.lds_bytes : size_t(160) << 10;
@@ -386,10 +423,9 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   if (tn.fft != 1 && g.kw <= 16 && pow2(g.nf1) && pow2(g.nf2) && g.nf1 >= 64 && g.nf2 >= 64 && g.nf1 <= 16384 &&
       g.nf2 <= 16384 && 2 * g.N1 <= g.nf1 && 2 * g.N2 <= g.nf2) {
     const int rpw = std::max(1, std::min(4096 / g.nf1, g.nf2));
-    const int cpw = std::max(1, std::min(4096 / g.nf2, 16));
     // the row kernels' static LDS (bin walk table) comes on top of the row
     const size_t rb = (size_t)(fftc::padded_size(rpw * g.nf1) + fftc::twiddle_entries(g.nf1)) * cs;
-    const size_t cb = (size_t)(fftc::padded_size(cpw * g.nf2) + fftc::twiddle_entries(g.nf2)) * cs;
+    const size_t cb = (size_t)(g.nf2 + g.nf2 / 16 + 16) * cs + 4096;  // one column, its twiddle table
     // A row part of a row split `split` ways (256 threads at most): FP32 rows
     // of 8192 in two parts of 4096, the length of the register-resident
     // plane-loop row kernels, all others kRowSplit ways.  Halves against whole
@@ -406,35 +442,17 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     const size_t rbp = (size_t)(fftc::padded_size(g.nf1 / split) + fftc::twiddle_entries(g.nf1)) * cs;
     const bool row_whole = rb + 2048 <= lds_max && rpw * g.nf1 / 16 <= max_threads;
     const bool row_split = rpw == 1 && g.nf1 >= 4096 && g.nf1 / split <= 16 * 256 && rbp + 2048 <= lds_max / 2;
-    const bool col_whole = cb <= lds_max && cpw * g.nf2 / 16 <= max_threads;
+    const bool col_whole = g.nf2 <= 8192 && cb <= lds_max && g.nf2 / 16 <= max_threads;
     // columns of 16384 held in registers (FP64: exchanged through LDS one
     // component at a time; FP32: the first and last stages in registers)
     const size_t cbr = colreg_lds_bytes(cs);
-    const bool col_reg = g.nf2 == 16384 && cbr <= lds_max && (dbl || col_reg_fp32());
-    if ((row_whole || row_split) && (col_whole || col_reg) && rpw * g.nf1 >= 16 * 64 && cpw * g.nf2 >= 16) {
+    const bool col_reg = g.nf2 == 16384 && cbr <= lds_max;
+    if ((row_whole || row_split) && (col_whole || col_reg) && rpw * g.nf1 >= 16 * 64) {
       g.fft_lds = 1;
       g.rpw = rpw;
       g.colreg = col_reg ? 1 : 0;
-      g.cpw = col_reg ? 1 : cpw;
       g.nslot = g.N1;
       g.lds_row_bytes = row_whole ? (int)rb : 0;
-      g.lds_col_bytes = (int)(col_reg ? cbr : cb);
-      // the dirty2ms column pass writes H: FP32 workgroups of fewer than
-      // kTile columns leave each 32-byte chunk to several workgroups, which
-      // reach a plane at different times, and the L2 then writes the chunk's
-      // lines back more than once (2.4x the bytes at 4096^2); with whole tiles
-      // a workgroup writes whole chunks (1.0x)
-      g.cpw_inv = g.cpw;
-      g.lds_coli_bytes = g.lds_col_bytes;
-      for (int c = kTile; !dbl && !col_reg && cpw < c && c >= 2; c /= 2) {
-        // whole tiles, else half tiles (16-byte pieces of a chunk)
-        const size_t cbi = (size_t)(fftc::padded_size(c * g.nf2) + fftc::twiddle_entries(g.nf2)) * cs;
-        if (cbi <= lds_max && c * g.nf2 / 16 <= max_threads) {
-          g.cpw_inv = c;
-          g.lds_coli_bytes = (int)cbi;
-          break;
-        }
-      }
       // rows too long for two workgroups per CU run split, and FP32 rows of 8192
       if (!row_whole || (rpw == 1 && rb + 2048 > lds_max / 2 && g.nf1 >= 4096) || (halves && row_split)) {
         g.rsplit = split;
@@ -457,6 +475,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   }
   g.Pb = std::max(1, std::min(Pb, g.P));
   g.nbatch = (g.P + g.Pb - 1) / g.Pb;
+  if (g.fft_lds) plan_columns(g, cs, lds_max, tn.compact != 0);
   // bins: full-width row strips for the LDS path (one workgroup owns grid rows),
   // T1 x T2 tiles for the tile-owner spread
   if (g.fft_lds) {
@@ -636,7 +655,7 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image,
     const size_t plane = (size_t)g.nf1 * g.nf2, pix = (size_t)g.N1 * g.N2;
     if (!g.fft_lds) grid = std::max(grid, plane * g.Pb);
     if (g.fft_lds) h = std::max(h, (size_t)g.nct * g.tstride * g.Pb);
-    npix = std::max(npix, pix);
+    npix = std::max(npix, pix * (to_image ? g.nacc : 1));
   }
   void *vp;
   CURIG_TRY(ws_get(dev, S_HIST, sizeof(int) * nbins, &vp));
@@ -938,7 +957,7 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.lds_coli_bytes << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
+      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
   k << b.dev << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc

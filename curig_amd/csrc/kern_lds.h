@@ -541,6 +541,18 @@ __device__ __forceinline__ int h_slot(const Geom &g, int s) {
   return (s >> kTileLog2) * g.tstride + (s & (kTile - 1));
 }
 
+// dirty2ms stores each block of kTile rows x kTile slots column by column
+// (ms2dirty: row by row): the column pass writes there, and kTile lanes of
+// consecutive rows then fill a whole 32-byte (FP64: 64-byte) sector in one
+// store (FP64 columns of 4096: 1.25 -> 0.76 ms per 30 planes of 2048 columns).
+// Blocks of 8 rows (64 bytes in FP32) halved the writes' time again but cost
+// the row pass, which reads 8 bytes of each piece, more (columns of 16384: 10.4
+// against 13.3 ms per 32 planes, rows 22.9 against 14.1 ms).
+__device__ __forceinline__ int ht_row(int k2) { return ((k2 & ~(kTile - 1)) << kTileLog2) + (k2 & (kTile - 1)); }
+__device__ __forceinline__ int ht_slot(const Geom &g, int s) {
+  return (s >> kTileLog2) * g.tstride + ((s & (kTile - 1)) << kTileLog2);
+}
+
 // Column slots of the tiled layout.  With whole rows the slot of image column
 // col is col.  With rows split S ways, the columns of part h (grid index h mod
 // S, col = S i + c_h with c_h = (h + N1/2) mod S) take slots h M + i, M = nf1 /
@@ -552,13 +564,6 @@ __device__ __forceinline__ int slot_column(int s, const Geom &g) {
   const int S = g.rsplit, h = s >> g.slot_lg, i = s & ((1 << g.slot_lg) - 1);
   const int col = S * i + ((h + g.N1 / 2) & (S - 1));
   return col < g.N1 ? col : -1;
-}
-
-// whether a column workgroup's slots [s0, s0 + cpw) hold any image column
-__device__ __forceinline__ bool slots_used(int s0, const Geom &g, int cpw) {
-  for (int c = 0; c < cpw; ++c)
-    if (slot_column(s0 + c, g) >= 0) return true;
-  return false;
 }
 
 // Workgroup id -> work item such that each XCD (workgroups are dispatched to
@@ -669,13 +674,13 @@ __global__ void __launch_bounds__(MaxThreads<T>::value) row_ifft_interp_kernel(c
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, pl = blockIdx.y, p = p0 + pl;
   const int lg = 31 - __clz(nf1);
   cpx<T> v[E];
-  const cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
+  const cpx<T> *hb = H + h_plane(g, pl);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int i = threadIdx.x + e * nt;  // < rpw * nf1 = E * nt
     const int r = i >> lg, k1 = i & (nf1 - 1);
     const int col = image_index(k1, N1, nf1);
-    v[e] = col >= 0 ? hb[h_slot(g, col) + (r << kTileLog2)]
+    v[e] = col >= 0 ? hb[ht_slot(g, col) + ht_row(row0 + r)]
                     : fftc::mk((T)0, (T)0);
   }
   const auto tv = lds_twiddles<T>(lds + fftc::padded_size(rpw * nf1), tw, nf1);
@@ -1030,7 +1035,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_kernel(
   const int item = xcd_group(blockIdx.x, gridDim.x);
   const int row0 = item / S, h = item % S, pl = blockIdx.y, p = p0 + pl;
   const int lgm = 31 - __clz(m);
-  const cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
+  const cpx<T> *hb = H + h_plane(g, pl) + ht_row(row0);
   // Input e of this thread is X[S i + h], i = tid + e nt (< m = E nt).  With
   // N1 <= nf1 / 2 only the first and last quarter of i can be image columns
   // (grid indices within N1 / 2 of 0); their column slots are
@@ -1038,7 +1043,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_kernel(
   // q = (h + N1 / 2) / S, so their addresses step by (nt / kTile) tiles.
   const int tid = threadIdx.x, h1 = N1 / 2, q = (h + h1) / S;
   const int k0 = S * tid + h + h1;  // column of e = 0 before the fold
-  const cpx<T> *a0 = hb + h_slot(g, (h << g.slot_lg) + tid + q);
+  const cpx<T> *a0 = hb + ht_slot(g, (h << g.slot_lg) + tid + q);
   const long estep = (long)(nt >> kTileLog2) * g.tstride, mstep = (long)(m >> kTileLog2) * g.tstride;
   cpx<T> v[E];
 #pragma unroll
@@ -1125,7 +1130,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_planes_kernel(
   // last quarters can be image columns (as in row_ifft_interp_part_kernel)
   const int h1 = N1 / 2, q = (h + h1) / S, k0 = S * j + h + h1;
   const long estep = (long)(nt >> kTileLog2) * g.tstride, mstep = (long)(m >> kTileLog2) * g.tstride;
-  const long a0off = (long)row0 * kTile + h_slot(g, (h << g.slot_lg) + j + q);
+  const long a0off = (long)ht_row(row0) + ht_slot(g, (h << g.slot_lg) + j + q);
   int cur = 0;
   for (int pl = 0; pl < nb; ++pl, cur ^= 1) {
     const int p = p0 + pl;
@@ -1180,213 +1185,6 @@ __device__ __forceinline__ double pixel_zp(int row, int col, const Geom &g) {
   double nm1, n;
   pixel_n(row, col, g, nm1, n);
   return (nm1 - g.D) * g.gamma * g.h;
-}
-
-// ms2dirty column pass fused with the w-accumulation (w_term_dft, cuft.cu:520-572):
-// a workgroup owns cpw grid columns (cpw * nf2 = E * blockDim.x) and walks the
-// batch's nb planes: load the row-transformed columns, FFT over nf2, then for
-// the N2 image rows accT[col][row] += F_p e^{+i z' (p - P/2)}: the phase
-// argument and its reduction in FP64 (sin / cos of the reduced argument at the
-// planes' precision) and the sum over planes in FP64 registers.  Image rows per thread:
-// cpw * N2 <= 8 * blockDim.x (the plan requires 2 N2 <= nf2).
-template <typename T, int E>
-__global__ void __launch_bounds__(MaxThreads<T>::value) col_fwd_kernel(const cpx<T> *__restrict__ H,
-                                                                      double2 *__restrict__ accT,
-                                                                      const cpx<T> *__restrict__ tw, Geom g,
-                                                                      int p0, int nb, int first) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
-  const int cpw = g.cpw, nf2 = g.nf2, N2 = g.N2, nt = blockDim.x;
-  const int s0 = xcd_group(blockIdx.x, gridDim.x) * cpw;  // first column slot
-  if (!slots_used(s0, g, cpw)) return;
-  const int lg = 31 - __clz(nf2);
-  const int nout = cpw * N2;
-  double ar[8], ai[8], zp[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    ar[e] = ai[e] = zp[e] = 0.0;
-    const int o = threadIdx.x + e * nt;
-    if (o < nout) {
-      const int ci = o / N2, row = o - ci * N2, col = slot_column(s0 + ci, g);
-      if (col >= 0) zp[e] = pixel_zp(row, col, g);
-    }
-  }
-  const auto tv = lds_twiddles<T>(lds + fftc::padded_size(cpw * nf2), tw, nf2);
-  for (int k = 0; k < nb; ++k) {
-    // opaque copy of the thread id: the per-plane addresses are formed inside
-    // the loop rather than held in registers across it
-    int tid = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid));
-    const cpx<T> *hk = H + h_plane(g, k);
-    cpx<T> v[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int i = tid + e * nt;
-      const int ci = i >> lg, k2 = i & (nf2 - 1), sl = s0 + ci;
-      v[e] = slot_column(sl, g) >= 0 ? hk[h_slot(g, sl) + (k2 << kTileLog2)]
-                                     : fftc::mk((T)0, (T)0);
-    }
-    __syncthreads();  // the previous plane's LDS reads are done
-#pragma unroll
-    for (int e = 0; e < E; ++e) lds[fftc::pad(tid + e * nt)] = v[e];
-    __syncthreads();
-    lds_fft_rows<T, E, 16>(lds, lg, cpw, +1, tv);
-    const double m = (double)(p0 + k - g.P / 2);
-    int tid2 = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid2));
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int o = tid2 + e * nt;
-      if (o < nout) {
-        const int ci = o / N2, row = o - ci * N2;
-        const cpx<T> f = lds[fftc::pad(ci * nf2 + grid_index(row, N2, nf2))];
-        double sn, cs;
-        plane_phase<T>(zp[e] * m, &sn, &cs);
-        const double fr = (double)f.x, fi = (double)f.y;
-        ar[e] += fr * cs - fi * sn;
-        ai[e] += fr * sn + fi * cs;
-      }
-      // one element's phase at a time (bounds the live FP64 temporaries)
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int o = threadIdx.x + e * nt;
-    if (o < nout) {
-      const int ci = o / N2, row = o - ci * N2, col = slot_column(s0 + ci, g);
-      if (col >= 0) {
-        const size_t a = (size_t)col * N2 + row;
-        double2 r = make_double2(ar[e], ai[e]);
-        if (!first) {
-          const double2 q = accT[a];
-          r.x += q.x;
-          r.y += q.y;
-        }
-        accT[a] = r;
-      }
-    }
-  }
-}
-
-// dirty2ms column pass fused with the w-fill (w_term_idft, cuft.cu:575-612): a
-// workgroup owns cpw grid columns and, for each of the batch's nb planes, places
-// gT[col][row] e^{-i z' (p - P/2)} (FP64 phase argument) at the image rows of its columns
-// (zeros elsewhere), runs the inverse FFT over nf2 and writes the full columns
-// to the column-tiled H.
-template <typename T, int E>
-__global__ void __launch_bounds__(MaxThreads<T>::value) col_inv_kernel(const cpx<T> *__restrict__ gT,
-                                                                      cpx<T> *__restrict__ H,
-                                                                      const cpx<T> *__restrict__ tw, Geom g,
-                                                                      int p0, int nb) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
-  const int cpw = g.cpw_inv, nf2 = g.nf2, N2 = g.N2, nt = blockDim.x;
-  const int s0 = xcd_group(blockIdx.x, gridDim.x) * cpw;  // first column slot
-  if (!slots_used(s0, g, cpw)) return;
-  const int lg = 31 - __clz(nf2);
-  const int nout = cpw * N2, nzero = cpw * (nf2 - N2), h2 = N2 / 2;
-  bool full = true;  // every column slot of the workgroup holds an image column
-  for (int c = 0; c < cpw; ++c) full = full && slot_column(s0 + c, g) >= 0;
-  cpx<T> gv[8];
-  double zp[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    gv[e] = fftc::mk((T)0, (T)0);
-    zp[e] = 0.0;
-    const int o = threadIdx.x + e * nt;
-    if (o < nout) {
-      const int ci = o / N2, row = o - ci * N2, col = slot_column(s0 + ci, g);
-      if (col >= 0) {
-        gv[e] = gT[(size_t)col * N2 + row];
-        zp[e] = pixel_zp(row, col, g);
-      }
-    }
-  }
-  const auto tv = lds_twiddles<T>(lds + fftc::padded_size(cpw * nf2), tw, nf2);
-  for (int k = 0; k < nb; ++k) {
-    const double m = (double)(p0 + k - g.P / 2);
-    int tid = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid));
-    __syncthreads();  // the previous plane's LDS reads are done
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int o = tid + e * nt;
-      if (o < nout) {
-        const int ci = o / N2, row = o - ci * N2;
-        double sn, cs;
-        plane_phase<T>(-zp[e] * m, &sn, &cs);
-        const double gr = (double)gv[e].x, gi = (double)gv[e].y;
-        lds[fftc::pad(ci * nf2 + grid_index(row, N2, nf2))] =
-            fftc::mk((T)(gr * cs - gi * sn), (T)(gr * sn + gi * cs));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    for (int z = tid; z < nzero; z += nt) {
-      const int ci = z / (nf2 - N2), j = z - ci * (nf2 - N2);
-      lds[fftc::pad(ci * nf2 + N2 - h2 + j)] = fftc::mk((T)0, (T)0);
-    }
-    __syncthreads();
-    lds_fft_rows<T, E, 16>(lds, lg, cpw, -1, tv);
-    int tid2 = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid2));
-    cpx<T> *hk = H + h_plane(g, k);
-    if (sizeof(T) == 4 && kTile == 4 && cpw == 2) {
-      // half tiles: thread k2 writes row k2's two columns as one 16-byte piece
-#pragma unroll
-      for (int q = 0; q < E / 2; ++q) {
-        const int k2 = tid2 + q * nt;
-        const cpx<T> a = lds[fftc::pad(k2)], b = lds[fftc::pad(nf2 + k2)];
-        cpx<T> *d = hk + h_slot(g, s0) + (k2 << kTileLog2);
-        if (full) {
-          *reinterpret_cast<float4 *>(d) = make_float4(a.x, a.y, b.x, b.y);
-        } else {
-          if (slot_column(s0, g) >= 0) d[0] = a;
-          if (slot_column(s0 + 1, g) >= 0) d[1] = b;
-        }
-      }
-    } else if (sizeof(T) == 4 && kTile == 4 && cpw % kTile == 0) {
-      // whole column tiles: 16-byte pieces, piece r of tile t holding row
-      // r / 2, columns 2 (r & 1) and 2 (r & 1) + 1 of the tile, so that
-      // consecutive lanes write consecutive 16 bytes of H
-      const int tlg = lg + 1;  // 2 nf2 pieces per tile
-      float4 w[E / 2];
-#pragma unroll
-      for (int q = 0; q < E / 2; ++q) {
-        const int P = tid2 + q * nt, t = P >> tlg, r = P & ((1 << tlg) - 1), c = kTile * t + 2 * (r & 1);
-        const cpx<T> a = lds[fftc::pad(c * nf2 + (r >> 1))], b = lds[fftc::pad((c + 1) * nf2 + (r >> 1))];
-        w[q] = make_float4(a.x, a.y, b.x, b.y);
-      }
-      if (full && cpw == kTile) {
-        // one tile: its pieces are contiguous
-        float4 *d = reinterpret_cast<float4 *>(hk + h_slot(g, s0)) + tid2;
-#pragma unroll
-        for (int q = 0; q < E / 2; ++q) d[q * nt] = w[q];
-      } else {
-#pragma unroll
-        for (int q = 0; q < E / 2; ++q) {
-          const int P = tid2 + q * nt, t = P >> tlg, r = P & ((1 << tlg) - 1), c = kTile * t + 2 * (r & 1);
-          cpx<T> *d = hk + h_slot(g, s0 + kTile * t) + 2 * r;  // 16-byte aligned: tiles start on 32 bytes
-          if (full) {
-            *reinterpret_cast<float4 *>(d) = w[q];
-          } else {
-            if (slot_column(s0 + c, g) >= 0) d[0] = fftc::mk((T)w[q].x, (T)w[q].y);
-            if (slot_column(s0 + c + 1, g) >= 0) d[1] = fftc::mk((T)w[q].z, (T)w[q].w);
-          }
-        }
-      }
-    } else {
-      cpx<T> v[E];
-#pragma unroll
-      for (int e = 0; e < E; ++e) v[e] = lds[fftc::pad(tid2 + e * nt)];
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int i = tid2 + e * nt;
-        const int ci = i >> lg, k2 = i & (nf2 - 1), sl = s0 + ci;
-        if (slot_column(sl, g) >= 0) hk[h_slot(g, sl) + (k2 << kTileLog2)] = v[e];
-      }
-    }
-  }
 }
 
 // --------------------------------------------------------------------------
@@ -1530,38 +1328,54 @@ __global__ void __launch_bounds__(colr::NT) col_fwd_reg_kernel(const cpx<T> *__r
   if (col < 0) return;
   const auto tv = lds_twiddles<T>(reinterpret_cast<cpx<T> *>(buf + colr::buf_scalars<T>()), tw, N);
   // output q of this thread: X[j + 1024 (q mod 4) + 4096 r], r = 0 (q < 4) or 3;
-  // its image row, or -1 (rows and w factors are recomputed per plane: held
-  // across the plane loop they would not fit the registers beside the column)
+  // its image row, or -1 (FP64: rows and w factors are recomputed per plane:
+  // held across the plane loop they would not fit the registers beside the
+  // column)
   auto out_row = [&](int q) { return image_index(colr::opaque_tid() + 1024 * (q & 3) + (q < 4 ? 0 : 3 * 4096), N2, N); };
-  double ar[8], ai[8], zq[8];
+  // FP32: Horner's rule over the planes, last to first (col_fwd_kernel)
+  constexpr bool horner = sizeof(T) == 4;
+  double ar[8], ai[8], er[8], ei[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    ar[q] = ai[q] = 0.0;
-    // FP32 columns leave room to keep the w arguments across the planes
-    const int row = out_row(q);
-    zq[q] = (sizeof(T) == 4 && row >= 0) ? pixel_zp(row, col, g) : 0.0;
+    ar[q] = ai[q] = er[q] = ei[q] = 0.0;
+    if (horner) {
+      const int row = out_row(q);
+      sincos_cw(row >= 0 ? pixel_zp(row, col, g) : 0.0, &ei[q], &er[q]);
+    }
   }
   __syncthreads();
-  const cpx<T> *hs = H + h_slot(g, sl);
-  for (int k = 0; k < nb; ++k) {
-    const cpx<T> *hk = hs + h_plane(g, k);
+  const unsigned off = sizeof(cpx<T>) * (unsigned)(h_slot(g, sl) + (j << kTileLog2));
+  for (int i = 0; i < nb; ++i) {
+    const int k = horner ? nb - 1 - i : i;
+    const cpx<T> *hk = H + h_plane(g, k);
     cpx<T> v[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = hk[(size_t)(j + 1024 * r) << kTileLog2];
+    for (int r = 0; r < 16; ++r)
+      v[r] = *reinterpret_cast<const cpx<T> *>(reinterpret_cast<const char *>(hk + ((1024 * r) << kTileLog2)) + off);
     colr::fft(v, buf, +1, tv);
-    const double m = (double)(p0 + k - g.P / 2);
+    if (horner) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int row = out_row(q);
-      if (row >= 0) {
+      for (int q = 0; q < 8; ++q) {
         const cpx<T> f = v[4 * (q & 3) + (q < 4 ? 0 : 3)];
-        double sn, cs;
-        plane_phase<T>((sizeof(T) == 4 ? zq[q] : pixel_zp(row, col, g)) * m, &sn, &cs);
-        const double fr = (double)f.x, fi = (double)f.y;
-        ar[q] += fr * cs - fi * sn;
-        ai[q] += fr * sn + fi * cs;
+        const double t = ar[q] * er[q] - ai[q] * ei[q] + (double)f.x;
+        ai[q] = ar[q] * ei[q] + ai[q] * er[q] + (double)f.y;
+        ar[q] = t;
       }
-      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      const double m = (double)(p0 + k - g.P / 2);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int row = out_row(q);
+        if (row >= 0) {
+          const cpx<T> f = v[4 * (q & 3) + (q < 4 ? 0 : 3)];
+          double sn, cs;
+          sincos_cw(pixel_zp(row, col, g) * m, &sn, &cs);
+          const double fr = (double)f.x, fi = (double)f.y;
+          ar[q] += fr * cs - fi * sn;
+          ai[q] += fr * sn + fi * cs;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
 #pragma unroll
@@ -1570,6 +1384,11 @@ __global__ void __launch_bounds__(colr::NT) col_fwd_reg_kernel(const cpx<T> *__r
     if (row >= 0) {
       const size_t a = (size_t)col * N2 + row;
       double2 r = make_double2(ar[q], ai[q]);
+      if (horner) {
+        double sn, cs;
+        sincos_cw(pixel_zp(row, col, g) * (double)(p0 - g.P / 2), &sn, &cs);
+        r = make_double2(ar[q] * cs - ai[q] * sn, ar[q] * sn + ai[q] * cs);
+      }
       if (!first) {
         const double2 o = accT[a];
         r.x += o.x;
@@ -1588,7 +1407,7 @@ template <typename T>
 __global__ void __launch_bounds__(colr::NT) col_inv_reg_kernel(const cpx<T> *__restrict__ gT,
                                                                cpx<T> *__restrict__ H,
                                                                const cpx<T> *__restrict__ tw, Geom g, int p0,
-                                                               int nb) {
+                                                               int nb, int pchunk) {
   using colr::N;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *buf = reinterpret_cast<T *>(smem_raw);
@@ -1596,45 +1415,65 @@ __global__ void __launch_bounds__(colr::NT) col_inv_reg_kernel(const cpx<T> *__r
   const int sl = xcd_group(blockIdx.x, gridDim.x);  // column slot
   const int col = slot_column(sl, g);
   if (col < 0) return;
+  const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const auto tv = lds_twiddles<T>(reinterpret_cast<cpx<T> *>(buf + colr::buf_scalars<T>()), tw, N);
   // input q of this thread: x[j + 1024 r], r = q (q < 4) or q + 8; its image
   // row, or -1 (recomputed per plane, as in col_fwd_reg_kernel)
   auto in_row = [&](int q) { return image_index(colr::opaque_tid() + 1024 * (q < 4 ? q : q + 8), N2, N); };
-  // FP32 columns leave room to keep the w arguments and the image values
-  // across the planes
-  constexpr bool keep = sizeof(T) == 4;
-  double zq[8];
-  cpx<T> gq[8];
+  // FP32: the phased image values are carried from plane to plane in FP64
+  // (col_inv_kernel)
+  constexpr bool carry = sizeof(T) == 4;
+  double xr[8], xi[8], er[8], ei[8];
   const cpx<T> *gc = gT + (size_t)col * N2;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
+    xr[q] = xi[q] = er[q] = ei[q] = 0.0;
     const int row = in_row(q);
-    zq[q] = (keep && row >= 0) ? pixel_zp(row, col, g) : 0.0;
-    gq[q] = (keep && row >= 0) ? gc[row] : fftc::mk((T)0, (T)0);
+    if (carry && row >= 0) {
+      const double zp = pixel_zp(row, col, g);
+      double sn, cs;
+      sincos_cw(-zp * (double)(p0 + k0 - g.P / 2), &sn, &cs);
+      const cpx<T> gv = gc[row];
+      xr[q] = (double)gv.x * cs - (double)gv.y * sn;
+      xi[q] = (double)gv.x * sn + (double)gv.y * cs;
+      sincos_cw(-zp, &ei[q], &er[q]);
+    }
   }
   __syncthreads();
-  cpx<T> *hs = H + h_slot(g, sl);
-  for (int k = 0; k < nb; ++k) {
-    const double m = (double)(p0 + k - g.P / 2);
+  const unsigned off = sizeof(cpx<T>) * (unsigned)(ht_slot(g, sl) + ht_row(j));
+  for (int k = k0; k < k1; ++k) {
     cpx<T> v[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) v[r] = fftc::mk((T)0, (T)0);
+    if (carry) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int row = in_row(q);
-      if (row >= 0) {
-        const cpx<T> gv = keep ? gq[q] : gc[row];
-        double sn, cs;
-        plane_phase<T>(-(keep ? zq[q] : pixel_zp(row, col, g)) * m, &sn, &cs);
-        const double gr = (double)gv.x, gi = (double)gv.y;
-        v[q < 4 ? q : q + 8] = fftc::mk((T)(gr * cs - gi * sn), (T)(gr * sn + gi * cs));
+      for (int q = 0; q < 8; ++q) {
+        v[q < 4 ? q : q + 8] = fftc::mk((T)xr[q], (T)xi[q]);
+        const double t = xr[q] * er[q] - xi[q] * ei[q];
+        xi[q] = xr[q] * ei[q] + xi[q] * er[q];
+        xr[q] = t;
       }
-      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      const double m = (double)(p0 + k - g.P / 2);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int row = in_row(q);
+        if (row >= 0) {
+          const cpx<T> gv = gc[row];
+          double sn, cs;
+          sincos_cw(-pixel_zp(row, col, g) * m, &sn, &cs);
+          const double gr = (double)gv.x, gi = (double)gv.y;
+          v[q < 4 ? q : q + 8] = fftc::mk((T)(gr * cs - gi * sn), (T)(gr * sn + gi * cs));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     colr::fft(v, buf, -1, tv);
-    cpx<T> *hk = hs + h_plane(g, k);
+    cpx<T> *hk = H + h_plane(g, k);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) hk[(size_t)(j + 1024 * (e >> 2) + 4096 * (e & 3)) << kTileLog2] = v[e];
+    for (int e = 0; e < 16; ++e)
+      *reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(hk + ((1024 * (e >> 2) + 4096 * (e & 3)) << kTileLog2)) + off) =
+          v[e];
   }
 }
 
@@ -1647,8 +1486,6 @@ int allow_lds(K kernel, int bytes) {
   if (bytes > 65536) CURIG_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   return kOk;
 }
-
-inline int col_groups(const Geom &g, int cpw) { return (g.nslot + cpw - 1) / cpw; }
 
 template <typename T> inline bool whole_row_planes(const Geom &g) {
   return g.rsplit == 0 && g.rpw == 1 && g.nf1 == 4096;
@@ -1786,46 +1623,6 @@ int allow_row_interp(const Geom &g) {
   return kOk;
 }
 
-// ms2dirty, one batch on the LDS path: column FFT + w-accumulation into accT
-template <typename T>
-void lds_cols_forward(const Geom &g, int p0, int nb, const cpx<T> *H, double2 *accT, const cpx<T> *tw2, int first,
-                      hipStream_t st) {
-  if (g.colreg) {
-    col_fwd_reg_kernel<T><<<col_groups(g, 1), colr::NT, g.lds_col_bytes, st>>>(H, accT, tw2, g, p0, nb, first);
-    return;
-  }
-  col_fwd_kernel<T, 16><<<col_groups(g, g.cpw), g.cpw * g.nf2 / 16, g.lds_col_bytes, st>>>(H, accT, tw2, g, p0, nb, first);
-}
-
-// dirty2ms, one batch on the LDS path: w-fill + inverse column FFT -> H (column-tiled)
-template <typename T>
-void lds_cols_backward(const Geom &g, int p0, int nb, const cpx<T> *gT, cpx<T> *H, const cpx<T> *tw2,
-                       hipStream_t st) {
-  if (g.colreg) {
-    col_inv_reg_kernel<T><<<col_groups(g, 1), colr::NT, g.lds_col_bytes, st>>>(gT, H, tw2, g, p0, nb);
-    return;
-  }
-  col_inv_kernel<T, 16><<<col_groups(g, g.cpw_inv), g.cpw_inv * g.nf2 / 16, g.lds_coli_bytes, st>>>(gT, H, tw2, g, p0, nb);
-}
-
-template <typename T>
-int allow_cols(const Geom &g) {
-  // every column workgroup needs its LDS block (a launch with less would
-  // address LDS it does not own)
-  if (g.lds_col_bytes <= 0 || (!g.colreg && g.lds_coli_bytes <= 0)) {
-    set_error("column pass without an LDS size (%d, %d)", g.lds_col_bytes, g.lds_coli_bytes);
-    return kErrArg;
-  }
-  if (g.colreg) {
-    CURIG_TRY(allow_lds(col_fwd_reg_kernel<T>, g.lds_col_bytes));
-    CURIG_TRY(allow_lds(col_inv_reg_kernel<T>, g.lds_col_bytes));
-    return kOk;
-  }
-  CURIG_TRY(allow_lds(col_fwd_kernel<T, 16>, g.lds_col_bytes));
-  CURIG_TRY(allow_lds(col_inv_kernel<T, 16>, g.lds_coli_bytes));
-  return kOk;
-}
-
 // one source per (precision, kernel group), so the heavy kernels compile in parallel
 #define CURIG_LDS_SPREAD_INST(T)                                                                                   \
   template void lds_spread_rows<T>(const Rec<T> *, const T *, const int *, const Geom &, int, int, cpx<T> *,       \
@@ -1835,11 +1632,4 @@ int allow_cols(const Geom &g) {
   template void lds_row_interp<T>(const Rec<T> *, const T *, const int *, const cpx<T> *, double2 *,              \
                                   const cpx<T> *, const Geom &, int, int, hipStream_t);                            \
   template int allow_row_interp<T>(const Geom &);
-#define CURIG_LDS_COLS_INST(T)                                                                                     \
-  template void lds_cols_forward<T>(const Geom &, int, int, const cpx<T> *, double2 *, const cpx<T> *, int,        \
-                                    hipStream_t);                                                                  \
-  template void lds_cols_backward<T>(const Geom &, int, int, const cpx<T> *, cpx<T> *, const cpx<T> *,             \
-                                     hipStream_t);                                                                 \
-  template int allow_cols<T>(const Geom &);
-
 }  // namespace curig

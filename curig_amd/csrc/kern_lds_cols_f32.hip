@@ -1,5 +1,5 @@
 // LDS path: cols kernels and launchers for float planes.
-#include "kern_lds.h"
+#include "kern_cols.h"
 
 namespace curig {
 CURIG_LDS_COLS_INST(float)

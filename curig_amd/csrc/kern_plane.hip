@@ -184,7 +184,12 @@ __global__ void __launch_bounds__(256) epilogue_kernel(const double2 *__restrict
     double scale, phase, s, c;
     pixel_correction(row, col, g, fk1, fk2, q, scale, phase);
     sincos(phase, &s, &c);
-    double2 a = acc[colmajor ? (long)col * g.N2 + row : idx];
+    const double2 *ac = acc + (colmajor ? (long)col * g.N2 + row : idx);
+    double2 a = ac[0];
+    for (int k = 1; k < g.nacc; ++k) {
+      a.x += ac[k * npix].x;
+      a.y += ac[k * npix].y;
+    }
     double re = (a.x * c - a.y * s) * scale, im = (a.x * s + a.y * c) * scale;
     if (accumulate)
       add_c<TO>(out, idx, re, im);

@@ -6,7 +6,8 @@
 // bits (n * part is exact for |n| < 2^25, i.e. |x| < 5.2e7), then Taylor
 // polynomials of sin and cos on [-pi/4, pi/4] (terms through r^17 and r^18;
 // the first omitted term is below 1e-19).  No branches: the quadrant is applied
-// by selects.
+// by selects.  The column passes evaluate them once per image cell and plane
+// chunk; from plane to plane they multiply by e^{i z'} in FP64.
 #pragma once
 
 #ifdef __HIPCC__
@@ -53,9 +54,8 @@ TRIG_HD void sincos_cw(double x, double *sp, double *cp) {
 }
 
 // Same reduction in FP64, then sin and cos of the reduced argument rounded to
-// FP32 (Taylor through r^9 and r^10, truncation below 2e-9): the phase of a
-// w-plane in the FP32-mixed path, where the plane values are FP32 themselves.
-// The argument x and its reduction stay FP64 (x reaches ~1e4 rad).
+// FP32 (Taylor through r^9 and r^10, truncation below 2e-9): a phase for FP32
+// values.  The argument x and its reduction stay FP64.
 TRIG_HD void sincos_rf(double x, float *sp, float *cp) {
   const double n = rint(x * 0x1.45f306dc9c883p-1);
   double r = x - n * 0x1.921fb54p+0;
@@ -76,18 +76,6 @@ TRIG_HD void sincos_rf(double x, float *sp, float *cp) {
   const float s1 = (q & 1) ? c : s, c1 = (q & 1) ? s : c;
   *sp = (q & 2) ? -s1 : s1;
   *cp = ((q + 1) & 2) ? -c1 : c1;
-}
-
-// Phase e^{i x} at the precision of the plane values T.
-template <typename T> TRIG_HD void plane_phase(double x, double *s, double *c) {
-  if (sizeof(T) == 4) {
-    float sf, cf;
-    sincos_rf(x, &sf, &cf);
-    *s = sf;
-    *c = cf;
-  } else {
-    sincos_cw(x, s, c);
-  }
 }
 
 }  // namespace curig

@@ -55,3 +55,18 @@ def test_rows_of_8192_in_halves(nx, ny, nrow, eps):
     e1, e2 = _both_paths("fp32", uvw, vis, wgt, img, nx, ny, fov, f0, eps)
     say(f"[rows of 8192] {nx}x{ny} rows {nrow} eps {eps}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
     assert e1 < 2e-6 and e2 < 2e-6
+
+
+# power-of-two columns (grid size along u) of every length the column kernels
+# are built for, few planes (several plane chunks per batch) and more than one
+# batch of planes; image rows at and below half the grid
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nx,ny,wmax", [(32, 64, 400.0), (63, 64, 4000.0), (128, 63, 400.0), (256, 64, 3000.0),
+                                        (509, 64, 400.0), (1024, 64, 400.0), (2048, 64, 400.0), (4096, 64, 400.0)])
+def test_columns_of_every_length(precision, nx, ny, wmax):
+    fov, eps = 2.0 if nx > 100 else 10.0, 1e-6
+    uvw, vis, wgt, img, f0 = _case(2000, nx, ny, fov, wmax, nx * 3 + ny)
+    e1, e2 = _both_paths(precision, uvw, vis, wgt, img, nx, ny, fov, f0, eps)
+    say(f"[columns] {precision} {nx}x{ny} wmax {wmax}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
+    tol = 1e-11 if precision == "fp64" else 2e-6
+    assert e1 < tol and e2 < tol
