@@ -96,6 +96,9 @@ struct Geom {
   int nquad;          // number of quadrature nodes for phihat3
   // pruned LDS FFT path (power-of-two grids); fft_lds == 0 selects rocFFT
   int fft_lds;
+  int mix;            // LDS path on axes 2^a 3^b 5^c (mixed-radix kernels), else powers of two
+  int nt_row, nt_col; // its threads per row and column workgroup
+  int pch_row;        // its planes per row workgroup
   int rpw;            // grid rows per workgroup in the row pass (rpw * nf1 = 16 * threads)
   int cpw;            // grid columns per workgroup in the column pass (cpw * nf2 = 16 * threads)
   int cpw_inv;        // the same for the dirty2ms column pass (whole column tiles where they fit)

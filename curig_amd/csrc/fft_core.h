@@ -245,13 +245,14 @@ template <typename T, typename Ptr> struct TwoLevel {
   int lb;
   FC_HD cpx<T> operator[](int t) const { return mul(hi[t >> lb], lo[t & ((1 << lb) - 1)]); }
 };
-// lb for a length-n table: ceil(log2(n) / 2); hi has n >> lb entries, lo 2^lb
+// lb for a length-n table: ceil(log2(n) / 2); hi has ceil(n / 2^lb) entries, lo 2^lb
 FC_HD int twiddle_split(int n) {
   int m = 0;
   while ((1 << m) < n) ++m;
   return (m + 1) / 2;
 }
-FC_HD int twiddle_entries(int n) { return (n >> twiddle_split(n)) + (1 << twiddle_split(n)); }
+FC_HD int twiddle_hi(int n) { return ((n - 1) >> twiddle_split(n)) + 1; }
+FC_HD int twiddle_entries(int n) { return twiddle_hi(n) + (1 << twiddle_split(n)); }
 
 // the same as constant expressions
 FC_HD constexpr int twiddle_split_c(int n, int m = 0) { return (1 << m) < n ? twiddle_split_c(n, m + 1) : (m + 1) / 2; }

@@ -323,6 +323,80 @@ static void plan_columns(Geom &g, size_t cs, size_t lds_max, bool compact) {
   g.nacc = (g.Pb + g.pch_fwd - 1) / g.pch_fwd;
 }
 
+// Threads for `count` sequences of n points: the fewest wavefronts (16 elements
+// per thread) whose cheapest factorisation is within 3% of the best found up to
+// half as many again; 0 when none fits max_threads.
+static int mixed_threads(int n, int count, int max_threads, int min_threads) {
+  const int lo = std::max({64, min_threads, (n * count / 16 + 63) / 64 * 64});
+  double best = 1e300;
+  int nt = 0;
+  for (int t = lo; t <= std::min(max_threads, std::max(lo + 128, lo * 3 / 2)); t += 64) {
+    fftm::Plan p;
+    if (!fftm::make_plan(p, n, count, t)) continue;
+    double c = 0;
+    for (int s = 0; s < p.ns; ++s) c += ((long)count * (n / p.R[s]) + 63) / 64 * fftm::radix_cost(p.R[s]);
+    if (c < 0.97 * best) {
+      best = c;
+      nt = t;
+    }
+  }
+  return nt;
+}
+
+// Grids of 2^a 3^b 5^c cells per axis that the power-of-two kernels do not take:
+// the mixed-radix LDS kernels where a row and a column fit a workgroup's LDS.
+// Against the full-plane path (tile spread, rocFFT, w-sum over whole planes):
+// 1500 x 1100 FP32 ms2dirty 19.6 -> 10.5 ms, 3000 x 2500 FP64 dirty2ms 185 ->
+// 47 ms, 512^2 FP64 at upsampling 1.25 (both directions, host arrays) 4.0 -> 2.3
+// ms, so the full planes remain for axes that do not fit (FP64 beyond about 9000
+// points), kernels wider than 16, and grids of few rows (a one-dimensional
+// transform's 2 kw rows: the row workgroups would hold all its points).
+static void plan_mixed(Geom &g, size_t cs, size_t lds_max) {
+  if (!fftm::smooth235(g.nf1) || !fftm::smooth235(g.nf2) || g.nf1 < 16 || g.nf2 < 40 || g.N1 > g.nf1 || g.N2 > g.nf2)
+    return;
+  const size_t room = lds_max > 8192 ? lds_max - 8192 : 0;  // walk tables, block table beside the rows
+  const int max_threads = cs == 16 ? 512 : 1024;
+  auto row_bytes = [&](int rows) {
+    return (size_t)(rows * fftm::seq_stride(g.nf1) + fftc::twiddle_entries(g.nf1)) * cs + (cs == 8 ? rows * (g.nf1 / 16 + 1) * 6 : 0);
+  };
+  auto col_bytes = [&](int cols) { return (size_t)(cols * fftm::seq_stride(g.nf2) + fftc::twiddle_entries(g.nf2)) * cs; };
+  if (row_bytes(1) > room || col_bytes(1) > room) return;
+  // about 2000 elements per row workgroup; whole column tiles (FP64: halves)
+  // where two such workgroups fit a CU
+  int rpw = 1;
+  while (rpw < 8 && 2 * rpw * g.nf1 <= 2048 && 2 * rpw <= g.nf2) rpw *= 2;
+  int cpw = cs == 8 ? 4 : 2;
+  while (cpw > 1 && (col_bytes(cpw) > lds_max / 2 || cpw * g.nf2 / 16 > max_threads)) cpw /= 2;
+  const int ntr = mixed_threads(g.nf1, rpw, max_threads, 64);
+  int ntc = 0;
+  for (; cpw >= 1 && !ntc; cpw /= 2) {
+    // at most 16 image cells per thread
+    ntc = mixed_threads(g.nf2, cpw, max_threads, (cpw * g.N2 / 16 + 64) / 64 * 64);
+    if (ntc) break;
+  }
+  if (!ntr || !ntc) return;
+  g.fft_lds = g.mix = 1;
+  g.rpw = rpw;
+  g.cpw = g.cpw_inv = cpw;
+  g.nt_row = ntr;
+  g.nt_col = ntc;
+  g.nslot = g.N1;
+  g.nct = (g.nslot + kTile - 1) / kTile;
+  // whole 4 x 4 blocks of the dirty2ms layout
+  g.tstride = (g.nf2 + kTile - 1) / kTile * kTile * kTile + (int)(kTilePadBytes / cs);
+}
+
+// Planes per workgroup of the mixed-radix passes (as plan_columns).
+static void plan_mixed_chunks(Geom &g) {
+  auto chunk = [&](int groups) {
+    const int n = std::min((1024 + groups - 1) / groups, 8);
+    return std::max(std::min(2, g.Pb), (g.Pb + n - 1) / n);
+  };
+  g.pch_row = chunk((g.nf2 + g.rpw - 1) / g.rpw);
+  g.pch_fwd = g.pch_inv = chunk((g.N1 + g.cpw - 1) / g.cpw);
+  g.nacc = (g.Pb + g.pch_fwd - 1) / g.pch_fwd;
+}
+
 int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, double eps, double sigma, int sign,
                   double wmin_m, double wmax_m, bool dbl, const Tuning *tune, Geom *gp, KernelOpts *kop,
                   const GridSpec *spec) {
@@ -416,6 +490,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   g.rpw = g.cpw = g.nct = g.tstride = g.nslot = g.slot_lg = g.lds_row_bytes = g.lds_col_bytes = g.rsplit =
       g.lds_rowp_bytes = g.colreg = g.cpw_inv = g.pch_fwd = g.pch_inv = 0;
   g.nacc = 1;
+  g.mix = g.nt_row = g.nt_col = g.pch_row = 0;
   auto pow2 = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
   const size_t cs = dbl ? 16 : 8;
   const size_t lds_max = tn.lds_bytes > 0 ? (size_t)tn.lds_bytes : size_t(160) << 10;
@@ -464,6 +539,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
       g.tstride = g.nf2 * kTile + (int)(kTilePadBytes / cs);
     }
   }
+  if (!g.fft_lds && tn.fft != 1 && !tn.compact && g.kw <= 16) plan_mixed(g, cs, lds_max);
   // planes per batch from the memory budget: full planes (rocFFT path) or, on
   // the LDS path, the compact plane plus the one or two column-pass buffers
   size_t per_plane = (size_t)g.nf1 * g.nf2 * cs;
@@ -475,7 +551,10 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   }
   g.Pb = std::max(1, std::min(Pb, g.P));
   g.nbatch = (g.P + g.Pb - 1) / g.Pb;
-  if (g.fft_lds) plan_columns(g, cs, lds_max, tn.compact != 0);
+  if (g.mix)
+    plan_mixed_chunks(g);
+  else if (g.fft_lds)
+    plan_columns(g, cs, lds_max, tn.compact != 0);
   // bins: full-width row strips for the LDS path (one workgroup owns grid rows),
   // T1 x T2 tiles for the tile-owner spread
   if (g.fft_lds) {
@@ -574,6 +653,12 @@ int plan_all(bool to_image, const Problem *pbs, int n, hipStream_t st, const Tun
     CURIG_TRY(plan_geometry((int)nvalid, pb.nx, pb.ny, pb.fov, pb.freq, pb.eps, pb.sigma, pb.sign, wmin, wmax,
                             pb.dbl, &tn, &cps[i].g, &cps[i].ko, &pb.spec));
     cps[i].nvalid = nvalid;
+    const Geom &g = cps[i].g;
+    if (g.mix && !(fftm::make_plan(cps[i].rowf, g.nf1, g.rpw, g.nt_row) &&
+                   fftm::make_plan(cps[i].colf, g.nf2, g.cpw, g.nt_col))) {
+      set_error("no mixed-radix plan for grid %d x %d", g.nf2, g.nf1);
+      return kErrArg;
+    }
   }
   return kOk;
 }
@@ -592,7 +677,7 @@ int twiddles(int dev, const Geom &g, hipStream_t st, const cpx<T> *&tw1, const c
   if (g_arena || key[0] != g.nf1 || key[1] != g.nf2 || key[2] != (int)sizeof(T)) {
     std::vector<cpx<T>> h(n1 + n2);
     auto fill = [](cpx<T> *o, int n) {
-      const int lb = fftc::twiddle_split(n), nhi = n >> lb, nlo = 1 << lb;
+      const int lb = fftc::twiddle_split(n), nhi = fftc::twiddle_hi(n), nlo = 1 << lb;
       for (int j = 0; j < nhi; ++j) {
         const double a = 2 * M_PI * ((double)j * nlo) / n;
         o[j] = fftc::mk((T)std::cos(a), (T)std::sin(a));
@@ -714,6 +799,10 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image,
     b.tw2 = t2;
     // channels may differ in how their rows are split
     for (const ChanPlan &cp : cps) {
+      if (cp.g.mix) {
+        CURIG_TRY(allow_mix<T>(cp));
+        continue;
+      }
       CURIG_TRY(to_image ? allow_spread_rows<T>(cp.g) : allow_row_interp<T>(cp.g));
       CURIG_TRY(allow_cols<T>(cp.g));
     }
@@ -795,10 +884,16 @@ int enqueue_ms2dirty(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
     if (g.fft_lds) {
       // spread + row FFT counts as spread (t_grid); the column FFT fused with
       // the w-accumulation as FFT (t_fft)
-      lds_spread_rows<T>(recs, (const T *)b.taps, b.off, g, p0, nb, (cpx<T> *)b.H, (const cpx<T> *)b.tw1, st);
+      if (g.mix)
+        mix_spread_rows<T>(recs, (const T *)b.taps, b.off, cp, p0, nb, (cpx<T> *)b.H, (const cpx<T> *)b.tw1, st);
+      else
+        lds_spread_rows<T>(recs, (const T *)b.taps, b.off, g, p0, nb, (cpx<T> *)b.H, (const cpx<T> *)b.tw1, st);
       CURIG_HIP(hipGetLastError());
       const int bm = tm.mark();
-      lds_cols_forward<T>(g, p0, nb, (const cpx<T> *)b.H, b.acc, (const cpx<T> *)b.tw2, bi == 0 ? 1 : 0, st);
+      if (g.mix)
+        mix_cols_forward<T>(cp, p0, nb, (const cpx<T> *)b.H, b.acc, (const cpx<T> *)b.tw2, bi == 0 ? 1 : 0, st);
+      else
+        lds_cols_forward<T>(g, p0, nb, (const cpx<T> *)b.H, b.acc, (const cpx<T> *)b.tw2, bi == 0 ? 1 : 0, st);
       CURIG_HIP(hipGetLastError());
       const int c = tm.mark();
       tm.span(a, bm, &t_spread);
@@ -867,10 +962,16 @@ int enqueue_dirty2ms(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
     if (g.fft_lds) {
       // w-fill + column iFFT counts as FFT (t_fft); the row iFFT fused with
       // the interpolation as interpolation (t_grid)
-      lds_cols_backward<T>(g, p0, nb, (const cpx<T> *)gimg, (cpx<T> *)b.H, (const cpx<T> *)b.tw2, st);
+      if (g.mix)
+        mix_cols_backward<T>(cp, p0, nb, (const cpx<T> *)gimg, (cpx<T> *)b.H, (const cpx<T> *)b.tw2, st);
+      else
+        lds_cols_backward<T>(g, p0, nb, (const cpx<T> *)gimg, (cpx<T> *)b.H, (const cpx<T> *)b.tw2, st);
       CURIG_HIP(hipGetLastError());
       const int c = tm.mark();
-      if (cp.nvalid > 0)
+      if (cp.nvalid > 0 && g.mix)
+        mix_row_interp<T>(recs, (const T *)b.taps, b.off, (const cpx<T> *)b.H, b.vacc, (const cpx<T> *)b.tw1, cp, p0, nb,
+                          st);
+      else if (cp.nvalid > 0)
         lds_row_interp<T>(recs, (const T *)b.taps, b.off, (const cpx<T> *)b.H, b.vacc, (const cpx<T> *)b.tw1, g, p0,
                           nb, st);
       CURIG_HIP(hipGetLastError());
@@ -957,7 +1058,7 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
+      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
   k << b.dev << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc

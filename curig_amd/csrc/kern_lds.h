@@ -152,7 +152,7 @@ __device__ __forceinline__ void walk_finish(WalkTable &wt, const WalkAhead &wa) 
 template <typename T>
 __device__ __forceinline__ fftc::TwoLevel<T, const cpx<T> *> lds_twiddles(cpx<T> *dst,
                                                                          const cpx<T> *__restrict__ src, int n) {
-  const int lb = fftc::twiddle_split(n), nhi = n >> lb, cnt = nhi + (1 << lb);
+  const int lb = fftc::twiddle_split(n), nhi = fftc::twiddle_hi(n), cnt = nhi + (1 << lb);
   for (int i = threadIdx.x; i < cnt; i += blockDim.x) dst[i] = src[i];
   return fftc::TwoLevel<T, const cpx<T> *>{dst, dst + nhi, lb};
 }

@@ -1,0 +1,551 @@
+// Row and column kernels of the LDS path for grids whose axes are 2^a 3^b 5^c
+// but not powers of two with the image inside half the grid (those run the
+// kernels of kern_lds.h and kern_cols.h).  The same passes over the same
+// column-tiled planes H, with the mixed-radix LDS transform of fft_mix.h: the
+// full grid planes of the rocFFT path (written and read five times per plane)
+// are never formed.  Each workgroup keeps its rows or columns and walks a chunk
+// of the batch's planes.
+//
+// What bounds them: VALU issue of the transform (about 100 instructions per
+// element: butterflies, twiddles and the run-time index arithmetic) and its LDS
+// passes, with one workgroup's memory phases behind another's transform.
+#pragma once
+#include "kern_lds.h"
+
+#include "fft_mix.h"
+
+namespace curig {
+
+template <typename T> struct MixThreads { static constexpr int value = sizeof(T) == 8 ? 512 : 1024; };
+
+// LDS of a row workgroup: the rows, the axis' twiddles and (FP32) the block
+// table of the block-floating-point spread.
+__host__ __device__ inline int mix_blocks(int nf1) { return (nf1 + (1 << kFixBlkLog2) - 1) >> kFixBlkLog2; }
+
+// stages [s0, P.ns) of the transform; the caller's barrier precedes it, a
+// barrier ends it
+template <typename T, int SIGN, typename Tw>
+__device__ __forceinline__ void mix_stages(cpx<T> *buf, const fftm::Plan &P, const Tw &tw, int s0, int Ns) {
+  for (int s = s0; s < P.ns; ++s) {
+    const int R = P.R[s];
+    // opaque copy of the thread id: every radix's addresses are formed where
+    // they are used (hoisted out of the plane loop they spill)
+    int tid = threadIdx.x;
+    __asm__ volatile("" : "+v"(tid));
+    fftm::with_radix(R, [&](auto tag) {
+      constexpr int RR = decltype(tag)::value;
+      cpx<T> v[RR * fftm::radix_nb(RR)];
+      fftm::stage_load<T, RR, SIGN>([&](int q, int k) { return buf[q * P.stride + fftc::pad(k)]; }, v, P, s, Ns, tw, tid);
+      __syncthreads();
+      fftm::stage_store<T, RR>([&](int q, int k, cpx<T> x) { buf[q * P.stride + fftc::pad(k)] = x; }, v, P, s, Ns, tid);
+    });
+    __syncthreads();
+    Ns *= R;
+  }
+}
+
+// the first stage on the integers of the block-floating-point spread: cell k of
+// sequence q in block k >> kFixBlkLog2 of exponent fexp[q * nblk + block]
+template <typename T, int SIGN, typename Tw>
+__device__ __forceinline__ void mix_first_fix(cpx<T> *buf, const fftm::Plan &P, const Tw &tw, const short *fexp, int nblk) {
+  int tid = threadIdx.x;
+  __asm__ volatile("" : "+v"(tid));
+  fftm::with_radix(P.R[0], [&](auto tag) {
+    constexpr int RR = decltype(tag)::value;
+    cpx<T> v[RR * fftm::radix_nb(RR)];
+    fftm::stage_load<T, RR, SIGN>(
+        [&](int q, int k) {
+          const int2 x = reinterpret_cast<const int2 *>(buf)[q * P.stride + fftc::pad(k)];
+          const int e = fexp[q * nblk + (k >> kFixBlkLog2)];
+          return fftc::mk((T)ldexpf((float)x.x, -e), (T)ldexpf((float)x.y, -e));
+        },
+        v, P, 0, 1, tw, tid);
+    __syncthreads();
+    fftm::stage_store<T, RR>([&](int q, int k, cpx<T> x) { buf[q * P.stride + fftc::pad(k)] = x; }, v, P, 0, 1, tid);
+  });
+  __syncthreads();
+}
+
+// Blocks of the cells ix .. ix + kw - 1 (cyclic, kw <= 16): at most b0, the
+// row's last block (when they wrap) and the last cell's.
+struct FixBlocks {
+  int b0, bm, b1;
+};
+__device__ __forceinline__ FixBlocks fix_blocks(int ix, int kw, int nf1) {
+  FixBlocks f;
+  const int last = ix + kw - 1;
+  f.b0 = ix >> kFixBlkLog2;
+  f.bm = last >= nf1 ? (nf1 - 1) >> kFixBlkLog2 : f.b0;
+  f.b1 = (last >= nf1 ? last - nf1 : last) >> kFixBlkLog2;
+  return f;
+}
+
+// plane tap of a record in plane p, or -1
+__device__ __forceinline__ int plane_tap(int iw, int p, const Geom &g) {
+  int k = p - iw;
+  if (k < 0) k += g.P;
+  return k < g.kww ? k : -1;
+}
+
+// ms2dirty: spread into the workgroup's rows (LDS), row FFT, image columns to H.
+// FP32 accumulates in block floating point (integer LDS atomics; kAccFix of
+// kern_lds.h), FP64 with FP64 LDS atomics.
+template <typename T, int KWM>
+__global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
+    const Rec<T> *__restrict__ recs, const T *__restrict__ taps, const int *__restrict__ off, cpx<T> *__restrict__ H,
+    const cpx<T> *__restrict__ tw, Geom g, fftm::Plan P, int p0, int nb, int pchunk) {
+  constexpr bool kFix = sizeof(T) == 4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ WalkTable wt[2];
+  __shared__ int fixnan;
+  const int nf1 = g.nf1, nf2 = g.nf2, kw = g.kw, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
+  const int nbuf = P.count * P.stride, nblk = mix_blocks(nf1), h1 = N1 / 2;
+  cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
+  float *fixt = reinterpret_cast<float *>(buf + nbuf + fftc::twiddle_entries(nf1));
+  short *fixe = reinterpret_cast<short *>(fixt + rpw * nblk);
+  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
+  const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
+  const auto tv = lds_twiddles<T>(buf + nbuf, tw, nf1);
+  if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, nrows);
+  for (int i = tid; i < nbuf; i += nt) buf[i] = fftc::mk((T)0, (T)0);
+  if (kFix) {
+    for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
+    if (tid == 0) fixnan = 0;
+  }
+  __syncthreads();
+  int cur = 0;
+  for (int pl = k0; pl < k1; ++pl, cur ^= 1) {
+    const int p = p0 + pl, total = wt[cur].total;
+    const bool more = pl + 1 < k1;
+    WalkAhead wa;
+    if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, nrows);
+    if (kFix && total > 0) {
+      for (int t = tid; t < total; t += nt) {
+        const int ia = walk_record(wt[cur], t);
+        const Rec<T> rc = recs[ia];
+        const int k = plane_tap(rc.iw, p, g);
+        if (k < 0) continue;
+        const T *tq = taps + (size_t)ia * (3 * KWM);
+        const float a = (fabsf((float)rc.re) + fabsf((float)rc.im)) * fabsf((float)tq[2 * KWM + k]);
+        const FixBlocks f = fix_blocks(rc.ix, kw, nf1);
+        for (int r = 0; r < nrows; ++r) {
+          int jj = row0 + r - rc.iy;
+          if (jj < 0) jj += nf2;
+          if (jj >= kw) continue;
+          const float b = a * fabsf((float)tq[KWM + jj]);
+          float *bs = fixt + r * nblk;
+          atomicAdd(bs + f.b0, b);
+          if (f.bm != f.b0) atomicAdd(bs + f.bm, b);
+          if (f.b1 != f.b0 && f.b1 != f.bm) atomicAdd(bs + f.b1, b);
+        }
+      }
+      __syncthreads();
+      for (int i = tid; i < nrows * nblk; i += nt) {
+        // published to the first stage by the barrier after the spread
+        const int e = fix_block_exp(fixt[i]);
+        fixe[i] = (short)(e == kFixNaN ? 0 : e);
+        if (e == kFixNaN) fixnan = 1;
+      }
+    }
+    for (int t = tid; t < total; t += nt) {
+      const int ia = walk_record(wt[cur], t);
+      const Rec<T> rc = recs[ia];
+      const int k = plane_tap(rc.iw, p, g);
+      if (k < 0) continue;
+      const T *tq = taps + (size_t)ia * (3 * KWM);
+      T kx[KWM];
+#pragma unroll
+      for (int i = 0; i < KWM; ++i) kx[i] = tq[i];
+      const T kz = tq[2 * KWM + k];
+      const FixBlocks f = fix_blocks(rc.ix, kw, nf1);
+      for (int r = 0; r < nrows; ++r) {
+        int jj = row0 + r - rc.iy;
+        if (jj < 0) jj += nf2;
+        if (jj >= kw) continue;
+        const T a = kz * tq[KWM + jj], vre = rc.re * a, vim = rc.im * a;
+        cpx<T> *row = buf + r * P.stride;
+        int e0 = 0, em = 0, e1 = 0;
+        if (kFix) {
+          const float *bs = fixt + r * nblk;
+          e0 = fix_block_exp(bs[f.b0]);
+          em = fix_block_exp(bs[f.bm]);
+          e1 = fix_block_exp(bs[f.b1]);
+          e0 = e0 == kFixNaN ? 0 : e0;
+          em = em == kFixNaN ? 0 : em;
+          e1 = e1 == kFixNaN ? 0 : e1;
+        }
+#pragma unroll
+        for (int i = 0; i < KWM; ++i) {
+          if (i < kw) {
+            int cx = rc.ix + i;
+            if (cx >= nf1) cx -= nf1;
+            const T re = vre * kx[i], im = vim * kx[i];
+            if (kFix) {
+              const int blk = cx >> kFixBlkLog2, e = blk == f.b0 ? e0 : blk == f.bm ? em : e1;
+              int *d = reinterpret_cast<int *>(row + fftc::pad(cx));
+              atomicAdd(d, __float2int_rn(ldexpf((float)re, e)));
+              atomicAdd(d + 1, __float2int_rn(ldexpf((float)im, e)));
+            } else {
+              T *d = reinterpret_cast<T *>(row + fftc::pad(cx));
+              atomicAdd(d, re);
+              atomicAdd(d + 1, im);
+            }
+          }
+        }
+      }
+    }
+    if (tid < 64 && more) walk_finish(wt[cur ^ 1], wa);
+    __syncthreads();  // spread done; the next plane's walk table is complete
+    cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
+    if (total == 0) {
+      // no visibility reaches these rows of this plane (and the LDS is still clear)
+      for (int r = 0; r < nrows; ++r)
+        for (int i = tid; i < N1; i += nt) hb[h_slot(g, i) + (r << kTileLog2)] = fftc::mk((T)0, (T)0);
+      continue;
+    }
+    const bool pnan = kFix && fixnan;  // cleared below, after the transform's barriers
+    if (kFix) {
+      mix_first_fix<T, +1>(buf, P, tv, fixe, nblk);
+      mix_stages<T, +1>(buf, P, tv, 1, P.R[0]);
+    } else {
+      mix_stages<T, +1>(buf, P, tv, 0, 1);
+    }
+    for (int r = 0; r < nrows; ++r)
+      for (int i = tid; i < N1; i += nt) {
+        const int k = i >= h1 ? i - h1 : nf1 + i - h1;
+        cpx<T> x = buf[r * P.stride + fftc::pad(k)];
+        if (pnan) x = fftc::mk((T)NAN, (T)NAN);
+        hb[h_slot(g, i) + (r << kTileLog2)] = x;
+      }
+    __syncthreads();  // every output read: clear for the next plane
+    for (int i = tid; i < nbuf; i += nt) buf[i] = fftc::mk((T)0, (T)0);
+    if (kFix) {
+      for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
+      if (tid == 0) fixnan = 0;
+    }
+    __syncthreads();
+  }
+}
+
+// dirty2ms: rows of H expanded to the grid, inverse row FFT, interpolation of
+// every record that touches the rows (FP64 atomics on its accumulator).
+template <typename T, int KWM>
+__global__ void __launch_bounds__(MixThreads<T>::value) row_interp_mix_kernel(
+    const cpx<T> *__restrict__ H, const Rec<T> *__restrict__ recs, const T *__restrict__ taps,
+    const int *__restrict__ off, double2 *__restrict__ vacc, const cpx<T> *__restrict__ tw, Geom g, fftm::Plan P, int p0,
+    int nb, int pchunk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ WalkTable wt[2];
+  const int nf1 = g.nf1, nf2 = g.nf2, kw = g.kw, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
+  cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
+  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
+  const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
+  const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
+  if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, nrows);
+  // rows past the grid (the last workgroup): zero sequences, transformed along
+  for (int i = tid; i < P.count * P.stride; i += nt) buf[i] = fftc::mk((T)0, (T)0);
+  __syncthreads();
+  int cur = 0;
+  for (int pl = k0; pl < k1; ++pl, cur ^= 1) {
+    const int p = p0 + pl, total = wt[cur].total;
+    const bool more = pl + 1 < k1;
+    WalkAhead wa;
+    if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, nrows);
+    if (total > 0) {
+      const cpx<T> *hb = H + h_plane(g, pl);
+      for (int r = 0; r < nrows; ++r) {
+        const cpx<T> *hr = hb + ht_row(row0 + r);
+        constexpr int B = 8;  // loads in flight
+        for (int i0 = tid; i0 < nf1; i0 += B * nt) {
+          cpx<T> v[B];
+#pragma unroll
+          for (int b = 0; b < B; ++b) {
+            const int i = i0 + b * nt, col = i < nf1 ? image_index(i, N1, nf1) : -1;
+            v[b] = col >= 0 ? hr[ht_slot(g, col)] : fftc::mk((T)0, (T)0);
+          }
+#pragma unroll
+          for (int b = 0; b < B; ++b) {
+            const int i = i0 + b * nt;
+            if (i < nf1) buf[r * P.stride + fftc::pad(i)] = v[b];
+          }
+        }
+      }
+      __syncthreads();
+      mix_stages<T, -1>(buf, P, tv, 0, 1);
+      for (int t = tid; t < total; t += nt) {
+        const int ia = walk_record(wt[cur], t);
+        const Rec<T> rc = recs[ia];
+        const int k = plane_tap(rc.iw, p, g);
+        if (k < 0) continue;
+        const T *tq = taps + (size_t)ia * (3 * KWM);
+        T kx[KWM];
+#pragma unroll
+        for (int i = 0; i < KWM; ++i) kx[i] = tq[i];
+        const T kz = tq[2 * KWM + k];
+        T sr = 0, si = 0;
+        bool hit = false;
+        for (int r = 0; r < nrows; ++r) {
+          int jj = row0 + r - rc.iy;
+          if (jj < 0) jj += nf2;
+          if (jj >= kw) continue;
+          hit = true;
+          const cpx<T> *row = buf + r * P.stride;
+          T rr = 0, ri = 0;
+#pragma unroll
+          for (int i = 0; i < KWM; ++i) {
+            if (i < kw) {
+              int cx = rc.ix + i;
+              if (cx >= nf1) cx -= nf1;
+              const cpx<T> f = row[fftc::pad(cx)];
+              rr += f.x * kx[i];
+              ri += f.y * kx[i];
+            }
+          }
+          const T ky = tq[KWM + jj];
+          sr += rr * ky;
+          si += ri * ky;
+        }
+        if (hit) {
+          atomicAdd(&vacc[ia].x, (double)(sr * kz));
+          atomicAdd(&vacc[ia].y, (double)(si * kz));
+        }
+      }
+    }
+    if (tid < 64 && more) walk_finish(wt[cur ^ 1], wa);
+    __syncthreads();  // the rows are free; the next plane's walk table is complete
+  }
+}
+
+// ms2dirty column pass (col_fwd_kernel's work): cpw columns, planes of a chunk
+// last to first, Horner's rule in FP64; NO image cells per thread, MT threads at
+// most (long FP32 columns only take more than 512, whose registers they halve).
+template <typename T, int NO, int MT>
+__global__ void __launch_bounds__(MT) col_fwd_mix_kernel(const cpx<T> *__restrict__ H,
+                                                                          double2 *__restrict__ accT,
+                                                                          const cpx<T> *__restrict__ tw, Geom g,
+                                                                          fftm::Plan P, int p0, int nb, int first,
+                                                                          int cpw_lg, int pchunk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
+  const int nf2 = g.nf2, N2 = g.N2, nt = blockDim.x, tid = threadIdx.x, cpw = 1 << cpw_lg;
+  const int s0 = xcd_group(blockIdx.x, gridDim.x) << cpw_lg, cols = min(cpw, g.N1 - s0);
+  const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk), nout = N2 << cpw_lg, nin = nf2 << cpw_lg;
+  const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf2);
+  double ar[NO], ai[NO], er[NO], ei[NO];
+#pragma unroll
+  for (int q = 0; q < NO; ++q) {
+    ar[q] = ai[q] = 0.0;
+    const int o = tid + q * nt, c = o & (cpw - 1), row = o >> cpw_lg;
+    sincos_cw(o < nout && c < cols ? pixel_zp(row, s0 + c, g) : 0.0, &ei[q], &er[q]);
+  }
+  for (int k = k1 - 1; k >= k0; --k) {
+    const cpx<T> *hk = H + h_plane(g, k);
+    __syncthreads();  // the previous plane's LDS reads are done
+    constexpr int B = 8;  // loads in flight
+    for (int i0 = tid; i0 < nin; i0 += B * nt) {
+      cpx<T> v[B];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int i = i0 + b * nt, c = i & (cpw - 1);
+        v[b] = i < nin && c < cols ? hk[h_slot(g, s0 + c) + ((i >> cpw_lg) << kTileLog2)] : fftc::mk((T)0, (T)0);
+      }
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int i = i0 + b * nt;
+        if (i < nin) buf[(i & (cpw - 1)) * P.stride + fftc::pad(i >> cpw_lg)] = v[b];
+      }
+    }
+    __syncthreads();
+    mix_stages<T, +1>(buf, P, tv, 0, 1);
+#pragma unroll
+    for (int q = 0; q < NO; ++q) {
+      const int o = tid + q * nt;
+      if (o < nout) {
+        const cpx<T> f = buf[(o & (cpw - 1)) * P.stride + fftc::pad(grid_index(o >> cpw_lg, N2, nf2))];
+        const double t = ar[q] * er[q] - ai[q] * ei[q] + (double)f.x;
+        ai[q] = ar[q] * ei[q] + ai[q] * er[q] + (double)f.y;
+        ar[q] = t;
+      }
+    }
+  }
+  double2 *out = accT + (size_t)blockIdx.y * g.N1 * N2;
+  const double m = (double)(p0 + k0 - g.P / 2);
+#pragma unroll
+  for (int q = 0; q < NO; ++q) {
+    const int o = tid + q * nt, c = o & (cpw - 1), row = o >> cpw_lg;
+    if (o < nout && c < cols) {
+      double sn, cs;
+      sincos_cw(pixel_zp(row, s0 + c, g) * m, &sn, &cs);
+      double2 r = make_double2(ar[q] * cs - ai[q] * sn, ar[q] * sn + ai[q] * cs);
+      double2 *d = out + (size_t)(s0 + c) * N2 + row;
+      if (!first) {
+        r.x += d->x;
+        r.y += d->y;
+      }
+      *d = r;
+    }
+  }
+}
+
+// dirty2ms column pass (col_inv_kernel's work): phased image cells carried from
+// plane to plane in FP64, inverse FFT, full columns to H.
+template <typename T, int NO, int MT>
+__global__ void __launch_bounds__(MT) col_inv_mix_kernel(const cpx<T> *__restrict__ gT,
+                                                                          cpx<T> *__restrict__ H,
+                                                                          const cpx<T> *__restrict__ tw, Geom g,
+                                                                          fftm::Plan P, int p0, int nb, int cpw_lg,
+                                                                          int pchunk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
+  const int nf2 = g.nf2, N2 = g.N2, h2 = N2 / 2, nt = blockDim.x, tid = threadIdx.x, cpw = 1 << cpw_lg;
+  const int s0 = xcd_group(blockIdx.x, gridDim.x) << cpw_lg, cols = min(cpw, g.N1 - s0);
+  const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk), nin = N2 << cpw_lg, nout = nf2 << cpw_lg;
+  const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf2);
+  double xr[NO], xi[NO], er[NO], ei[NO];
+  const double m = (double)(p0 + k0 - g.P / 2);
+#pragma unroll
+  for (int q = 0; q < NO; ++q) {
+    xr[q] = xi[q] = er[q] = ei[q] = 0.0;
+    const int o = tid + q * nt, c = o & (cpw - 1), row = o >> cpw_lg;
+    if (o < nin && c < cols) {
+      const double zp = pixel_zp(row, s0 + c, g);
+      double sn, cs;
+      sincos_cw(-zp, &ei[q], &er[q]);
+      sincos_cw(-zp * m, &sn, &cs);
+      const cpx<T> gv = gT[(size_t)(s0 + c) * N2 + row];
+      xr[q] = (double)gv.x * cs - (double)gv.y * sn;
+      xi[q] = (double)gv.x * sn + (double)gv.y * cs;
+    }
+  }
+  for (int k = k0; k < k1; ++k) {
+    __syncthreads();  // the previous plane's LDS reads are done
+#pragma unroll
+    for (int q = 0; q < NO; ++q) {
+      const int o = tid + q * nt;
+      if (o < nin) {
+        buf[(o & (cpw - 1)) * P.stride + fftc::pad(grid_index(o >> cpw_lg, N2, nf2))] = fftc::mk((T)xr[q], (T)xi[q]);
+        const double t = xr[q] * er[q] - xi[q] * ei[q];
+        xi[q] = xr[q] * ei[q] + xi[q] * er[q];
+        xr[q] = t;
+      }
+    }
+    for (int z = tid; z < (nf2 - N2) << cpw_lg; z += nt)
+      buf[(z & (cpw - 1)) * P.stride + fftc::pad(N2 - h2 + (z >> cpw_lg))] = fftc::mk((T)0, (T)0);
+    __syncthreads();
+    mix_stages<T, -1>(buf, P, tv, 0, 1);
+    cpx<T> *hk = H + h_plane(g, k);
+    for (int i = tid; i < nout; i += nt) {
+      const int c = i & (cpw - 1), k2 = i >> cpw_lg;
+      if (c < cols) hk[ht_slot(g, s0 + c) + ht_row(k2)] = buf[c * P.stride + fftc::pad(k2)];
+    }
+  }
+}
+
+// --------------------------------------------------------------------------
+// launchers
+// --------------------------------------------------------------------------
+template <typename T> inline int mix_row_lds(const Geom &g) {
+  int b = (int)sizeof(cpx<T>) * (g.rpw * fftm::seq_stride(g.nf1) + fftc::twiddle_entries(g.nf1));
+  if (sizeof(T) == 4) b += g.rpw * mix_blocks(g.nf1) * 6 + 2;
+  return b;
+}
+template <typename T> inline int mix_col_lds(const Geom &g, int cpw) {
+  return (int)sizeof(cpx<T>) * (cpw * fftm::seq_stride(g.nf2) + fftc::twiddle_entries(g.nf2));
+}
+// f(cells per thread 8 or 16, threads at most 512 or 1024)
+template <typename T, typename F> inline void with_cells(int cells, int nt, F f) {
+  using std::integral_constant;
+  if (sizeof(T) == 4 && nt > 512) {
+    if (cells <= 8)
+      f(integral_constant<int, 8>(), integral_constant<int, 1024>());
+    else
+      f(integral_constant<int, 16>(), integral_constant<int, 1024>());
+  } else if (cells <= 8) {
+    f(integral_constant<int, 8>(), integral_constant<int, 512>());
+  } else {
+    f(integral_constant<int, 16>(), integral_constant<int, 512>());
+  }
+}
+inline int mix_cells(int cpw, int N2, int nt) { return (cpw * N2 + nt - 1) / nt; }
+
+template <typename T>
+void mix_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const ChanPlan &cp, int p0, int nb, cpx<T> *H,
+                     const cpx<T> *tw1, hipStream_t st) {
+  const Geom &g = cp.g;
+  const dim3 grd((g.nf2 + g.rpw - 1) / g.rpw, (nb + g.pch_row - 1) / g.pch_row);
+  const int lb = mix_row_lds<T>(g), nt = cp.rowf.nt;
+  if (g.kw <= 8)
+    spread_row_mix_kernel<T, 8><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, cp.rowf, p0, nb, g.pch_row);
+  else
+    spread_row_mix_kernel<T, 16><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, cp.rowf, p0, nb, g.pch_row);
+}
+
+template <typename T>
+void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, double2 *vacc, const cpx<T> *tw1,
+                    const ChanPlan &cp, int p0, int nb, hipStream_t st) {
+  const Geom &g = cp.g;
+  const dim3 grd((g.nf2 + g.rpw - 1) / g.rpw, (nb + g.pch_row - 1) / g.pch_row);
+  const int lb = mix_row_lds<T>(g), nt = cp.rowf.nt;
+  if (g.kw <= 8)
+    row_interp_mix_kernel<T, 8><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, cp.rowf, p0, nb, g.pch_row);
+  else
+    row_interp_mix_kernel<T, 16><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, cp.rowf, p0, nb, g.pch_row);
+}
+
+template <typename T>
+void mix_cols_forward(const ChanPlan &cp, int p0, int nb, const cpx<T> *H, double2 *accT, const cpx<T> *tw2, int first,
+                      hipStream_t st) {
+  const Geom &g = cp.g;
+  const int nt = cp.colf.nt, lb = mix_col_lds<T>(g, g.cpw), lg = 31 - __builtin_clz(g.cpw);
+  const dim3 grd((g.N1 + g.cpw - 1) / g.cpw, (nb + g.pch_fwd - 1) / g.pch_fwd);
+  with_cells<T>(mix_cells(g.cpw, g.N2, nt), nt, [&](auto NO, auto MT) {
+    col_fwd_mix_kernel<T, NO.value, MT.value><<<grd, nt, lb, st>>>(H, accT, tw2, g, cp.colf, p0, nb, first, lg, g.pch_fwd);
+  });
+}
+
+template <typename T>
+void mix_cols_backward(const ChanPlan &cp, int p0, int nb, const cpx<T> *gT, cpx<T> *H, const cpx<T> *tw2,
+                       hipStream_t st) {
+  const Geom &g = cp.g;
+  const int nt = cp.colf.nt, lb = mix_col_lds<T>(g, g.cpw), lg = 31 - __builtin_clz(g.cpw);
+  const dim3 grd((g.N1 + g.cpw - 1) / g.cpw, (nb + g.pch_inv - 1) / g.pch_inv);
+  with_cells<T>(mix_cells(g.cpw, g.N2, nt), nt, [&](auto NO, auto MT) {
+    col_inv_mix_kernel<T, NO.value, MT.value><<<grd, nt, lb, st>>>(gT, H, tw2, g, cp.colf, p0, nb, lg, g.pch_inv);
+  });
+}
+
+template <typename T> int allow_mix(const ChanPlan &cp) {
+  const Geom &g = cp.g;
+  const int top = MixThreads<T>::value, rows = cp.rowf.nt, cols = cp.colf.nt;
+  // what the kernels assume of their launches
+  if (cp.rowf.n != g.nf1 || cp.rowf.count != g.rpw || cp.colf.n != g.nf2 || cp.colf.count != g.cpw || rows < 64 ||
+      rows > top || cols < 64 || cols > top || mix_cells(g.cpw, g.N2, cols) > 16 || g.pch_row < 1 || g.pch_fwd < 1 ||
+      g.pch_inv < 1 || (g.cpw & (g.cpw - 1)) != 0) {
+    set_error("mixed-radix plan of grid %d x %d does not fit its kernels", g.nf2, g.nf1);
+    return kErrArg;
+  }
+  const int lr = mix_row_lds<T>(g), lc = mix_col_lds<T>(g, g.cpw);
+  CURIG_TRY((allow_lds(spread_row_mix_kernel<T, 8>, lr)));
+  CURIG_TRY((allow_lds(spread_row_mix_kernel<T, 16>, lr)));
+  CURIG_TRY((allow_lds(row_interp_mix_kernel<T, 8>, lr)));
+  CURIG_TRY((allow_lds(row_interp_mix_kernel<T, 16>, lr)));
+  int ier = kOk;
+  with_cells<T>(mix_cells(g.cpw, g.N2, cols), cols, [&](auto NO, auto MT) {
+    ier = allow_lds(col_fwd_mix_kernel<T, NO.value, MT.value>, lc);
+    if (ier == kOk) ier = allow_lds(col_inv_mix_kernel<T, NO.value, MT.value>, lc);
+  });
+  return ier;
+}
+
+#define CURIG_MIX_INST(T)                                                                                          \
+  template void mix_spread_rows<T>(const Rec<T> *, const T *, const int *, const ChanPlan &, int, int, cpx<T> *,   \
+                                   const cpx<T> *, hipStream_t);                                                   \
+  template void mix_row_interp<T>(const Rec<T> *, const T *, const int *, const cpx<T> *, double2 *,               \
+                                  const cpx<T> *, const ChanPlan &, int, int, hipStream_t);                        \
+  template void mix_cols_forward<T>(const ChanPlan &, int, int, const cpx<T> *, double2 *, const cpx<T> *, int,    \
+                                    hipStream_t);                                                                  \
+  template void mix_cols_backward<T>(const ChanPlan &, int, int, const cpx<T> *, cpx<T> *, const cpx<T> *,         \
+                                     hipStream_t);                                                                 \
+  template int allow_mix<T>(const ChanPlan &);
+
+}  // namespace curig

@@ -10,6 +10,7 @@
 
 #include "curig_internal.h"
 #include "fft_core.h"
+#include "fft_mix.h"
 #include "gridder.h"
 
 namespace curig {
@@ -39,6 +40,7 @@ struct ChanPlan {
   Geom g;
   KernelOpts ko;
   long nvalid = 0;
+  fftm::Plan rowf, colf;  // g.mix: the axes' transforms
 };
 
 // Device pointers of one call's working set (slots of the per-device workspace).
@@ -159,5 +161,21 @@ void lds_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx
 template <typename T> int allow_spread_rows(const Geom &g);
 template <typename T> int allow_row_interp(const Geom &g);
 template <typename T> int allow_cols(const Geom &g);
+
+// ---- kern_mix_*.hip: the LDS path on mixed-radix grids (Geom::mix) -----------
+template <typename T>
+void mix_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const ChanPlan &cp, int p0, int nb, cpx<T> *H,
+                     const cpx<T> *tw1, hipStream_t st);
+template <typename T>
+void mix_cols_forward(const ChanPlan &cp, int p0, int nb, const cpx<T> *H, double2 *accT, const cpx<T> *tw2, int first,
+                      hipStream_t st);
+template <typename T>
+void mix_cols_backward(const ChanPlan &cp, int p0, int nb, const cpx<T> *gT, cpx<T> *H, const cpx<T> *tw2,
+                       hipStream_t st);
+template <typename T>
+void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, double2 *vacc, const cpx<T> *tw1,
+                    const ChanPlan &cp, int p0, int nb, hipStream_t st);
+// checks a plan against the kernels' launch limits and raises their dynamic LDS
+template <typename T> int allow_mix(const ChanPlan &cp);
 
 }  // namespace curig

@@ -70,3 +70,51 @@ def test_columns_of_every_length(precision, nx, ny, wmax):
     say(f"[columns] {precision} {nx}x{ny} wmax {wmax}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
     tol = 1e-11 if precision == "fp64" else 2e-6
     assert e1 < tol and e2 < tol
+
+
+# mixed-radix grids (axes 2^a 3^b 5^c, not both powers of two, or an image wider
+# than half the grid): rows sharing a workgroup with a short last one, column
+# tiles with a short last one, one and several stages, a kernel that wraps past
+# a last block of fewer than 16 cells, long axes near the LDS limit, kernels of
+# up to 16, upsampling 1.25, more than one batch of planes
+MIXED = [
+    # precision, nx, ny, eps, sigma, wmax
+    ("fp64", 25, 31, 1e-6, 2.0, 400.0), ("fp32", 25, 31, 1e-6, 2.0, 400.0),
+    ("fp64", 75, 1125, 1e-6, 2.0, 300.0), ("fp32", 75, 1125, 1e-6, 2.0, 300.0),
+    ("fp32", 1500, 75, 1e-5, 2.0, 300.0), ("fp64", 1499, 77, 1e-12, 2.0, 300.0),
+    ("fp64", 3000, 40, 1e-6, 2.0, 200.0), ("fp64", 40, 3000, 1e-6, 2.0, 200.0),
+    ("fp32", 6000, 48, 1e-6, 2.0, 100.0), ("fp32", 48, 6000, 1e-6, 2.0, 100.0),
+    ("fp32", 90, 7300, 1e-6, 2.0, 100.0), ("fp32", 7300, 90, 1e-6, 2.0, 100.0),
+    ("fp64", 512, 512, 1e-6, 1.25, 500.0), ("fp32", 500, 819, 1e-4, 1.25, 500.0),
+    ("fp64", 100, 100, 1e-6, 2.0, 9000.0), ("fp32", 1024, 100, 1e-6, 2.0, 900.0),
+]
+
+
+@pytest.mark.parametrize("case", MIXED, ids=[f"{c[0]}-{c[1]}x{c[2]}-{c[3]:g}-{c[4]:g}" for c in MIXED])
+def test_mixed_radix_grids(case):
+    from curig_amd import _lib as L
+
+    precision, nx, ny, eps, sigma, wmax = case
+    fov = 2.0
+    uvw, vis, wgt, img, f0 = _case(3000, nx, ny, fov, wmax, nx + 7 * ny, span=1.4)
+    info = L.plan_info(len(uvw), nx, ny, fov, f0, eps, sigma, -1, float(uvw[:, 2].min()), float(uvw[:, 2].max()),
+                       0 if precision == "fp64" else 1)
+    assert info["fft_lds"] == 1
+    e1, e2 = _both_paths(precision, uvw, vis, wgt, img, nx, ny, fov, f0, eps, sigma)
+    say(f"[mixed radix] {case} grid {info['nf2']}x{info['nf1']}x{info['nf3']}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
+    # FP32 at upsampling 1.25: the corrections amplify both sides' rounding
+    tol = 1e-10 if precision == "fp64" else 2e-6 if sigma == 2.0 else 2e-5
+    assert e1 < tol and e2 < tol
+
+
+def test_mixed_radix_empty_rows_and_non_finite_values():
+    """A few visibilities (most rows of most planes empty), and an infinite one:
+    the image is then not finite, as on the rocFFT path."""
+    nx, ny, fov, eps = 300, 250, 2.0, 1e-6
+    for precision in ("fp64", "fp32"):
+        uvw, vis, wgt, img, f0 = _case(5, nx, ny, fov, 2000.0, 3)
+        e1, e2 = _both_paths(precision, uvw, vis, wgt, img, nx, ny, fov, f0, eps)
+        assert e1 < 2e-6 and e2 < 2e-6
+        vis[2] = np.inf
+        d = (gpu_ms2dirty if precision == "fp64" else (lambda *a: gpu_f32(True, *a)))(uvw, vis, wgt, nx, ny, fov, f0, eps)
+        assert not np.isfinite(d).any()
