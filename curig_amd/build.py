@@ -15,7 +15,8 @@ INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(HERE, "libcurafft.so")
 OBJDIR = os.path.join(HERE, "_build")
 SOURCES = ["kern_lds_spread_f32.hip", "kern_lds_interp_f32.hip", "kern_lds_cols_f32.hip", "kern_lds_spread_f64.hip",
-           "kern_lds_interp_f64.hip", "kern_lds_cols_f64.hip", "kern_mix_f32.hip", "kern_mix_f64.hip", "kern_plane.hip", "kern_prep.hip", "gridder.hip",
+           "kern_lds_interp_f64.hip", "kern_lds_cols_f64.hip", "kern_mix_f32.hip", "kern_mix_f64.hip",
+           "kern_rowreg_f32.hip", "kern_rowreg_f64.hip", "kern_plane.hip", "kern_prep.hip", "gridder.hip",
            "plan_math.cpp", "fft.cpp", "capi.cpp"]
 ARCH = os.environ.get("CURIG_OFFLOAD_ARCH", "gfx950")
 

@@ -97,8 +97,12 @@ struct Geom {
   // pruned LDS FFT path (power-of-two grids); fft_lds == 0 selects rocFFT
   int fft_lds;
   int mix;            // LDS path on axes 2^a 3^b 5^c (mixed-radix kernels), else powers of two
+  int rowreg;         // whole power-of-two rows in the kernels of kern_rowreg.h
+  int acc64;          // ms2dirty, FP32, dense records: rows summed in FP64 (rowreg and mix)
+  int zrow;           // ms2dirty: workgroups that share the records of a row group (rowreg and mix)
   int nt_row, nt_col; // its threads per row and column workgroup
   int pch_row;        // its planes per row workgroup
+  int gather;         // dirty2ms: rows written out as full planes, each record's cells gathered from them
   int rpw;            // grid rows per workgroup in the row pass (rpw * nf1 = 16 * threads)
   int cpw;            // grid columns per workgroup in the column pass (cpw * nf2 = 16 * threads)
   int cpw_inv;        // the same for the dirty2ms column pass (whole column tiles where they fit)

@@ -8,6 +8,8 @@
 // runs: they are read once and held.  One workgroup may run several
 // transforms side by side (its barriers cover all of them).
 #pragma once
+#include <type_traits>
+
 #include "dev_common.h"
 
 namespace curig {
@@ -178,6 +180,11 @@ template <typename T, int N, int SIGN, int TW = kTwHeld> struct RegFft {
     stage<16>(v, buf, j);
   }
 };
+
+// element e = q or q + 8 of RegFft's sixteen that can be an image row or column:
+// with the image at most half the grid, its grid indices lie in the first and
+// last quarter
+__device__ __forceinline__ constexpr int image_elem(int q) { return q < 4 ? q : q + 8; }
 
 // f(std::integral_constant<int, N>()) for the supported lengths
 template <typename F> inline bool with_reg_fft(int n, F f) {

@@ -289,8 +289,9 @@ static void plan_columns(Geom &g, size_t cs, size_t lds_max, bool compact) {
     // column each, share lines of H in fours, and the further they drift apart
     // over the planes the more partial lines the L2 writes back (8192^2, 32
     // planes: 19.9 ms walking all planes, 17.7, 13.9 and 16.1 ms in chunks of 8,
-    // 4 and 2; a chunk's setup costs about one plane)
-    g.pch_inv = std::min(4, g.Pb);
+    // 4 and 2; a chunk's setup costs about one plane; FP64 stores whole 64-byte
+    // pieces)
+    if (cs == 8) g.pch_inv = std::min(4, g.Pb);
     g.lds_col_bytes = (int)colreg_lds_bytes(cs);
     return;
   }
@@ -352,6 +353,11 @@ static int mixed_threads(int n, int count, int max_threads, int min_threads) {
 // points), kernels wider than 16, and grids of few rows (a one-dimensional
 // transform's 2 kw rows: the row workgroups would hold all its points).
 static void plan_mixed(Geom &g, size_t cs, size_t lds_max) {
+  // FP32 with the image beyond half the grid keeps the full planes: its
+  // corrections amplify rounding up to 1e-4 of the result, and another
+  // transform's rounding is as far from the present results as they are from
+  // the exact ones
+  if (cs == 8 && (2 * g.N1 > g.nf1 || 2 * g.N2 > g.nf2)) return;
   if (!fftm::smooth235(g.nf1) || !fftm::smooth235(g.nf2) || g.nf1 < 16 || g.nf2 < 40 || g.N1 > g.nf1 || g.N2 > g.nf2)
     return;
   const size_t room = lds_max > 8192 ? lds_max - 8192 : 0;  // walk tables, block table beside the rows
@@ -490,8 +496,11 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   g.rpw = g.cpw = g.nct = g.tstride = g.nslot = g.slot_lg = g.lds_row_bytes = g.lds_col_bytes = g.rsplit =
       g.lds_rowp_bytes = g.colreg = g.cpw_inv = g.pch_fwd = g.pch_inv = 0;
   g.nacc = 1;
-  g.mix = g.nt_row = g.nt_col = g.pch_row = 0;
+  g.mix = g.nt_row = g.nt_col = g.pch_row = g.gather = g.rowreg = g.acc64 = 0;
+  g.zrow = 1;
   auto pow2 = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
+  // record visits per grid row and plane
+  const double visits = (double)nrow_valid * g.kw * g.kww / ((double)g.P * g.nf2);
   const size_t cs = dbl ? 16 : 8;
   const size_t lds_max = tn.lds_bytes > 0 ? (size_t)tn.lds_bytes : size_t(160) << 10;
   const int max_threads = dbl ? 512 : 1024;
@@ -506,13 +515,11 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     // plane-loop row kernels, all others kRowSplit ways.  Halves against whole
     // rows: 4 channels of 4096^2 (90 planes, ~80 record visits per row and
     // plane) 5.1 against 8.1 ms per launch (ms2dirty), a dirty2ms call 115
-    // against 153 ms.  Each part adds its own share of every visit to the
-    // record's accumulator, so dirty2ms keeps dense rows whole: the one plane of
-    // a 20M-point 2-D transform (15,000 visits per row) took 6.8 ms in halves
-    // against 3.4; equal near 1,000 visits.  ms2dirty has halves ahead there
-    // too (5.8 against 7.3 ms: integer LDS atomics).
-    const double visits = (double)nrow_valid * g.kw * g.kww / ((double)g.P * g.nf2);
-    const bool halves = !dbl && g.nf1 == 8192 && !tn.compact && (!tn.to_vis || visits <= 1024);
+    // against 153 ms.  Halves read every record twice, so dense rows stay whole:
+    // the one plane of a 20M-point 2-D transform (15,000 visits per row) took 5.7
+    // ms in halves against 2.7 (ms2dirty), 6.8 against 3.4 (dirty2ms, equal near
+    // 1,000 visits).
+    const bool halves = !dbl && g.nf1 == 8192 && !tn.compact && visits <= 1000;
     const int split = halves ? 2 : kRowSplit;
     const size_t rbp = (size_t)(fftc::padded_size(g.nf1 / split) + fftc::twiddle_entries(g.nf1)) * cs;
     const bool row_whole = rb + 2048 <= lds_max && rpw * g.nf1 / 16 <= max_threads;
@@ -540,10 +547,43 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     }
   }
   if (!g.fft_lds && tn.fft != 1 && !tn.compact && g.kw <= 16) plan_mixed(g, cs, lds_max);
+  if (g.fft_lds) {
+    // Dense records: dirty2ms writes the planes' rows out and gathers each
+    // record's cells once.  The fused row pass visits a record in every row and
+    // plane of its support with two FP64 atomics each; the gather pays one write
+    // and read of the planes.  Both sides, interpolation kernels only, by record
+    // visits (nvalid kw kww) per grid cell: 0.02 (1500 x 1100 FP32) 0.95 against
+    // 0.97 ms per launch, 0.17 (3000^2 modes, 1M points) 0.34 / 0.40 ms, 0.5 (600^2
+    // FP64) 0.85 / 0.38, 0.8 (3000^2, 5M) 0.96 / 0.73, 13 (1500^2, 20M) 4.3 / 1.7.
+    const bool rows = g.mix || (pow2(g.nf1) && !g.rsplit);
+    g.gather = tn.to_vis && rows && !tn.compact &&
+               nrow_valid * (double)g.kw * g.kww > 0.3 * g.P * (double)g.nf1 * g.nf2;
+    // FP32 rows with many records are summed in FP64 (twice the LDS, no bound
+    // pass): by record visits per row and plane, FP64 against integer sums, 41
+    // (1500 x 1100) 1.27 / 1.08 ms, 615 (1024^2, 33 planes) 0.76 / 0.77, 2,000
+    // (1500^2 modes, 1M points) 0.21 / 0.23, 15,000 (4096^2, 20M) 2.7 / 4.0 ms; up
+    // to 1024 cells, where a row takes little LDS anyway, 190 (256^2 image) 77 /
+    // 138 us.  The integers' bound grows with a block's records, their sum with
+    // the square root: error against 64 bits, thousands of records per block
+    // (uv data within 2.4% of a 512^2 grid), 1.4e-6 in integers, 1.3e-7 in FP64.
+    const bool few_cells = g.nf1 <= 1024;
+    const bool dense = !dbl && !tn.to_vis && rows && visits > (g.nf1 >= 4096 ? 1000 : few_cells ? 100 : 600);
+    if (!g.mix && !g.rsplit && (g.nf1 <= 2048 || g.nf1 == 8192 || g.gather || dense)) {
+      g.rowreg = 1;
+      // 256 threads, or one row's; fewer while that leaves fewer than 1024
+      // workgroups (one wavefront at least)
+      const int G = g.nf1 / 16;
+      int r = std::max(1, (dbl ? 128 : 256) / G);
+      while (r > 1 && (r / 2) * G >= 64 && g.nf2 / r < 1024) r /= 2;
+      while (r * G < 64) r *= 2;
+      g.rpw = std::min(r, g.nf2);
+    }
+    if (dense && (size_t)g.rpw * (g.nf1 + g.nf1 / 16 + 16) * 16 + 8192 <= lds_max) g.acc64 = 1;
+  }
   // planes per batch from the memory budget: full planes (rocFFT path) or, on
   // the LDS path, the compact plane plus the one or two column-pass buffers
   size_t per_plane = (size_t)g.nf1 * g.nf2 * cs;
-  if (g.fft_lds) per_plane = (size_t)g.nct * g.tstride * cs;
+  if (g.fft_lds) per_plane = (size_t)g.nct * g.tstride * cs + (g.gather ? (size_t)g.nf1 * g.nf2 * cs : 0);
   int Pb = tn.Pb;
   if (Pb <= 0) {
     Pb = (int)std::max<size_t>(1, tn.grid_budget_bytes / per_plane);
@@ -555,6 +595,18 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     plan_mixed_chunks(g);
   else if (g.fft_lds)
     plan_columns(g, cs, lds_max, tn.compact != 0);
+  if (g.rowreg) {
+    const int groups = g.nf2 / g.rpw, n = std::min((1024 + groups - 1) / groups, 8);
+    g.pch_row = std::max(std::min(2, g.Pb), (g.Pb + n - 1) / n);
+  }
+  if ((g.rowreg || g.mix) && !tn.to_vis) {
+    // Few row workgroups with many records each (a small grid, one plane): they
+    // are shared by zrow workgroups, at least 4096 record visits each, whose
+    // transforms add up in H (5M points on 128^2 modes: 12.9 -> 0.7 ms)
+    const double groups = (double)((g.nf2 + g.rpw - 1) / g.rpw) * ((g.Pb + g.pch_row - 1) / g.pch_row);
+    const double per_group = (double)nrow_valid * g.kww * (g.kw + g.rpw - 1) / ((double)g.P * g.nf2) * g.pch_row;
+    if (groups < 1024) g.zrow = std::max(1, (int)std::min({std::ceil(1024 / groups), per_group / 4096, 64.0}));
+  }
   // bins: full-width row strips for the LDS path (one workgroup owns grid rows),
   // T1 x T2 tiles for the tile-owner spread
   if (g.fft_lds) {
@@ -738,7 +790,7 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image,
     nrow = std::max(nrow, (size_t)std::max(pbs[i].nrow, 1));
     nvalid = std::max(nvalid, (size_t)std::max<long>(cps[i].nvalid, 1));
     const size_t plane = (size_t)g.nf1 * g.nf2, pix = (size_t)g.N1 * g.N2;
-    if (!g.fft_lds) grid = std::max(grid, plane * g.Pb);
+    if (!g.fft_lds || g.gather) grid = std::max(grid, plane * g.Pb);
     if (g.fft_lds) h = std::max(h, (size_t)g.nct * g.tstride * g.Pb);
     npix = std::max(npix, pix * (to_image ? g.nacc : 1));
   }
@@ -803,7 +855,10 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image,
         CURIG_TRY(allow_mix<T>(cp));
         continue;
       }
-      CURIG_TRY(to_image ? allow_spread_rows<T>(cp.g) : allow_row_interp<T>(cp.g));
+      if (cp.g.rowreg)
+        CURIG_TRY(allow_rowreg<T>(cp.g, to_image));
+      else
+        CURIG_TRY(to_image ? allow_spread_rows<T>(cp.g) : allow_row_interp<T>(cp.g));
       CURIG_TRY(allow_cols<T>(cp.g));
     }
   } else {
@@ -886,6 +941,8 @@ int enqueue_ms2dirty(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
       // the w-accumulation as FFT (t_fft)
       if (g.mix)
         mix_spread_rows<T>(recs, (const T *)b.taps, b.off, cp, p0, nb, (cpx<T> *)b.H, (const cpx<T> *)b.tw1, st);
+      else if (g.rowreg)
+        rowreg_spread<T>(recs, (const T *)b.taps, b.off, g, p0, nb, (cpx<T> *)b.H, (const cpx<T> *)b.tw1, st);
       else
         lds_spread_rows<T>(recs, (const T *)b.taps, b.off, g, p0, nb, (cpx<T> *)b.H, (const cpx<T> *)b.tw1, st);
       CURIG_HIP(hipGetLastError());
@@ -969,8 +1026,11 @@ int enqueue_dirty2ms(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
       CURIG_HIP(hipGetLastError());
       const int c = tm.mark();
       if (cp.nvalid > 0 && g.mix)
-        mix_row_interp<T>(recs, (const T *)b.taps, b.off, (const cpx<T> *)b.H, b.vacc, (const cpx<T> *)b.tw1, cp, p0, nb,
-                          st);
+        mix_row_interp<T>(recs, (const T *)b.taps, b.off, (const cpx<T> *)b.H, b.grid, b.vacc, (const cpx<T> *)b.tw1, cp,
+                          p0, nb, st);
+      else if (cp.nvalid > 0 && g.rowreg)
+        rowreg_interp<T>(recs, (const T *)b.taps, b.off, (const cpx<T> *)b.H, b.grid, b.vacc, (const cpx<T> *)b.tw1, g,
+                         cp.nvalid, p0, nb, st);
       else if (cp.nvalid > 0)
         lds_row_interp<T>(recs, (const T *)b.taps, b.off, (const cpx<T> *)b.H, b.vacc, (const cpx<T> *)b.tw1, g, p0,
                           nb, st);
@@ -1058,7 +1118,7 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
+      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
   k << b.dev << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc

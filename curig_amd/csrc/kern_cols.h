@@ -35,10 +35,6 @@ template <typename T, int N> struct ColCfg {
   static size_t inv_lds(int cpw) { return sizeof(cpx<T>) * (size_t)(cpw * Inv::kStride + Inv::kTwLds); }
 };
 
-// element e = q or q + 8 of RegFft's sixteen that can be an image row: with
-// 2 N2 <= nf2 the image rows' grid indices lie in the first and last quarter
-__device__ __forceinline__ constexpr int image_elem(int q) { return q < 4 ? q : q + 8; }
-
 // ms2dirty column pass fused with the w-accumulation (w_term_dft, cuft.cu:520-572):
 // a workgroup owns cpw columns and walks planes [blockIdx.y pchunk, + pchunk) of
 // the batch's nb, last to first: load the row-transformed columns, FFT over nf2,

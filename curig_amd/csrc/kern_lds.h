@@ -157,38 +157,6 @@ __device__ __forceinline__ fftc::TwoLevel<T, const cpx<T> *> lds_twiddles(cpx<T>
   return fftc::TwoLevel<T, const cpx<T> *>{dst, dst + nhi, lb};
 }
 
-template <typename T, int E, int MAXR = 16, typename Tw>
-__device__ __forceinline__ void lds_fft(cpx<T> *buf, const fftc::Layout &L, int sign, const Tw tw, int n_tw) {
-  cpx<T> v[E];
-  const int nt = blockDim.x;
-  for (int Ns = 1; Ns < L.n;) {
-    const int R = fftc::stage_radix(L.n, Ns, MAXR);
-    // opaque copy of the thread id: keeps each stage's address arithmetic inside
-    // the stage (hoisted out of the loop it is held for all stages and spills)
-    int tid = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid));
-    if (R == 16)
-      fftc::stage_load<T, E, 16>(buf, v, L, Ns, sign, tw, n_tw, tid, nt);
-    else if (R == 8)
-      fftc::stage_load<T, E, 8>(buf, v, L, Ns, sign, tw, n_tw, tid, nt);
-    else if (R == 4)
-      fftc::stage_load<T, E, 4>(buf, v, L, Ns, sign, tw, n_tw, tid, nt);
-    else
-      fftc::stage_load<T, E, 2>(buf, v, L, Ns, sign, tw, n_tw, tid, nt);
-    __syncthreads();
-    if (R == 16)
-      fftc::stage_store<T, E, 16>(buf, v, L, Ns, tid, nt);
-    else if (R == 8)
-      fftc::stage_store<T, E, 8>(buf, v, L, Ns, tid, nt);
-    else if (R == 4)
-      fftc::stage_store<T, E, 4>(buf, v, L, Ns, tid, nt);
-    else
-      fftc::stage_store<T, E, 2>(buf, v, L, Ns, tid, nt);
-    __syncthreads();
-    Ns *= R;
-  }
-}
-
 // Stockham stages of `count` contiguous length-N sequences (buffer index
 // pad(s * N + k)) with N a compile-time constant: every stage's radix, stride
 // and twiddle step fold to constants, and the element indexing to shifts.
@@ -396,22 +364,6 @@ __device__ __forceinline__ void fft4096_part_to_regs(cpx<T> *buf, cpx<T> *v, int
   fftc::dft_small<T, 16>(v, sign);
 }
 
-// FFT of `count` contiguous sequences of length n = 2^lg (6 <= lg <= 14) in LDS.
-template <typename T, int E, int MAXR, typename Tw>
-__device__ __forceinline__ void lds_fft_rows(cpx<T> *buf, int lg, int count, int sign, const Tw &tw) {
-  switch (lg) {
-    case 6: fixed_stages<T, E, MAXR, 64, 1>(buf, count, sign, tw); break;
-    case 7: fixed_stages<T, E, MAXR, 128, 1>(buf, count, sign, tw); break;
-    case 8: fixed_stages<T, E, MAXR, 256, 1>(buf, count, sign, tw); break;
-    case 9: fixed_stages<T, E, MAXR, 512, 1>(buf, count, sign, tw); break;
-    case 10: fixed_stages<T, E, MAXR, 1024, 1>(buf, count, sign, tw); break;
-    case 11: fixed_stages<T, E, MAXR, 2048, 1>(buf, count, sign, tw); break;
-    case 12: fixed_stages<T, E, MAXR, 4096, 1>(buf, count, sign, tw); break;
-    case 13: fixed_stages<T, E, MAXR, 8192, 1>(buf, count, sign, tw); break;
-    default: fixed_stages<T, E, MAXR, 16384, 1>(buf, count, sign, tw); break;
-  }
-}
-
 __device__ __forceinline__ int image_index(int k, int N, int nf) {
   // grid index (FFT order) -> image index (centred), or -1 outside the image
   const int h = N / 2;
@@ -454,78 +406,6 @@ template <typename T, int KWM> __device__ __forceinline__ T sel_tap(const T *a, 
   }
   return r;
 }
-
-// Spread of one record into the workgroup's grid rows [row0, row0 + rpw) of plane p (LDS).
-template <typename T, int KWM>
-__device__ __forceinline__ void spread_rows(const Rec<T> rc, const Taps<T, KWM> &tp, T *ldsf, const Geom &g, int p,
-                                            int row0) {
-  const int kw = g.kw, nf1 = g.nf1, nf2 = g.nf2, rpw = g.rpw;
-  int k = p - rc.iw;
-  if (k < 0) k += g.P;
-  if (k >= g.kww) return;
-  int ry = rc.iy - row0;
-  if (ry < 0) ry += nf2;
-  if (!(ry < rpw || ry + kw - 1 >= nf2)) return;
-  const T vw = sel_tap<T, KWM>(tp.z, k);
-  const T vre = rc.re * vw, vim = rc.im * vw;
-  for (int jj = 0; jj < kw; ++jj) {
-    int cy = ry + jj;
-    if (cy >= nf2) cy -= nf2;
-    if (cy >= rpw) continue;
-    const T ky = sel_tap<T, KWM>(tp.y, jj);
-    const T are = vre * ky, aim = vim * ky;
-    const int base = cy * nf1;
-#pragma unroll
-    for (int i = 0; i < KWM; ++i) {
-      if (i < kw) {
-        int cx = rc.ix + i;
-        if (cx >= nf1) cx -= nf1;
-        const int a = 2 * fftc::pad(base + cx);
-        atomicAdd(ldsf + a, are * tp.x[i]);
-        atomicAdd(ldsf + a + 1, aim * tp.x[i]);
-      }
-    }
-  }
-}
-
-// Interpolation of one record from the workgroup's rows of plane p (LDS): its
-// partial sum over those rows, added to the record's FP64 accumulator.
-template <typename T, int KWM>
-__device__ __forceinline__ void interp_rows(const Rec<T> rc, const Taps<T, KWM> &tp, int idx, const cpx<T> *lds,
-                                            const Geom &g, int p, int row0, double2 *__restrict__ vacc) {
-  const int kw = g.kw, nf1 = g.nf1, nf2 = g.nf2, rpw = g.rpw;
-  int k = p - rc.iw;
-  if (k < 0) k += g.P;
-  if (k >= g.kww) return;
-  int ry = rc.iy - row0;
-  if (ry < 0) ry += nf2;
-  if (!(ry < rpw || ry + kw - 1 >= nf2)) return;
-  T sr = 0, si = 0;
-  for (int jj = 0; jj < kw; ++jj) {
-    int cy = ry + jj;
-    if (cy >= nf2) cy -= nf2;
-    if (cy >= rpw) continue;
-    const int base = cy * nf1;
-    T rr = 0, ri = 0;
-#pragma unroll
-    for (int i = 0; i < KWM; ++i) {
-      if (i < kw) {
-        int cx = rc.ix + i;
-        if (cx >= nf1) cx -= nf1;
-        const cpx<T> f = lds[fftc::pad(base + cx)];
-        rr += f.x * tp.x[i];
-        ri += f.y * tp.x[i];
-      }
-    }
-    const T ky = sel_tap<T, KWM>(tp.y, jj);
-    sr += rr * ky;
-    si += ri * ky;
-  }
-  const T kz = sel_tap<T, KWM>(tp.z, k);
-  atomicAdd(&vacc[idx].x, (double)(sr * kz));
-  atomicAdd(&vacc[idx].y, (double)(si * kz));
-}
-
 
 // The intermediate planes live in a column-tiled layout: element (plane k,
 // grid row k2, column slot s) at (k * nct + s / kTile) * tstride + k2 * kTile
@@ -580,133 +460,6 @@ __device__ __forceinline__ int xcd_interleave(int bid, int n, int blk) {
   if (n % (8 * blk)) return xcd_group(bid, n);
   const int x = bid & 7, k = bid >> 3;
   return ((k / blk) * 8 + x) * blk + k % blk;
-}
-
-template <typename T> struct MaxThreads { static constexpr int value = sizeof(T) == 8 ? 512 : 1024; };
-
-// ms2dirty: spread into full grid rows held in LDS, then the row FFT (length
-// nf1), keeping the N1 image columns, written to the column-tiled layout H.  One
-// workgroup owns rpw rows of one w plane (rpw * nf1 = E * blockDim.x); rows are
-// binned into full-width strips of T2 rows.
-template <typename T, int E, int KWM>
-__global__ void __launch_bounds__(MaxThreads<T>::value) spread_row_fft_kernel(const Rec<T> *__restrict__ recs,
-                                                                             const T *__restrict__ taps,
-                                                                             const int *__restrict__ off,
-                                                                             cpx<T> *__restrict__ H,
-                                                                             const cpx<T> *__restrict__ tw, Geom g,
-                                                                             int p0) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ WalkTable wt;
-  cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
-  T *ldsf = reinterpret_cast<T *>(smem_raw);
-  const int rpw = g.rpw, nf1 = g.nf1, nt = blockDim.x;
-  // rows in XCD-contiguous order: the rows sharing a tile's lines are written
-  // through one L2, which merges their chunks into whole lines
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, pl = blockIdx.y, p = p0 + pl;
-  const int ntot = fftc::padded_size(rpw * nf1);
-  const auto tv = lds_twiddles<T>(lds + ntot, tw, nf1);
-  if (threadIdx.x < 64) walk_table_build(wt, off, g, p, row0, rpw);
-  for (int i = threadIdx.x; i < ntot; i += nt) lds[i] = fftc::mk((T)0, (T)0);
-  __syncthreads();
-  const int total = wt.total;
-  const int N1 = g.N1, nout = rpw * N1, h1 = N1 / 2;
-  cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
-  if (total == 0) {
-    // no visibility reaches these rows of this plane: the transform is zero
-    for (int i = threadIdx.x; i < nout; i += nt) {
-      const int r = rpw == 1 ? 0 : i / N1, col = i - r * N1;
-      hb[h_slot(g, col) + (r << kTileLog2)] = fftc::mk((T)0, (T)0);
-    }
-    return;
-  }
-  for (int t0 = threadIdx.x; t0 < total; t0 += nt) {
-    const int ia = walk_record(wt, t0);
-    const Rec<T> ra = recs[ia];
-    Taps<T, KWM> ta;
-    load_taps<T, KWM>(taps, ia, ta);
-    spread_rows<T, KWM>(ra, ta, ldsf, g, p, row0);
-  }
-  __syncthreads();
-  lds_fft_rows<T, E, 16>(lds, 31 - __clz(nf1), rpw, +1, tv);
-  // pruned write: all LDS reads first, then the stores (kTile-column chunks);
-  // offsets from the row's base in 32 bits (a plane holds < 2^31 elements)
-  int tid = threadIdx.x;
-  __asm__ volatile("" : "+v"(tid));
-  cpx<T> o[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int i = tid + e * nt;
-    if (i < nout) {
-      const int r = rpw == 1 ? 0 : i / N1, col = i - r * N1;
-      const int k1 = col >= h1 ? col - h1 : nf1 + col - h1;
-      o[e] = lds[fftc::pad(r * nf1 + k1)];
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int i = tid + e * nt;
-    if (i < nout) {
-      const int r = rpw == 1 ? 0 : i / N1, col = i - r * N1;
-      hb[h_slot(g, col) + (r << kTileLog2)] = o[e];
-    }
-  }
-}
-
-
-// dirty2ms: row pass of the column-transformed planes (H as col_inv_kernel
-// writes it; each row expanded to nf1 cells, zero outside the image columns),
-// inverse row FFT in LDS, then interpolation of every record touching the workgroup's rows of
-// plane p: per record a partial sum, added to its FP64 accumulator (atomics),
-// so the full grid planes are never written.
-template <typename T, int E, int KWM>
-__global__ void __launch_bounds__(MaxThreads<T>::value) row_ifft_interp_kernel(const cpx<T> *__restrict__ H,
-                                                                              const Rec<T> *__restrict__ recs,
-                                                                              const T *__restrict__ taps,
-                                                                              const int *__restrict__ off,
-                                                                              double2 *__restrict__ vacc,
-                                                                              const cpx<T> *__restrict__ tw,
-                                                                              Geom g, int p0, int sign) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ WalkTable wt;
-  cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
-  const int rpw = g.rpw, nf1 = g.nf1, N1 = g.N1, nt = blockDim.x;
-  // rows in XCD-contiguous order: the 16 rows sharing a column line run together
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, pl = blockIdx.y, p = p0 + pl;
-  const int lg = 31 - __clz(nf1);
-  cpx<T> v[E];
-  const cpx<T> *hb = H + h_plane(g, pl);
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int i = threadIdx.x + e * nt;  // < rpw * nf1 = E * nt
-    const int r = i >> lg, k1 = i & (nf1 - 1);
-    const int col = image_index(k1, N1, nf1);
-    v[e] = col >= 0 ? hb[ht_slot(g, col) + ht_row(row0 + r)]
-                    : fftc::mk((T)0, (T)0);
-  }
-  const auto tv = lds_twiddles<T>(lds + fftc::padded_size(rpw * nf1), tw, nf1);
-  if (threadIdx.x < 64) walk_table_build(wt, off, g, p, row0, rpw);
-#pragma unroll
-  for (int e = 0; e < E; ++e) lds[fftc::pad(threadIdx.x + e * nt)] = v[e];
-  __syncthreads();
-  const int total = wt.total;
-  if (total == 0) return;  // no visibility reaches these rows of this plane
-  // first record of this thread, loaded while the FFT runs
-  int idx0 = 0;
-  Rec<T> r0;
-  Taps<T, KWM> q0;
-  if (threadIdx.x < total) {
-    idx0 = walk_record(wt, threadIdx.x);
-    r0 = recs[idx0];
-    load_taps<T, KWM>(taps, idx0, q0);
-  }
-  lds_fft_rows<T, E, 16>(lds, lg, rpw, sign, tv);
-  if (threadIdx.x < total) interp_rows<T, KWM>(r0, q0, idx0, lds, g, p, row0, vacc);
-  for (int t = threadIdx.x + nt; t < total; t += nt) {
-    const int idx = walk_record(wt, t);
-    Taps<T, KWM> q;
-    load_taps<T, KWM>(taps, idx, q);
-    interp_rows<T, KWM>(recs[idx], q, idx, lds, g, p, row0, vacc);
-  }
 }
 
 // Spread of one record into part h of a row split S ways (ms2dirty): part h
@@ -1524,18 +1277,10 @@ void lds_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const Ge
       spread_row_part_planes_kernel<T, 16, 16, 1><<<g.nf2, 256, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
     return;
   }
-  const dim3 grd(g.nf2 / g.rpw, nb);
-  const int nt = g.rpw * g.nf1 / 16;
-  if (g.kw <= 8)
-    spread_row_fft_kernel<T, 16, 8><<<grd, nt, g.lds_row_bytes, st>>>(recs, taps, off, H, tw1, g, p0);
-  else
-    spread_row_fft_kernel<T, 16, 16><<<grd, nt, g.lds_row_bytes, st>>>(recs, taps, off, H, tw1, g, p0);
 }
 
 template <typename T>
 int allow_spread_rows(const Geom &g) {
-  CURIG_TRY(allow_lds(spread_row_fft_kernel<T, 16, 8>, g.lds_row_bytes));
-  CURIG_TRY(allow_lds(spread_row_fft_kernel<T, 16, 16>, g.lds_row_bytes));
   if (whole_row_planes<T>(g)) {
     const int lb = g.lds_row_bytes;
     CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 8, 1>, lb)));
@@ -1591,18 +1336,10 @@ void lds_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx
       row_ifft_interp_part_kernel<T, 16, 16, kRowSplit><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, -1);
     return;
   }
-  const dim3 grd(g.nf2 / g.rpw, nb);
-  const int nt = g.rpw * g.nf1 / 16;
-  if (g.kw <= 8)
-    row_ifft_interp_kernel<T, 16, 8><<<grd, nt, g.lds_row_bytes, st>>>(H, recs, taps, off, vacc, tw1, g, p0, -1);
-  else
-    row_ifft_interp_kernel<T, 16, 16><<<grd, nt, g.lds_row_bytes, st>>>(H, recs, taps, off, vacc, tw1, g, p0, -1);
 }
 
 template <typename T>
 int allow_row_interp(const Geom &g) {
-  CURIG_TRY(allow_lds(row_ifft_interp_kernel<T, 16, 8>, g.lds_row_bytes));
-  CURIG_TRY(allow_lds(row_ifft_interp_kernel<T, 16, 16>, g.lds_row_bytes));
   if (interp_planes<T>(g)) {
     const bool s1 = g.rsplit <= 1;
     const int lb = s1 ? g.lds_row_bytes : g.lds_rowp_bytes;

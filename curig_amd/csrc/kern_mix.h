@@ -10,17 +10,13 @@
 // element: butterflies, twiddles and the run-time index arithmetic) and its LDS
 // passes, with one workgroup's memory phases behind another's transform.
 #pragma once
-#include "kern_lds.h"
+#include "kern_rows.h"
 
 #include "fft_mix.h"
 
 namespace curig {
 
 template <typename T> struct MixThreads { static constexpr int value = sizeof(T) == 8 ? 512 : 1024; };
-
-// LDS of a row workgroup: the rows, the axis' twiddles and (FP32) the block
-// table of the block-floating-point spread.
-__host__ __device__ inline int mix_blocks(int nf1) { return (nf1 + (1 << kFixBlkLog2) - 1) >> kFixBlkLog2; }
 
 // stages [s0, P.ns) of the transform; the caller's barrier precedes it, a
 // barrier ends it
@@ -44,10 +40,12 @@ __device__ __forceinline__ void mix_stages(cpx<T> *buf, const fftm::Plan &P, con
   }
 }
 
-// the first stage on the integers of the block-floating-point spread: cell k of
-// sequence q in block k >> kFixBlkLog2 of exponent fexp[q * nblk + block]
-template <typename T, int SIGN, typename Tw>
-__device__ __forceinline__ void mix_first_fix(cpx<T> *buf, const fftm::Plan &P, const Tw &tw, const short *fexp, int nblk) {
+// the first stage on the spread's cells: integers scaled by block (cell k of
+// sequence q in block k >> kFixBlkLog2 of exponent fexp[q * nblk + block]), or
+// FP64 sums whose first half the transform then runs in
+template <typename T, int SIGN, bool ACC64, typename Tw>
+__device__ __forceinline__ void mix_first_cells(cpx<T> *buf, const typename RowAcc<T, ACC64>::cell *acc, const fftm::Plan &P,
+                                                const Tw &tw, const short *fexp, int nblk) {
   int tid = threadIdx.x;
   __asm__ volatile("" : "+v"(tid));
   fftm::with_radix(P.R[0], [&](auto tag) {
@@ -55,9 +53,14 @@ __device__ __forceinline__ void mix_first_fix(cpx<T> *buf, const fftm::Plan &P, 
     cpx<T> v[RR * fftm::radix_nb(RR)];
     fftm::stage_load<T, RR, SIGN>(
         [&](int q, int k) {
-          const int2 x = reinterpret_cast<const int2 *>(buf)[q * P.stride + fftc::pad(k)];
-          const int e = fexp[q * nblk + (k >> kFixBlkLog2)];
-          return fftc::mk((T)ldexpf((float)x.x, -e), (T)ldexpf((float)x.y, -e));
+          const int at = q * P.stride + fftc::pad(k);
+          if constexpr (RowAcc<T, ACC64>::fix) {
+            const int2 x = reinterpret_cast<const int2 *>(buf)[at];
+            const int e = fexp[q * nblk + (k >> kFixBlkLog2)];
+            return fftc::mk((T)ldexpf((float)x.x, -e), (T)ldexpf((float)x.y, -e));
+          } else {
+            return fftc::mk((T)acc[at].x, (T)acc[at].y);
+          }
         },
         v, P, 0, 1, tw, tid);
     __syncthreads();
@@ -66,48 +69,31 @@ __device__ __forceinline__ void mix_first_fix(cpx<T> *buf, const fftm::Plan &P, 
   __syncthreads();
 }
 
-// Blocks of the cells ix .. ix + kw - 1 (cyclic, kw <= 16): at most b0, the
-// row's last block (when they wrap) and the last cell's.
-struct FixBlocks {
-  int b0, bm, b1;
-};
-__device__ __forceinline__ FixBlocks fix_blocks(int ix, int kw, int nf1) {
-  FixBlocks f;
-  const int last = ix + kw - 1;
-  f.b0 = ix >> kFixBlkLog2;
-  f.bm = last >= nf1 ? (nf1 - 1) >> kFixBlkLog2 : f.b0;
-  f.b1 = (last >= nf1 ? last - nf1 : last) >> kFixBlkLog2;
-  return f;
-}
-
-// plane tap of a record in plane p, or -1
-__device__ __forceinline__ int plane_tap(int iw, int p, const Geom &g) {
-  int k = p - iw;
-  if (k < 0) k += g.P;
-  return k < g.kww ? k : -1;
-}
-
 // ms2dirty: spread into the workgroup's rows (LDS), row FFT, image columns to H.
-// FP32 accumulates in block floating point (integer LDS atomics; kAccFix of
-// kern_lds.h), FP64 with FP64 LDS atomics.
-template <typename T, int KWM>
+// Accumulation as RowAcc says; outputs added to H where gridDim.z workgroups share
+// the rows' records.
+template <typename T, int KWM, bool ACC64>
 __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
     const Rec<T> *__restrict__ recs, const T *__restrict__ taps, const int *__restrict__ off, cpx<T> *__restrict__ H,
     const cpx<T> *__restrict__ tw, Geom g, fftm::Plan P, int p0, int nb, int pchunk) {
-  constexpr bool kFix = sizeof(T) == 4;
+  using Cell = typename RowAcc<T, ACC64>::cell;
+  constexpr bool kFix = RowAcc<T, ACC64>::fix;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ WalkTable wt[2];
   __shared__ int fixnan;
-  const int nf1 = g.nf1, nf2 = g.nf2, kw = g.kw, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
-  const int nbuf = P.count * P.stride, nblk = mix_blocks(nf1), h1 = N1 / 2;
+  const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
+  const int nbuf = P.count * P.stride, nblk = fix_row_blocks(nf1), h1 = N1 / 2;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
-  float *fixt = reinterpret_cast<float *>(buf + nbuf + fftc::twiddle_entries(nf1));
+  Cell *acc = reinterpret_cast<Cell *>(smem_raw);
+  cpx<T> *ltw = reinterpret_cast<cpx<T> *>(acc + nbuf);
+  float *fixt = reinterpret_cast<float *>(ltw + fftc::twiddle_entries(nf1));
   short *fixe = reinterpret_cast<short *>(fixt + rpw * nblk);
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
-  const auto tv = lds_twiddles<T>(buf + nbuf, tw, nf1);
+  const bool add = gridDim.z > 1;
+  const auto tv = lds_twiddles<T>(ltw, tw, nf1);
   if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, nrows);
-  for (int i = tid; i < nbuf; i += nt) buf[i] = fftc::mk((T)0, (T)0);
+  for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{0, 0};
   if (kFix) {
     for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
     if (tid == 0) fixnan = 0;
@@ -120,92 +106,23 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
     WalkAhead wa;
     if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, nrows);
     if (kFix && total > 0) {
-      for (int t = tid; t < total; t += nt) {
-        const int ia = walk_record(wt[cur], t);
-        const Rec<T> rc = recs[ia];
-        const int k = plane_tap(rc.iw, p, g);
-        if (k < 0) continue;
-        const T *tq = taps + (size_t)ia * (3 * KWM);
-        const float a = (fabsf((float)rc.re) + fabsf((float)rc.im)) * fabsf((float)tq[2 * KWM + k]);
-        const FixBlocks f = fix_blocks(rc.ix, kw, nf1);
-        for (int r = 0; r < nrows; ++r) {
-          int jj = row0 + r - rc.iy;
-          if (jj < 0) jj += nf2;
-          if (jj >= kw) continue;
-          const float b = a * fabsf((float)tq[KWM + jj]);
-          float *bs = fixt + r * nblk;
-          atomicAdd(bs + f.b0, b);
-          if (f.bm != f.b0) atomicAdd(bs + f.bm, b);
-          if (f.b1 != f.b0 && f.b1 != f.bm) atomicAdd(bs + f.b1, b);
-        }
-      }
+      bound_records<T, KWM>(wt[cur], total, recs, taps, g, p, row0, nrows, fixt, nblk);
       __syncthreads();
-      for (int i = tid; i < nrows * nblk; i += nt) {
-        // published to the first stage by the barrier after the spread
-        const int e = fix_block_exp(fixt[i]);
-        fixe[i] = (short)(e == kFixNaN ? 0 : e);
-        if (e == kFixNaN) fixnan = 1;
-      }
+      block_exponents(fixt, fixe, nrows * nblk, &fixnan);
     }
-    for (int t = tid; t < total; t += nt) {
-      const int ia = walk_record(wt[cur], t);
-      const Rec<T> rc = recs[ia];
-      const int k = plane_tap(rc.iw, p, g);
-      if (k < 0) continue;
-      const T *tq = taps + (size_t)ia * (3 * KWM);
-      T kx[KWM];
-#pragma unroll
-      for (int i = 0; i < KWM; ++i) kx[i] = tq[i];
-      const T kz = tq[2 * KWM + k];
-      const FixBlocks f = fix_blocks(rc.ix, kw, nf1);
-      for (int r = 0; r < nrows; ++r) {
-        int jj = row0 + r - rc.iy;
-        if (jj < 0) jj += nf2;
-        if (jj >= kw) continue;
-        const T a = kz * tq[KWM + jj], vre = rc.re * a, vim = rc.im * a;
-        cpx<T> *row = buf + r * P.stride;
-        int e0 = 0, em = 0, e1 = 0;
-        if (kFix) {
-          const float *bs = fixt + r * nblk;
-          e0 = fix_block_exp(bs[f.b0]);
-          em = fix_block_exp(bs[f.bm]);
-          e1 = fix_block_exp(bs[f.b1]);
-          e0 = e0 == kFixNaN ? 0 : e0;
-          em = em == kFixNaN ? 0 : em;
-          e1 = e1 == kFixNaN ? 0 : e1;
-        }
-#pragma unroll
-        for (int i = 0; i < KWM; ++i) {
-          if (i < kw) {
-            int cx = rc.ix + i;
-            if (cx >= nf1) cx -= nf1;
-            const T re = vre * kx[i], im = vim * kx[i];
-            if (kFix) {
-              const int blk = cx >> kFixBlkLog2, e = blk == f.b0 ? e0 : blk == f.bm ? em : e1;
-              int *d = reinterpret_cast<int *>(row + fftc::pad(cx));
-              atomicAdd(d, __float2int_rn(ldexpf((float)re, e)));
-              atomicAdd(d + 1, __float2int_rn(ldexpf((float)im, e)));
-            } else {
-              T *d = reinterpret_cast<T *>(row + fftc::pad(cx));
-              atomicAdd(d, re);
-              atomicAdd(d + 1, im);
-            }
-          }
-        }
-      }
-    }
+    spread_records<T, KWM, ACC64>(wt[cur], total, recs, taps, g, p, row0, nrows, acc, P.stride, fixt, nblk);
     if (tid < 64 && more) walk_finish(wt[cur ^ 1], wa);
     __syncthreads();  // spread done; the next plane's walk table is complete
     cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
     if (total == 0) {
       // no visibility reaches these rows of this plane (and the LDS is still clear)
-      for (int r = 0; r < nrows; ++r)
+      for (int r = 0; r < nrows && !add; ++r)
         for (int i = tid; i < N1; i += nt) hb[h_slot(g, i) + (r << kTileLog2)] = fftc::mk((T)0, (T)0);
       continue;
     }
     const bool pnan = kFix && fixnan;  // cleared below, after the transform's barriers
-    if (kFix) {
-      mix_first_fix<T, +1>(buf, P, tv, fixe, nblk);
+    if (kFix || ACC64) {
+      mix_first_cells<T, +1, ACC64>(buf, acc, P, tv, fixe, nblk);
       mix_stages<T, +1>(buf, P, tv, 1, P.R[0]);
     } else {
       mix_stages<T, +1>(buf, P, tv, 0, 1);
@@ -215,15 +132,39 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
         const int k = i >= h1 ? i - h1 : nf1 + i - h1;
         cpx<T> x = buf[r * P.stride + fftc::pad(k)];
         if (pnan) x = fftc::mk((T)NAN, (T)NAN);
-        hb[h_slot(g, i) + (r << kTileLog2)] = x;
+        put_row(hb + h_slot(g, i) + (r << kTileLog2), x, add);
       }
     __syncthreads();  // every output read: clear for the next plane
-    for (int i = tid; i < nbuf; i += nt) buf[i] = fftc::mk((T)0, (T)0);
+    for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{0, 0};
     if (kFix) {
       for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
       if (tid == 0) fixnan = 0;
     }
     __syncthreads();
+  }
+}
+
+// rows [row0, row0 + nrows) of a dirty2ms plane into LDS, expanded to nf1 cells
+template <typename T>
+__device__ __forceinline__ void mix_load_rows(cpx<T> *buf, const cpx<T> *hb, const Geom &g, const fftm::Plan &P, int row0,
+                                              int nrows, int N1) {
+  const int nt = blockDim.x, nf1 = g.nf1;
+  for (int r = 0; r < nrows; ++r) {
+    const cpx<T> *hr = hb + ht_row(row0 + r);
+    constexpr int B = 8;  // loads in flight
+    for (int i0 = threadIdx.x; i0 < nf1; i0 += B * nt) {
+      cpx<T> v[B];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int i = i0 + b * nt, col = i < nf1 ? image_index(i, N1, nf1) : -1;
+        v[b] = col >= 0 ? hr[ht_slot(g, col)] : fftc::mk((T)0, (T)0);
+      }
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int i = i0 + b * nt;
+        if (i < nf1) buf[r * P.stride + fftc::pad(i)] = v[b];
+      }
+    }
   }
 }
 
@@ -236,7 +177,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_interp_mix_kernel(
     int nb, int pchunk) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ WalkTable wt[2];
-  const int nf1 = g.nf1, nf2 = g.nf2, kw = g.kw, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
+  const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
@@ -252,67 +193,41 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_interp_mix_kernel(
     WalkAhead wa;
     if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, nrows);
     if (total > 0) {
-      const cpx<T> *hb = H + h_plane(g, pl);
-      for (int r = 0; r < nrows; ++r) {
-        const cpx<T> *hr = hb + ht_row(row0 + r);
-        constexpr int B = 8;  // loads in flight
-        for (int i0 = tid; i0 < nf1; i0 += B * nt) {
-          cpx<T> v[B];
-#pragma unroll
-          for (int b = 0; b < B; ++b) {
-            const int i = i0 + b * nt, col = i < nf1 ? image_index(i, N1, nf1) : -1;
-            v[b] = col >= 0 ? hr[ht_slot(g, col)] : fftc::mk((T)0, (T)0);
-          }
-#pragma unroll
-          for (int b = 0; b < B; ++b) {
-            const int i = i0 + b * nt;
-            if (i < nf1) buf[r * P.stride + fftc::pad(i)] = v[b];
-          }
-        }
-      }
+      mix_load_rows<T>(buf, H + h_plane(g, pl), g, P, row0, nrows, N1);
       __syncthreads();
       mix_stages<T, -1>(buf, P, tv, 0, 1);
-      for (int t = tid; t < total; t += nt) {
-        const int ia = walk_record(wt[cur], t);
-        const Rec<T> rc = recs[ia];
-        const int k = plane_tap(rc.iw, p, g);
-        if (k < 0) continue;
-        const T *tq = taps + (size_t)ia * (3 * KWM);
-        T kx[KWM];
-#pragma unroll
-        for (int i = 0; i < KWM; ++i) kx[i] = tq[i];
-        const T kz = tq[2 * KWM + k];
-        T sr = 0, si = 0;
-        bool hit = false;
-        for (int r = 0; r < nrows; ++r) {
-          int jj = row0 + r - rc.iy;
-          if (jj < 0) jj += nf2;
-          if (jj >= kw) continue;
-          hit = true;
-          const cpx<T> *row = buf + r * P.stride;
-          T rr = 0, ri = 0;
-#pragma unroll
-          for (int i = 0; i < KWM; ++i) {
-            if (i < kw) {
-              int cx = rc.ix + i;
-              if (cx >= nf1) cx -= nf1;
-              const cpx<T> f = row[fftc::pad(cx)];
-              rr += f.x * kx[i];
-              ri += f.y * kx[i];
-            }
-          }
-          const T ky = tq[KWM + jj];
-          sr += rr * ky;
-          si += ri * ky;
-        }
-        if (hit) {
-          atomicAdd(&vacc[ia].x, (double)(sr * kz));
-          atomicAdd(&vacc[ia].y, (double)(si * kz));
-        }
-      }
+      interp_records<T, KWM>(wt[cur], total, recs, taps, g, p, row0, nrows, buf, P.stride, vacc);
     }
     if (tid < 64 && more) walk_finish(wt[cur ^ 1], wa);
     __syncthreads();  // the rows are free; the next plane's walk table is complete
+  }
+}
+
+// dirty2ms where the records are dense on the grid (Geom::gather): the rows are
+// written out as full planes, and interp_gather_kernel reads each record's cells
+// from there, once per record, where the fused row pass would visit the record
+// in every row and plane of its support and add two FP64 atomics each time.
+template <typename T>
+__global__ void __launch_bounds__(MixThreads<T>::value) row_planes_mix_kernel(const cpx<T> *__restrict__ H,
+                                                                             cpx<T> *__restrict__ grid,
+                                                                             const cpx<T> *__restrict__ tw, Geom g,
+                                                                             fftm::Plan P, int nb, int pchunk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
+  cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
+  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
+  const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
+  const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
+  for (int i = tid; i < P.count * P.stride; i += nt) buf[i] = fftc::mk((T)0, (T)0);
+  for (int pl = k0; pl < k1; ++pl) {
+    __syncthreads();  // the previous plane's rows are written
+    mix_load_rows<T>(buf, H + h_plane(g, pl), g, P, row0, nrows, N1);
+    __syncthreads();
+    mix_stages<T, -1>(buf, P, tv, 0, 1);
+    for (int r = 0; r < nrows; ++r) {
+      cpx<T> *out = grid + ((size_t)pl * nf2 + row0 + r) * nf1;
+      for (int i = tid; i < nf1; i += nt) out[i] = buf[r * P.stride + fftc::pad(i)];
+    }
   }
 }
 
@@ -444,9 +359,10 @@ __global__ void __launch_bounds__(MT) col_inv_mix_kernel(const cpx<T> *__restric
 // --------------------------------------------------------------------------
 // launchers
 // --------------------------------------------------------------------------
-template <typename T> inline int mix_row_lds(const Geom &g) {
-  int b = (int)sizeof(cpx<T>) * (g.rpw * fftm::seq_stride(g.nf1) + fftc::twiddle_entries(g.nf1));
-  if (sizeof(T) == 4) b += g.rpw * mix_blocks(g.nf1) * 6 + 2;
+template <typename T> inline int mix_row_lds(const Geom &g, bool spread) {
+  const int cells = g.rpw * fftm::seq_stride(g.nf1);
+  int b = cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>)) + fftc::twiddle_entries(g.nf1) * (int)sizeof(cpx<T>);
+  if (sizeof(T) == 4 && spread && !g.acc64) b += g.rpw * fix_row_blocks(g.nf1) * 6 + 2;
   return b;
 }
 template <typename T> inline int mix_col_lds(const Geom &g, int cpw) {
@@ -472,20 +388,29 @@ template <typename T>
 void mix_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const ChanPlan &cp, int p0, int nb, cpx<T> *H,
                      const cpx<T> *tw1, hipStream_t st) {
   const Geom &g = cp.g;
-  const dim3 grd((g.nf2 + g.rpw - 1) / g.rpw, (nb + g.pch_row - 1) / g.pch_row);
-  const int lb = mix_row_lds<T>(g), nt = cp.rowf.nt;
-  if (g.kw <= 8)
-    spread_row_mix_kernel<T, 8><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, cp.rowf, p0, nb, g.pch_row);
-  else
-    spread_row_mix_kernel<T, 16><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, cp.rowf, p0, nb, g.pch_row);
+  const dim3 grd((g.nf2 + g.rpw - 1) / g.rpw, (nb + g.pch_row - 1) / g.pch_row, g.zrow);
+  const int lb = mix_row_lds<T>(g, true), nt = cp.rowf.nt;
+  if (g.zrow > 1) zero_planes<T>(H, g, nb, st);
+  with_acc64<T>(g.acc64, [&](auto A) {
+    if (g.kw <= 8)
+      spread_row_mix_kernel<T, 8, A.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, cp.rowf, p0, nb, g.pch_row);
+    else
+      spread_row_mix_kernel<T, 16, A.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, cp.rowf, p0, nb, g.pch_row);
+  });
 }
 
 template <typename T>
-void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, double2 *vacc, const cpx<T> *tw1,
-                    const ChanPlan &cp, int p0, int nb, hipStream_t st) {
+void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, void *grid, double2 *vacc,
+                    const cpx<T> *tw1, const ChanPlan &cp, int p0, int nb, hipStream_t st) {
   const Geom &g = cp.g;
   const dim3 grd((g.nf2 + g.rpw - 1) / g.rpw, (nb + g.pch_row - 1) / g.pch_row);
-  const int lb = mix_row_lds<T>(g), nt = cp.rowf.nt;
+  const int lb = mix_row_lds<T>(g, false), nt = cp.rowf.nt;
+  if (g.gather) {
+    cpx<T> *planes = (cpx<T> *)grid;
+    row_planes_mix_kernel<T><<<grd, nt, lb, st>>>(H, planes, tw1, g, cp.rowf, nb, g.pch_row);
+    launch_gather<T>(recs, taps, off, planes, vacc, g, cp.nvalid, p0, nb, st);
+    return;
+  }
   if (g.kw <= 8)
     row_interp_mix_kernel<T, 8><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, cp.rowf, p0, nb, g.pch_row);
   else
@@ -520,16 +445,20 @@ template <typename T> int allow_mix(const ChanPlan &cp) {
   // what the kernels assume of their launches
   if (cp.rowf.n != g.nf1 || cp.rowf.count != g.rpw || cp.colf.n != g.nf2 || cp.colf.count != g.cpw || rows < 64 ||
       rows > top || cols < 64 || cols > top || mix_cells(g.cpw, g.N2, cols) > 16 || g.pch_row < 1 || g.pch_fwd < 1 ||
-      g.pch_inv < 1 || (g.cpw & (g.cpw - 1)) != 0) {
+      g.pch_inv < 1 || g.zrow < 1 || (g.cpw & (g.cpw - 1)) != 0) {
     set_error("mixed-radix plan of grid %d x %d does not fit its kernels", g.nf2, g.nf1);
     return kErrArg;
   }
-  const int lr = mix_row_lds<T>(g), lc = mix_col_lds<T>(g, g.cpw);
-  CURIG_TRY((allow_lds(spread_row_mix_kernel<T, 8>, lr)));
-  CURIG_TRY((allow_lds(spread_row_mix_kernel<T, 16>, lr)));
+  const int ls = mix_row_lds<T>(g, true), lr = mix_row_lds<T>(g, false), lc = mix_col_lds<T>(g, g.cpw);
+  int ier = kOk;
+  with_acc64<T>(g.acc64, [&](auto A) {
+    ier = allow_lds(spread_row_mix_kernel<T, 8, A.value>, ls);
+    if (ier == kOk) ier = allow_lds(spread_row_mix_kernel<T, 16, A.value>, ls);
+  });
+  CURIG_TRY(ier);
   CURIG_TRY((allow_lds(row_interp_mix_kernel<T, 8>, lr)));
   CURIG_TRY((allow_lds(row_interp_mix_kernel<T, 16>, lr)));
-  int ier = kOk;
+  CURIG_TRY((allow_lds(row_planes_mix_kernel<T>, lr)));
   with_cells<T>(mix_cells(g.cpw, g.N2, cols), cols, [&](auto NO, auto MT) {
     ier = allow_lds(col_fwd_mix_kernel<T, NO.value, MT.value>, lc);
     if (ier == kOk) ier = allow_lds(col_inv_mix_kernel<T, NO.value, MT.value>, lc);
@@ -540,7 +469,7 @@ template <typename T> int allow_mix(const ChanPlan &cp) {
 #define CURIG_MIX_INST(T)                                                                                          \
   template void mix_spread_rows<T>(const Rec<T> *, const T *, const int *, const ChanPlan &, int, int, cpx<T> *,   \
                                    const cpx<T> *, hipStream_t);                                                   \
-  template void mix_row_interp<T>(const Rec<T> *, const T *, const int *, const cpx<T> *, double2 *,               \
+  template void mix_row_interp<T>(const Rec<T> *, const T *, const int *, const cpx<T> *, void *, double2 *,       \
                                   const cpx<T> *, const ChanPlan &, int, int, hipStream_t);                        \
   template void mix_cols_forward<T>(const ChanPlan &, int, int, const cpx<T> *, double2 *, const cpx<T> *, int,    \
                                     hipStream_t);                                                                  \

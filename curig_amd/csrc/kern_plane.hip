@@ -252,28 +252,6 @@ __global__ void __launch_bounds__(256) wfill_kernel(const double2 *__restrict__ 
   }
 }
 
-// Records whose first plane lies in the cyclic interval [lo, lo + len) (len <= P):
-// up to two ranges of bin layers, read from the bin offsets on the device.
-__device__ __forceinline__ void layer_ranges(const int *__restrict__ off, const Geom &g, int lo, int len, int &a0,
-                                             int &a1, int &b0, int &b1) {
-  if (len > g.P) len = g.P;
-  const int first = lo / g.Pbin;
-  const int last_plane = lo + len - 1;
-  a0 = off[(long)first * g.ntiles];
-  b0 = b1 = 0;
-  if (last_plane < g.P) {
-    a1 = off[(long)(last_plane / g.Pbin + 1) * g.ntiles];
-  } else {
-    a1 = off[(long)g.nlayer * g.ntiles];
-    int lastl = (last_plane - g.P) / g.Pbin;
-    if (lastl >= first) lastl = first - 1;  // the whole circle is covered
-    if (lastl >= 0) {
-      b0 = off[0];
-      b1 = off[(long)(lastl + 1) * g.ntiles];
-    }
-  }
-}
-
 // interpolation (dirty2ms): per record, sum over the kernel support inside the
 // batch's planes; FP32 (or FP64) multiply-accumulate per plane, FP64 across planes.
 // src/fourier/interp.cu:143-228.

@@ -162,6 +162,16 @@ template <typename T> int allow_spread_rows(const Geom &g);
 template <typename T> int allow_row_interp(const Geom &g);
 template <typename T> int allow_cols(const Geom &g);
 
+// ---- kern_rowreg_*.hip: whole power-of-two rows of the LDS path (Geom::rowreg) -
+template <typename T>
+void rowreg_spread(const Rec<T> *recs, const T *taps, const int *off, const Geom &g, int p0, int nb, cpx<T> *H,
+                   const cpx<T> *tw1, hipStream_t st);
+// grid: room for the batch's planes where g.gather
+template <typename T>
+void rowreg_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, void *grid, double2 *vacc,
+                   const cpx<T> *tw1, const Geom &g, long nvalid, int p0, int nb, hipStream_t st);
+template <typename T> int allow_rowreg(const Geom &g, bool spread);
+
 // ---- kern_mix_*.hip: the LDS path on mixed-radix grids (Geom::mix) -----------
 template <typename T>
 void mix_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const ChanPlan &cp, int p0, int nb, cpx<T> *H,
@@ -173,8 +183,8 @@ template <typename T>
 void mix_cols_backward(const ChanPlan &cp, int p0, int nb, const cpx<T> *gT, cpx<T> *H, const cpx<T> *tw2,
                        hipStream_t st);
 template <typename T>
-void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, double2 *vacc, const cpx<T> *tw1,
-                    const ChanPlan &cp, int p0, int nb, hipStream_t st);
+void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<T> *H, void *grid, double2 *vacc,
+                    const cpx<T> *tw1, const ChanPlan &cp, int p0, int nb, hipStream_t st);
 // checks a plan against the kernels' launch limits and raises their dynamic LDS
 template <typename T> int allow_mix(const ChanPlan &cp);
 
