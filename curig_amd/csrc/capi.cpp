@@ -368,14 +368,6 @@ extern "C" int curig_nifty_dirty2ms(int nrow, int nchan, const double *uvw, cons
 // nufft_1d_test.cu ground truths).  Dimension 1 runs as N2 = 1; dimension 3
 // as N3 passes of the 2-D transform over c_j e^{i iflag k3' w_j}.
 // ---------------------------------------------------------------------------
-__global__ void pack_nufft_kernel(const double *u, const double *v, double *uvw, int n, double s) {
-  for (long j = blockIdx.x * (long)blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x) {
-    uvw[3 * j] = v ? s * v[j] : 0.0;  // slow image axis (N2) pairs with v
-    uvw[3 * j + 1] = s * u[j];       // fast image axis (N1) pairs with u
-    uvw[3 * j + 2] = 0.0;
-  }
-}
-
 template <typename T> struct Cx;
 template <> struct Cx<double> { using type = double2; };
 template <> struct Cx<float> { using type = float2; };
@@ -418,17 +410,10 @@ static int nufft_run(int type, int dim, int N1, int N2, int N3, int M, const dou
   using C2 = typename Cx<T>::type;
   const bool dbl = sizeof(T) == 8;
   const int n2 = dim >= 2 ? N2 : 1, n3 = dim == 3 ? N3 : 1;
-  double *d_uvw = nullptr;
   C2 *tmp = nullptr;
   int ier = kOk;
   const int nb = std::max(1, std::min((M + 255) / 256, 65536));
-  if (M > 0) {
-    CURIG_HIP(hipMalloc(&d_uvw, sizeof(double) * 3 * (size_t)M));
-    // type 1 runs ms2dirty (e^{+i x.k}); type 2 runs dirty2ms (e^{-i x.k})
-    pack_nufft_kernel<<<nb, 256, 0, st>>>(d_u, dim >= 2 ? d_v : nullptr, d_uvw, M, type == 1 ? iflag : -iflag);
-    ier = hipGetLastError() == hipSuccess ? kOk : kErrHip;
-    if (ier == kOk && dim == 3 && hipMalloc(&tmp, sizeof(C2) * (size_t)M) != hipSuccess) ier = kErrAlloc;
-  }
+  if (dim == 3 && M > 0) CURIG_HIP(hipMalloc(&tmp, sizeof(C2) * (size_t)M));
   Problem pb;
   pb.nrow = M;
   pb.nx = n2;
@@ -438,7 +423,11 @@ static int nufft_run(int type, int dim, int N1, int N2, int N3, int M, const dou
   pb.sigma = sigma;
   pb.sign = -1;
   pb.dbl = dbl;
-  pb.uvw = d_uvw;
+  pb.cols.set = true;
+  pb.cols.c[0] = dim >= 2 ? d_v : nullptr;  // slow image axis (N2) pairs with v
+  pb.cols.c[1] = d_u;                       // fast image axis (N1) pairs with u
+  // type 1 runs ms2dirty (e^{+i x.k}); type 2 runs dirty2ms (e^{-i x.k})
+  pb.cols.scale = type == 1 ? iflag : -iflag;
   pb.spec.radians = true;
   pb.spec.wstack = false;
   const size_t slab = (size_t)N1 * n2;
@@ -459,7 +448,6 @@ static int nufft_run(int type, int dim, int N1, int N2, int N3, int M, const dou
     }
   }
   if (ier == kOk && hipStreamSynchronize(st) != hipSuccess) ier = kErrHip;
-  if (d_uvw) (void)hipFree(d_uvw);
   if (tmp) (void)hipFree(tmp);
   return ier;
 }
@@ -505,14 +493,6 @@ extern "C" int curig_nufft_dev(int type, int dim, int N1, int N2, int N3, int M,
 // reference's drivers test/nufft_1d_3_1_test.cu, nufft_1d_3_2_test.cu):
 //   direction 1: f_i = sum_j c_j e^{i iflag s_i x_j}
 //   direction 0: c_j = sum_i f_i e^{i iflag s_i x_j}
-__global__ void pack_type3_kernel(const double *x, double *uvw, int n, double s) {
-  for (long j = blockIdx.x * (long)blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x) {
-    uvw[3 * j] = 0.0;
-    uvw[3 * j + 1] = 0.0;
-    uvw[3 * j + 2] = s * x[j];
-  }
-}
-
 static int nufft3_checked(int M, int N, const double *d_x, const double *d_s, void *d_c, void *d_f, int iflag,
                           int direction, double epsilon, double sigma, int precision, void *stream, const Tuning &tn) {
   CURIG_TRY(check_precision(precision));
@@ -548,13 +528,6 @@ static int nufft3_checked(int M, int N, const double *d_x, const double *d_s, vo
     smin = std::min(smin, v);
     smax = std::max(smax, v);
   }
-  double *d_uvw = nullptr;
-  if (M > 0) {
-    CURIG_HIP(hipMalloc(&d_uvw, sizeof(double) * 3 * (size_t)M));
-    // direction 1 runs ms2dirty (e^{+i w z}), direction 0 dirty2ms (e^{-i w z})
-    const int nb = std::max(1, std::min((M + 255) / 256, 65536));
-    pack_type3_kernel<<<nb, 256, 0, st>>>(d_x, d_uvw, M, direction == 1 ? iflag : -iflag);
-  }
   Problem pb;
   pb.nrow = M;
   pb.nx = 1;
@@ -564,7 +537,10 @@ static int nufft3_checked(int M, int N, const double *d_x, const double *d_s, vo
   pb.sigma = sigma;
   pb.sign = 1;
   pb.dbl = precision == 0;
-  pb.uvw = d_uvw;
+  pb.cols.set = true;
+  pb.cols.c[2] = d_x;
+  // direction 1 runs ms2dirty (e^{+i w z}), direction 0 dirty2ms (e^{-i w z})
+  pb.cols.scale = direction == 1 ? iflag : -iflag;
   pb.vis = d_c;
   pb.dirty = d_f;
   pb.spec.radians = true;
@@ -573,7 +549,6 @@ static int nufft3_checked(int M, int N, const double *d_x, const double *d_s, vo
   pb.spec.zmax = smax;
   int ier = direction == 1 ? ms2dirty_device(pb, st, &tn, stats_ptr()) : dirty2ms_device(pb, st, &tn, stats_ptr());
   if (ier == kOk && hipStreamSynchronize(st) != hipSuccess) ier = kErrHip;
-  if (d_uvw) (void)hipFree(d_uvw);
   return ier;
 }
 

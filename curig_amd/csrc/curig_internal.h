@@ -59,6 +59,16 @@ struct KernelOpts {
   double beta = 0, c = 0, halfwidth = 0, upsampfac = 2.0;
 };
 
+constexpr int kMaxCheb = 64;
+
+// kernel_quadrature's rule, passed to kernels by value, and the number of terms
+// of the Chebyshev series of phihat3 on |z| <= zmax
+struct QuadRule {
+  int n = 0, nc = 0;
+  double zmax = 0;
+  double x[kMaxQuadNodes], g[kMaxQuadNodes];
+};
+
 // Host plan math (plan_math.cpp)
 int setup_conv_opts(KernelOpts &o, double eps, double upsampfac);
 int next235beven(int n, int b);
@@ -67,6 +77,9 @@ void set_nhg_type3(double S, double X, const KernelOpts &o, int &nf, double &h, 
 void gauss_legendre(int n, double *x, double *w);
 // 2p scaled nodes x_n and weights g_n = alpha w_n phi_norm(x_n); returns 2p
 int kernel_quadrature(const KernelOpts &o, double *x, double *g);
+int quadrature_nodes(const KernelOpts &o);  // 2p
+// terms of phihat3(z)'s series in T_k(2 (z / zmax)^2 - 1), zmax = pi / sigma; 0: not used
+int cheb_terms(const KernelOpts &o);
 // phihat_norm(k) (-1)^k for k = 0..nf/2 (normalised kernel, peak 1)
 void fseries_grid(const KernelOpts &o, int nf, double *out);
 // piecewise-polynomial kernel: kw intervals x (deg + 1) coefficients in powers
@@ -94,6 +107,9 @@ struct Geom {
   int Pb, nbatch;     // planes per batch, number of batches
   int Pbin, nlayer;   // planes per bin layer (rows are binned by first plane / Pbin), layers
   int nquad;          // number of quadrature nodes for phihat3
+  int ncheb;          // terms of its Chebyshev series, which holds for |z| <= zcheb; 0: none; -1: none,
+                      // and the correction tables computed on the host
+  double zcheb;
   // pruned LDS FFT path (power-of-two grids); fft_lds == 0 selects rocFFT
   int fft_lds;
   int mix;            // LDS path on axes 2^a 3^b 5^c (mixed-radix kernels), else powers of two

@@ -21,6 +21,14 @@ struct GridSpec {
   double zmin = 0, zmax = 0;
 };
 
+// Coordinates given as separate columns (null: zeros), packed into uvw = scale * column
+// in the workspace by the call.
+struct Columns {
+  const double *c[3] = {};
+  double scale = 1.0;
+  bool set = false;
+};
+
 struct Problem {
   int nrow = 0, nx = 0, ny = 0;
   double fov = 0, freq = 0, eps = 1e-6, sigma = 2.0;
@@ -35,6 +43,7 @@ struct Problem {
   long flag_stride = 1;
   void *dirty = nullptr;        // complex [nx][ny]
   bool accumulate = false;      // ms2dirty adds into dirty instead of overwriting it
+  Columns cols;                 // instead of uvw
   GridSpec spec;                // explicit pixel sizes / grid size / w handling (defaults: from fov, sigma)
 };
 

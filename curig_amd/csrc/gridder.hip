@@ -54,12 +54,15 @@ namespace {
 // previous call's waits for that call's launches on the device (ws_order).
 enum Slot {
   S_PART, S_CNT, S_HIST, S_OFF, S_BSUM, S_BINRANK, S_RECS, S_PERM, S_GRID, S_ACC, S_VACC, S_TAB, S_FFTW,
-  S_H, S_TW, S_HC, S_TAPS,
+  S_H, S_TW, S_HC, S_TAPS, S_UVW,
   S_NSLOT
 };
 struct Workspace {
   void *p[S_NSLOT] = {};
   size_t n[S_NSLOT] = {};
+  // pinned host memory the w-range kernels write (read after the call's wait)
+  void *pin = nullptr;
+  size_t pin_n = 0;
   int tw_key[3] = {-1, -1, -1};  // (nf1, nf2, sizeof(T)) of the twiddles held in S_TW
   // the last call's stream and an event recorded there after its last launch:
   // a call on another stream waits for it before touching the buffers
@@ -132,6 +135,25 @@ int ws_get(int dev, Slot s, size_t bytes, void **out) {
     if (s == S_TW) w.tw_key[0] = w.tw_key[1] = w.tw_key[2] = -1;
   }
   *out = w.p[s];
+  return kOk;
+}
+
+// Pinned host memory of at least bytes, addressed by the device too.  A call
+// reads it after its own wait with the lock held, so the next may overwrite it.
+int ws_pinned(int dev, size_t bytes, void **out) {
+  Workspace &w = g_ws[dev];
+  if (w.pin_n < bytes) {
+    if (w.pin) {
+      // a call that failed before its wait may have left a kernel that writes here
+      if (w.pending) CURIG_HIP(hipEventSynchronize(w.done));
+      CURIG_HIP(hipHostFree(w.pin));
+      w.pin = nullptr;
+      w.pin_n = 0;
+    }
+    CURIG_HIP(hipHostMalloc(&w.pin, bytes, hipHostMallocDefault));
+    w.pin_n = bytes;
+  }
+  *out = w.pin;
   return kOk;
 }
 
@@ -264,7 +286,7 @@ int check_args(const Problem &pb) {
     set_error("fov (%g) and freq (%g) must be positive and finite", pb.fov, pb.freq);
     return kErrNonFinite;
   }
-  if (!pb.dirty || (pb.nrow > 0 && (!pb.uvw || !pb.vis))) {
+  if (!pb.dirty || (pb.nrow > 0 && ((!pb.uvw && !pb.cols.set) || !pb.vis))) {
     set_error("NULL data pointer");
     return kErrArg;
   }
@@ -403,6 +425,11 @@ static void plan_mixed_chunks(Geom &g) {
   g.nacc = (g.Pb + g.pch_fwd - 1) / g.pch_fwd;
 }
 
+// the upsampling factor: a given grid size fixes it
+static double grid_sigma(int nx, int ny, double sigma, const GridSpec &sp) {
+  return sp.nu != 0 || sp.nv != 0 ? std::min((double)sp.nu / nx, (double)sp.nv / ny) : sigma;
+}
+
 int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, double eps, double sigma, int sign,
                   double wmin_m, double wmax_m, bool dbl, const Tuning *tune, Geom *gp, KernelOpts *kop,
                   const GridSpec *spec) {
@@ -414,7 +441,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
       set_error("grid %d x %d must be even and larger than the image %d x %d", sp.nu, sp.nv, nx, ny);
       return kErrSize;
     }
-    sigma = std::min((double)sp.nu / nx, (double)sp.nv / ny);
+    sigma = grid_sigma(nx, ny, sigma, sp);
   }
   KernelOpts ko;
   int ier = setup_conv_opts(ko, eps, sigma);
@@ -635,8 +662,13 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     set_error("too many bins (%d layers x %d tiles)", g.nlayer, g.ntiles);
     return kErrSize;
   }
-  double qx[kMaxQuadNodes], qg[kMaxQuadNodes];
-  g.nquad = kernel_quadrature(ko, qx, qg);
+  g.nquad = quadrature_nodes(ko);
+  // Full planes below an upsampling of 2 (FP32, or kernels wider than 16): the
+  // corrections span so many decades (1e11 at 1.25 and width 17) that one unit in
+  // the last place of a table moves the results by the rounding of the whole
+  // transform, 1e-8 in FP64; they keep the host's cosines.
+  g.ncheb = !g.fft_lds && sigma < 2.0 ? -1 : cheb_terms(ko);
+  g.zcheb = M_PI / sigma;
   *gp = g;
   if (kop) *kop = ko;
   return kOk;
@@ -658,27 +690,52 @@ int device_lds_bytes() {
 
 
 // Phase 1 (one wait): w range and unflagged count of every problem, then their geometries.
-int plan_all(bool to_image, const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int dev, std::vector<ChanPlan> &cps) {
+// The rows' ranges come back through pinned memory the kernels write; the
+// kernel's quadrature rule is computed meanwhile.
+int plan_all(bool to_image, const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int dev,
+             std::vector<ChanPlan> &cps, QuadRule &rule) {
   std::vector<int> nbm(n), base(n + 1, 0);
   for (int i = 0; i < n; ++i) {
     nbm[i] = pbs[i].nrow > 0 ? std::min(nblocks(pbs[i].nrow), 1024) : 0;
     base[i + 1] = base[i] + nbm[i];
   }
   void *vp;
-  CURIG_TRY(ws_get(dev, S_PART, sizeof(double) * 2 * std::max(base[n], 1), &vp));
-  double *part = (double *)vp;
-  CURIG_TRY(ws_get(dev, S_CNT, sizeof(int) * std::max(base[n], 1), &vp));
-  int *cnt = (int *)vp;
+  double *part;
+  int *cnt;
+  const size_t slots = std::max(base[n], 1);
+  if (g_arena) {
+    CURIG_TRY(ws_get(dev, S_PART, sizeof(double) * 2 * slots, &vp));
+    part = (double *)vp;
+    CURIG_TRY(ws_get(dev, S_CNT, sizeof(int) * slots, &vp));
+    cnt = (int *)vp;
+  } else {
+    CURIG_TRY(ws_pinned(dev, (2 * sizeof(double) + sizeof(int)) * slots, &vp));
+    part = (double *)vp;
+    cnt = (int *)(part + 2 * slots);
+  }
   for (int i = 0; i < n; ++i)
     if (nbm[i] > 0)
       launch_w_minmax(nbm[i], pbs[i].uvw, pbs[i].nrow, pbs[i].flag, pbs[i].flag_stride, part + 2 * base[i],
                       cnt + base[i], st);
   CURIG_HIP(hipGetLastError());
-  std::vector<double> hp(2 * std::max(base[n], 1));
-  std::vector<int> hc(std::max(base[n], 1));
-  if (base[n] > 0) {
-    CURIG_HIP(hipMemcpyAsync(hp.data(), part, sizeof(double) * 2 * base[n], hipMemcpyDeviceToHost, st));
-    CURIG_HIP(hipMemcpyAsync(hc.data(), cnt, sizeof(int) * base[n], hipMemcpyDeviceToHost, st));
+  KernelOpts ko;
+  const double sigma = grid_sigma(pbs[0].nx, pbs[0].ny, pbs[0].sigma, pbs[0].spec);
+  if (setup_conv_opts(ko, pbs[0].eps, sigma) == kOk) {
+    rule.n = kernel_quadrature(ko, rule.x, rule.g);
+    rule.nc = cheb_terms(ko);
+    rule.zmax = M_PI / ko.upsampfac;
+  }
+  std::vector<double> hpv;
+  std::vector<int> hcv;
+  const double *hp = part;
+  const int *hc = cnt;
+  if (g_arena && base[n] > 0) {
+    hpv.resize(2 * slots);
+    hcv.resize(slots);
+    CURIG_HIP(hipMemcpyAsync(hpv.data(), part, sizeof(double) * 2 * slots, hipMemcpyDeviceToHost, st));
+    CURIG_HIP(hipMemcpyAsync(hcv.data(), cnt, sizeof(int) * slots, hipMemcpyDeviceToHost, st));
+    hp = hpv.data();
+    hc = hcv.data();
   }
   CURIG_HIP(hipStreamSynchronize(st));
   Tuning tn = tune ? *tune : Tuning();
@@ -775,7 +832,8 @@ int batch_fft(int dev, const Geom &g, int nb, int sign, void *grid, hipStream_t 
 // correction tables and twiddles, create FFT plans and kernel attributes, so
 // that phase 3 queues kernels only.
 template <typename T>
-int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image, int dev, hipStream_t st, Bufs &b) {
+int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule &rule, bool to_image, int dev,
+            hipStream_t st, Bufs &b) {
   const Geom &g0 = cps[0].g;
   size_t nbins = 1, nscan = 1, nrow = 1, grid = 1, h = 1, npix = 1, nvalid = 1;
   for (size_t i = 0; i < cps.size(); ++i) {
@@ -879,16 +937,21 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, bool to_image,
     }
   }
   // correction tables (shared by all channels: same kernel and grid sizes)
-  const KernelOpts &ko = cps[0].ko;
-  size_t n1 = g0.nf1 / 2 + 1, n2 = g0.nf2 / 2 + 1;
-  std::vector<double> ht(n1 + n2 + 2 * kMaxQuadNodes);
-  fseries_grid(ko, g0.nf1, ht.data());
-  fseries_grid(ko, g0.nf2, ht.data() + n1);
-  kernel_quadrature(ko, ht.data() + n1 + n2, ht.data() + n1 + n2 + g0.nquad);
-  CURIG_TRY(ws_get(dev, S_TAB, sizeof(double) * ht.size(), &vp));
+  const size_t ntab = g0.nf1 / 2 + g0.nf2 / 2 + 2 + 2 * (size_t)g0.nquad + kMaxCheb;
+  CURIG_TRY(ws_get(dev, S_TAB, sizeof(double) * ntab, &vp));
   b.tabs = (double *)vp;
-  CURIG_HIP(hipMemcpyAsync(b.tabs, ht.data(), sizeof(double) * ht.size(), hipMemcpyHostToDevice, st));
-  CURIG_HIP(hipStreamSynchronize(st));
+  if (g0.ncheb < 0) {
+    std::vector<double> ht(ntab);
+    const size_t n1 = g0.nf1 / 2 + 1, n2 = g0.nf2 / 2 + 1;
+    fseries_grid(cps[0].ko, g0.nf1, ht.data());
+    fseries_grid(cps[0].ko, g0.nf2, ht.data() + n1);
+    kernel_quadrature(cps[0].ko, ht.data() + n1 + n2, ht.data() + n1 + n2 + g0.nquad);
+    CURIG_HIP(hipMemcpyAsync(b.tabs, ht.data(), sizeof(double) * ntab, hipMemcpyHostToDevice, st));
+    CURIG_HIP(hipStreamSynchronize(st));
+  } else {
+    launch_corr_tables(rule, g0.nf1, g0.nf2, b.tabs, st);
+    CURIG_HIP(hipGetLastError());
+  }
   b.dev = dev;
   return kOk;
 }
@@ -1118,7 +1181,7 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
+      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
   k << b.dev << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc
@@ -1139,8 +1202,21 @@ void drop_graph(GraphCache &gc) {
 template <typename T>
 int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const Tuning *tune, int graph_mode,
                Stats *sts, int dev) {
+  Problem packed;
+  if (n == 1 && pbs[0].cols.set) {
+    packed = pbs[0];
+    if (packed.nrow > 0) {
+      void *vp;
+      CURIG_TRY(ws_get(dev, S_UVW, sizeof(double) * 3 * (size_t)packed.nrow, &vp));
+      launch_pack_columns(packed.cols, (double *)vp, packed.nrow, st);
+      CURIG_HIP(hipGetLastError());
+      packed.uvw = (const double *)vp;
+    }
+    pbs = &packed;
+  }
   std::vector<ChanPlan> cps;
-  CURIG_TRY(plan_all(to_image, pbs, n, st, tune, dev, cps));
+  QuadRule rule;
+  CURIG_TRY(plan_all(to_image, pbs, n, st, tune, dev, cps, rule));
   Bufs b;
   if (g_arena) {
     // no-allocation call: the LDS FFT path only (rocFFT plans allocate), and
@@ -1160,12 +1236,12 @@ int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const T
         cp.g.nbatch = (cp.g.P + cp.g.Pb - 1) / cp.g.Pb;
       }
       g_arena->used = used0;
-      ier = reserve<T>(cps, pbs, to_image, dev, st, b);
+      ier = reserve<T>(cps, pbs, rule, to_image, dev, st, b);
       if (ier != kErrScratch) break;
     }
     CURIG_TRY(ier);
   } else {
-    CURIG_TRY((reserve<T>(cps, pbs, to_image, dev, st, b)));
+    CURIG_TRY((reserve<T>(cps, pbs, rule, to_image, dev, st, b)));
   }
   for (ChanPlan &cp : cps) {
     cp.g.hcoef_d = b.hc_d;
@@ -1351,6 +1427,7 @@ void release_workspace() {
     if (g_ws[d].done) (void)hipEventDestroy(g_ws[d].done);
     for (int s = 0; s < S_NSLOT; ++s)
       if (g_ws[d].p[s]) (void)hipFree(g_ws[d].p[s]);
+    if (g_ws[d].pin) (void)hipHostFree(g_ws[d].pin);
   }
   g_ws.clear();
   (void)hipSetDevice(cur);

@@ -51,6 +51,13 @@ __global__ void __launch_bounds__(256) w_minmax_kernel(const double *__restrict_
   }
 }
 
+// uvw = scale * columns (null: zeros)
+__global__ void __launch_bounds__(256) pack_columns_kernel(Columns c, double *__restrict__ uvw, int n) {
+  for (long j = blockIdx.x * (long)blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) uvw[3 * j + i] = c.c[i] ? c.scale * c.c[i][j] : 0.0;
+}
+
 __global__ void fill_int_kernel(int *__restrict__ p, long n, int v) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = v;
 }
@@ -223,6 +230,10 @@ __global__ void __launch_bounds__(256) bin_scatter_kernel(const double *__restri
 void launch_w_minmax(int nblk, const double *uvw, int nrow, const uint8_t *flag, long fs, double *part, int *cnt,
                      hipStream_t st) {
   w_minmax_kernel<<<nblk, 256, 0, st>>>(uvw, nrow, flag, fs, part, cnt);
+}
+
+void launch_pack_columns(const Columns &c, double *uvw, int n, hipStream_t st) {
+  pack_columns_kernel<<<nblocks(n), 256, 0, st>>>(c, uvw, n);
 }
 
 void launch_fill_zero_c128(double2 *p, long n, hipStream_t st) {

@@ -110,6 +110,7 @@ constexpr int kScanTile = kScanBlock * kScanItems;
 // ---- kern_prep.hip: w range, binning, fills --------------------------------
 void launch_w_minmax(int nblk, const double *uvw, int nrow, const uint8_t *flag, long fs, double *part, int *cnt,
                      hipStream_t st);
+void launch_pack_columns(const Columns &c, double *uvw, int n, hipStream_t st);
 // count, scan and scatter of one problem's rows into bin order (records and permutation)
 template <typename T>
 void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipStream_t st, bool with_value);
@@ -117,6 +118,7 @@ void launch_fill_zero_c128(double2 *p, long n, hipStream_t st);
 void launch_zero_rows(bool dbl, void *vis, long stride, int nrow, hipStream_t st);
 
 // ---- kern_plane.hip: full-plane path (rocFFT grids), corrections, direct sums
+void launch_corr_tables(const QuadRule &q, int nf1, int nf2, double *tabs, hipStream_t st);
 template <typename T>
 void spread_dispatch(const Rec<T> *recs, const int *off, v2_t<T> *grid, const Geom &g, int p0, int nb, hipStream_t st);
 template <typename T>

@@ -174,3 +174,17 @@ def test_dense_records(precision, nx, ny, nrow):
     say(f"[dense] {precision} {nx}x{ny} rows {nrow}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
     tol = 1e-11 if precision == "fp64" else 2e-6
     assert e1 < tol and e2 < tol
+
+
+# the corrections' w factor by its series, kernels of 5 to 14, against the direct sum
+@pytest.mark.parametrize("eps", [1e-4, 1e-11, 1e-13])
+def test_w_correction_against_direct_sum(eps):
+    nx, ny, fov, sigma = 60, 44, 20.0, 2.0
+    uvw, vis, wgt, img, f0 = _case(2000, nx, ny, fov, 60.0, 31)
+    d = gpu_ms2dirty(uvw, vis, wgt, nx, ny, fov, f0, eps, sigma)
+    v = gpu_dirty2ms(uvw, img, wgt, nx, ny, fov, f0, eps, sigma)
+    e1 = O.l2error(O.dft_ms2dirty(uvw, vis, wgt, nx, ny, fov, f0, -1), d)
+    e2 = O.l2error(O.dft_dirty2ms(uvw, img, wgt, nx, ny, fov, f0, -1), v)
+    say(f"[w correction] eps {eps}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
+    tol = max(3 * eps, 1e-12)
+    assert e1 < tol and e2 < tol
