@@ -112,6 +112,8 @@ struct Geom {
   double zcheb;
   // pruned LDS FFT path (power-of-two grids); fft_lds == 0 selects rocFFT
   int fft_lds;
+  const uint64_t *occ; // [P] planes' occupied row blocks: bit b for rows b << occ_lg .. (null: all taken as
+  int occ_lg;          // occupied); rows of the other blocks are neither written to nor read from H
   int mix;            // LDS path on axes 2^a 3^b 5^c (mixed-radix kernels), else powers of two
   int rowreg;         // whole power-of-two rows in the kernels of kern_rowreg.h
   int acc64;          // ms2dirty, FP32, dense records: rows summed in FP64 (rowreg and mix)

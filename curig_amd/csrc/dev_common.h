@@ -141,6 +141,43 @@ __device__ __forceinline__ Coords row_coords(const double *__restrict__ uvw, lon
   return c;
 }
 
+// occupied row blocks of plane p (Geom::occ), and whether row is in one
+__device__ __forceinline__ uint64_t occ_mask(const Geom &g, int p) { return g.occ ? g.occ[p] : ~uint64_t(0); }
+__device__ __forceinline__ bool occ_row(uint64_t mask, int row, const Geom &g) { return (mask >> (row >> g.occ_lg)) & 1; }
+
+__device__ __forceinline__ bool occ_full(uint64_t mask, const Geom &g) {
+  const int n = ((g.nf2 - 1) >> g.occ_lg) + 1;
+  return ~(mask | (n < 64 ? ~uint64_t(0) << n : 0)) == 0;
+}
+
+// The planes k of [k0, k1) of a batch that starts at plane p0 in which the block
+// of row ra or of row rb is occupied, in order (Geom::occ, 64 planes at a time;
+// every lane of a wavefront takes part, and every wavefront finds the same).
+struct PlaneWalk {
+  const Geom &g;
+  int p0, k1, ra, rb, base;
+  uint64_t m = 0;
+  __device__ __forceinline__ PlaneWalk(const Geom &g_, int p0_, int k0, int k1_, int ra_, int rb_)
+      : g(g_), p0(p0_), k1(k1_), ra(ra_), rb(rb_), base(k0 - 64) {}
+  // the next plane, or k1
+  __device__ __forceinline__ int next() {
+    while (m == 0) {
+      base += 64;
+      if (base >= k1) return k1;
+      const int k = base + (threadIdx.x & 63);
+      bool on = false;
+      if (k < k1) {
+        const uint64_t o = occ_mask(g, p0 + k);
+        on = occ_row(o, ra, g) || occ_row(o, rb, g);
+      }
+      m = __ballot(on);
+    }
+    const int k = base + __ffsll((unsigned long long)m) - 1;
+    m &= m - 1;
+    return __builtin_amdgcn_readfirstlane(k);
+  }
+};
+
 __device__ __forceinline__ int row_bin(const Coords &c, const Geom &g) {
   int tile = (c.iy / g.T2) * g.ntx + (c.ix / g.T1);
   return (c.iw / g.Pbin) * g.ntiles + tile;

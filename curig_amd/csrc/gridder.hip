@@ -54,7 +54,7 @@ namespace {
 // previous call's waits for that call's launches on the device (ws_order).
 enum Slot {
   S_PART, S_CNT, S_HIST, S_OFF, S_BSUM, S_BINRANK, S_RECS, S_PERM, S_GRID, S_ACC, S_VACC, S_TAB, S_FFTW,
-  S_H, S_TW, S_HC, S_TAPS, S_UVW,
+  S_H, S_TW, S_HC, S_TAPS, S_UVW, S_OCC,
   S_NSLOT
 };
 struct Workspace {
@@ -643,6 +643,9 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     g.T1 = std::min(tn.T1 > 0 ? tn.T1 : (dbl ? 32 : 64), g.nf1);
     g.T2 = std::min(tn.T2 > 0 ? tn.T2 : 32, g.nf2);
   }
+  // 64 blocks of rows at most, 64 rows each or a power of two more
+  g.occ_lg = 6;
+  while ((g.nf2 - 1) >> g.occ_lg >= 64) ++g.occ_lg;
   g.ntx = (g.nf1 + g.T1 - 1) / g.T1;
   g.nty = (g.nf2 + g.T2 - 1) / g.T2;
   if (g.fft_lds) {
@@ -835,7 +838,7 @@ template <typename T>
 int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule &rule, bool to_image, int dev,
             hipStream_t st, Bufs &b) {
   const Geom &g0 = cps[0].g;
-  size_t nbins = 1, nscan = 1, nrow = 1, grid = 1, h = 1, npix = 1, nvalid = 1;
+  size_t nbins = 1, nscan = 1, nrow = 1, grid = 1, h = 1, npix = 1, nvalid = 1, nplane = 1;
   for (size_t i = 0; i < cps.size(); ++i) {
     const Geom &g = cps[i].g;
     if (g.kw != g0.kw || g.nf1 != g0.nf1 || g.nf2 != g0.nf2 || g.N1 != g0.N1 || g.N2 != g0.N2) {
@@ -847,6 +850,7 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule
     nscan = std::max(nscan, (nb + kScanTile - 1) / kScanTile + 1);
     nrow = std::max(nrow, (size_t)std::max(pbs[i].nrow, 1));
     nvalid = std::max(nvalid, (size_t)std::max<long>(cps[i].nvalid, 1));
+    nplane = std::max(nplane, (size_t)g.P);
     const size_t plane = (size_t)g.nf1 * g.nf2, pix = (size_t)g.N1 * g.N2;
     if (!g.fft_lds || g.gather) grid = std::max(grid, plane * g.Pb);
     if (g.fft_lds) h = std::max(h, (size_t)g.nct * g.tstride * g.Pb);
@@ -952,6 +956,14 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule
     launch_corr_tables(rule, g0.nf1, g0.nf2, b.tabs, st);
     CURIG_HIP(hipGetLastError());
   }
+  b.occ = nullptr;
+  if (g0.fft_lds) {
+    // (last: a full scratch goes without)
+    if (ws_get(dev, S_OCC, sizeof(uint64_t) * nplane, &vp) == kOk)
+      b.occ = (uint64_t *)vp;
+    else if (!g_arena)
+      return kErrAlloc;
+  }
   b.dev = dev;
   return kOk;
 }
@@ -988,6 +1000,7 @@ int enqueue_ms2dirty(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   {
     Range r("curig ms2dirty binning");
     enqueue_binning<T>(pb, cp, b, st, true);
+    if (g.occ) launch_occ(b.off, g, b.occ, st);
   }
   CURIG_HIP(hipGetLastError());
   int e1 = tm.mark();
@@ -1061,6 +1074,7 @@ int enqueue_dirty2ms(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   int e0 = tm.mark();
   Range rp("curig dirty2ms binning and prologue");
   enqueue_binning<T>(pb, cp, b, st, false);
+  if (g.occ) launch_occ(b.off, g, b.occ, st);
   // every output row is written: flagged rows get 0
   launch_zero_rows(pb.dbl, pb.vis, pb.vis_stride, pb.nrow, st);
   const Rec<T> *recs = (const Rec<T> *)b.recs;
@@ -1181,10 +1195,10 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
+      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.occ_lg << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
-  k << b.dev << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc
+  k << b.dev << b.occ << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc
     << b.vacc << b.tw1 << b.tw2 << b.hc_d << b.hc_f;
   return k.h;
 }
@@ -1244,6 +1258,7 @@ int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const T
     CURIG_TRY((reserve<T>(cps, pbs, rule, to_image, dev, st, b)));
   }
   for (ChanPlan &cp : cps) {
+    cp.g.occ = b.occ;
     cp.g.hcoef_d = b.hc_d;
     cp.g.hcoef_f = b.hc_f;
   }

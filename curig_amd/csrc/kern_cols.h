@@ -75,11 +75,19 @@ __global__ void __launch_bounds__((ColCfg<T, N>::fwd_threads), (ColCfg<T, N>::fw
   // base, 32-bit offset); threads without a column read the first one's and
   // store nothing
   const unsigned off = sizeof(cpx<T>) * (unsigned)((col >= 0 ? h_slot(g, sl) : 0) + (j << kTileLog2));
+  // a wavefront's rows j + G e lie in one block of Geom::occ for each e; the rows
+  // of blocks without records are zero and not in H
+  const int jw = __builtin_amdgcn_readfirstlane(j);
   auto load = [&](cpx<T> *v, int k) {
     const cpx<T> *hk = H + h_plane(g, k);
+    const uint64_t occ = occ_mask(g, p0 + k);
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      v[e] = *reinterpret_cast<const cpx<T> *>(reinterpret_cast<const char *>(hk + ((G * e) << kTileLog2)) + off);
+    for (int e = 0; e < 16; ++e) {
+      if (occ_row(occ, jw + G * e, g))
+        v[e] = *reinterpret_cast<const cpx<T> *>(reinterpret_cast<const char *>(hk + ((G * e) << kTileLog2)) + off);
+      else
+        v[e] = fftc::mk((T)0, (T)0);
+    }
   };
   cpx<T> nx[16];
   if (ColCfg<T, N>::prefetch) load(nx, k1 - 1);
@@ -164,6 +172,7 @@ __global__ void __launch_bounds__((ColCfg<T, N>::inv_threads), (ColCfg<T, N>::in
     }
   }
   const unsigned off = sizeof(cpx<T>) * (unsigned)((col >= 0 ? ht_slot(g, sl) : 0) + ht_row(j));
+  const int jw = __builtin_amdgcn_readfirstlane(j);  // col_fwd_kernel: rows outside Geom::occ are not read
   for (int k = k0; k < k1; ++k) {
     cpx<T> v[16];
 #pragma unroll
@@ -179,10 +188,12 @@ __global__ void __launch_bounds__((ColCfg<T, N>::inv_threads), (ColCfg<T, N>::in
 #pragma unroll
     for (int e = 0; e < 16; ++e) __asm__ volatile("" : "+v"(v[e].x), "+v"(v[e].y));
     cpx<T> *hk = H + h_plane(g, k);
+    const uint64_t occ = occ_mask(g, p0 + k);
     if (col >= 0) {
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        *reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(hk + ((G * e) << kTileLog2)) + off) = v[e];
+        if (occ_row(occ, jw + G * e, g))
+          *reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(hk + ((G * e) << kTileLog2)) + off) = v[e];
     }
   }
 }

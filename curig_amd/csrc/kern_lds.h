@@ -604,6 +604,10 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
   // consecutive items of one XCD; the XCDs take such blocks in turn
   const int item = xcd_interleave(blockIdx.x, gridDim.x, 4 * S);
   const int row0 = item / S, h = item % S;
+  // planes whose block of rows holds no record are passed over
+  PlaneWalk pw(g, p0, 0, nb, row0, row0);
+  int pn = pw.next();
+  if (pn >= nb) return;
   // FP32 parts of 4096 accumulate in block floating point (kAccFix), not
   // with LDS float atomics
   const bool regs = E == 16 && m == 4096, fix = kFixable && regs;
@@ -612,7 +616,7 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
   if (kFixable && j == 0) fixnan = 0;
   const int ntot = fftc::padded_size(m);
   const auto tv = lds_twiddles<T>(lds + ntot, tw, nf1);
-  if (j < 64) walk_table_build(wt[0], off, g, p0, row0, 1);
+  if (j < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, 1);
   for (int i = j; i < ntot; i += nt) lds[i] = fftc::mk((T)0, (T)0);
   if (j < KWM) {
     // w^(sign h i) for the taps i (part h's decimation factor), from the
@@ -637,11 +641,12 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
     r0 = recs[idx0];
   }
   int cur = 0;
-  for (int pl = 0; pl < nb; ++pl, cur ^= 1) {
+  for (int pl = pn; pl < nb; pl = pn, cur ^= 1) {
     const int p = p0 + pl, total = wt[cur].total;
-    const bool more = pl + 1 < nb;
+    pn = pw.next();
+    const bool more = pn < nb;
     WalkAhead wa;
-    if (j < 64 && more) walk_issue(wa, off, g, p + 1, row0);
+    if (j < 64 && more) walk_issue(wa, off, g, p0 + pn, row0);
     if (fix && total > 0) {
       // block bounds (kAccFix); a plane without records leaves the table zero
       if (j < total) bound_row_part<T, KWM>(r0, idx0, taps, g, p, row0, m - 1, fixt);
@@ -787,6 +792,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_kernel(
   const int nf1 = g.nf1, m = nf1 / S, N1 = g.N1, nt = blockDim.x;
   const int item = xcd_group(blockIdx.x, gridDim.x);
   const int row0 = item / S, h = item % S, pl = blockIdx.y, p = p0 + pl;
+  if (!occ_row(occ_mask(g, p), row0, g)) return;
   const int lgm = 31 - __clz(m);
   const cpx<T> *hb = H + h_plane(g, pl) + ht_row(row0);
   // Input e of this thread is X[S i + h], i = tid + e nt (< m = E nt).  With
@@ -867,8 +873,11 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_planes_kernel(
   const int nf1 = g.nf1, N1 = g.N1, nt = blockDim.x, j = threadIdx.x;
   const int item = xcd_interleave(blockIdx.x, gridDim.x, 4 * S);
   const int row0 = item / S, h = item % S;
+  PlaneWalk pw(g, p0, 0, nb, row0, row0);
+  int pn = pw.next();
+  if (pn >= nb) return;
   const auto tv = lds_twiddles<T>(lds + fftc::padded_size(m), tw, nf1);
-  if (j < 64) walk_table_build(wt[0], off, g, p0, row0, 1);
+  if (j < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, 1);
   if (j < KWM) {
     // w^(sign h i) for the taps i, from the global table (the LDS copy is being written)
     const int lb = fftc::twiddle_split(nf1);
@@ -885,9 +894,10 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_planes_kernel(
   const long estep = (long)(nt >> kTileLog2) * g.tstride, mstep = (long)(m >> kTileLog2) * g.tstride;
   const long a0off = (long)ht_row(row0) + ht_slot(g, (h << g.slot_lg) + j + q);
   int cur = 0;
-  for (int pl = 0; pl < nb; ++pl, cur ^= 1) {
+  for (int pl = pn; pl < nb; pl = pn, cur ^= 1) {
     const int p = p0 + pl;
-    const bool more = pl + 1 < nb;
+    pn = pw.next();
+    const bool more = pn < nb;
     cpx<T> v[E];
     {
       const cpx<T> *a0 = H + h_plane(g, pl) + a0off;
@@ -902,7 +912,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_planes_kernel(
       }
     }
     WalkAhead wa;
-    if (j < 64 && more) walk_issue(wa, off, g, p + 1, row0);
+    if (j < 64 && more) walk_issue(wa, off, g, p0 + pn, row0);
     __syncthreads();  // the previous plane's interpolation is done with the LDS; this plane's walk table is complete
     const int total = wt[cur].total;
     if (total > 0) {
@@ -1102,9 +1112,15 @@ __global__ void __launch_bounds__(colr::NT) col_fwd_reg_kernel(const cpx<T> *__r
     const int k = horner ? nb - 1 - i : i;
     const cpx<T> *hk = H + h_plane(g, k);
     cpx<T> v[16];
+    const uint64_t occ = occ_mask(g, p0 + k);  // as in col_fwd_kernel
+    const int jw = __builtin_amdgcn_readfirstlane(j);
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      v[r] = *reinterpret_cast<const cpx<T> *>(reinterpret_cast<const char *>(hk + ((1024 * r) << kTileLog2)) + off);
+    for (int r = 0; r < 16; ++r) {
+      if (occ_row(occ, jw + 1024 * r, g))
+        v[r] = *reinterpret_cast<const cpx<T> *>(reinterpret_cast<const char *>(hk + ((1024 * r) << kTileLog2)) + off);
+      else
+        v[r] = fftc::mk((T)0, (T)0);
+    }
     colr::fft(v, buf, +1, tv);
     if (horner) {
 #pragma unroll
@@ -1223,10 +1239,14 @@ __global__ void __launch_bounds__(colr::NT) col_inv_reg_kernel(const cpx<T> *__r
     }
     colr::fft(v, buf, -1, tv);
     cpx<T> *hk = H + h_plane(g, k);
+    const uint64_t occ = occ_mask(g, p0 + k);
+    const int jw = __builtin_amdgcn_readfirstlane(j);
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      *reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(hk + ((1024 * (e >> 2) + 4096 * (e & 3)) << kTileLog2)) + off) =
-          v[e];
+    for (int e = 0; e < 16; ++e) {
+      const int r = 1024 * (e >> 2) + 4096 * (e & 3);
+      if (occ_row(occ, jw + r, g))
+        *reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(hk + (r << kTileLog2)) + off) = v[e];
+    }
   }
 }
 

@@ -91,8 +91,12 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
+  // planes whose blocks of rows (two at most, rpw <= 64) hold no record are passed over
+  PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
+  int pn = pw.next();
+  if (pn >= k1) return;
   const auto tv = lds_twiddles<T>(ltw, tw, nf1);
-  if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, nrows);
+  if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, nrows);
   for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{0, 0};
   if (kFix) {
     for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
@@ -100,11 +104,12 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
   }
   __syncthreads();
   int cur = 0;
-  for (int pl = k0; pl < k1; ++pl, cur ^= 1) {
+  for (int pl = pn; pl < k1; pl = pn, cur ^= 1) {
     const int p = p0 + pl, total = wt[cur].total;
-    const bool more = pl + 1 < k1;
+    pn = pw.next();
+    const bool more = pn < k1;
     WalkAhead wa;
-    if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, nrows);
+    if (tid < 64 && more) walk_issue(wa, off, g, p0 + pn, row0, nrows);
     if (kFix && total > 0) {
       bound_records<T, KWM>(wt[cur], total, recs, taps, g, p, row0, nrows, fixt, nblk);
       __syncthreads();
@@ -116,8 +121,9 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
     cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
     if (total == 0) {
       // no visibility reaches these rows of this plane (and the LDS is still clear)
+      const uint64_t occ = occ_mask(g, p);
       for (int r = 0; r < nrows && !add; ++r)
-        for (int i = tid; i < N1; i += nt) hb[h_slot(g, i) + (r << kTileLog2)] = fftc::mk((T)0, (T)0);
+        for (int i = occ_row(occ, row0 + r, g) ? tid : N1; i < N1; i += nt) hb[h_slot(g, i) + (r << kTileLog2)] = fftc::mk((T)0, (T)0);
       continue;
     }
     const bool pnan = kFix && fixnan;  // cleared below, after the transform's barriers
@@ -181,17 +187,21 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_interp_mix_kernel(
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
+  PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
+  int pn = pw.next();
+  if (pn >= k1) return;
   const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
-  if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, nrows);
+  if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, nrows);
   // rows past the grid (the last workgroup): zero sequences, transformed along
   for (int i = tid; i < P.count * P.stride; i += nt) buf[i] = fftc::mk((T)0, (T)0);
   __syncthreads();
   int cur = 0;
-  for (int pl = k0; pl < k1; ++pl, cur ^= 1) {
+  for (int pl = pn; pl < k1; pl = pn, cur ^= 1) {
     const int p = p0 + pl, total = wt[cur].total;
-    const bool more = pl + 1 < k1;
+    pn = pw.next();
+    const bool more = pn < k1;
     WalkAhead wa;
-    if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, nrows);
+    if (tid < 64 && more) walk_issue(wa, off, g, p0 + pn, row0, nrows);
     if (total > 0) {
       mix_load_rows<T>(buf, H + h_plane(g, pl), g, P, row0, nrows, N1);
       __syncthreads();
@@ -211,7 +221,7 @@ template <typename T>
 __global__ void __launch_bounds__(MixThreads<T>::value) row_planes_mix_kernel(const cpx<T> *__restrict__ H,
                                                                              cpx<T> *__restrict__ grid,
                                                                              const cpx<T> *__restrict__ tw, Geom g,
-                                                                             fftm::Plan P, int nb, int pchunk) {
+                                                                             fftm::Plan P, int p0, int nb, int pchunk) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
@@ -219,7 +229,8 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_planes_mix_kernel(co
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
   for (int i = tid; i < P.count * P.stride; i += nt) buf[i] = fftc::mk((T)0, (T)0);
-  for (int pl = k0; pl < k1; ++pl) {
+  PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
+  for (int pl = pw.next(); pl < k1; pl = pw.next()) {
     __syncthreads();  // the previous plane's rows are written
     mix_load_rows<T>(buf, H + h_plane(g, pl), g, P, row0, nrows, N1);
     __syncthreads();
@@ -255,21 +266,30 @@ __global__ void __launch_bounds__(MT) col_fwd_mix_kernel(const cpx<T> *__restric
   }
   for (int k = k1 - 1; k >= k0; --k) {
     const cpx<T> *hk = H + h_plane(g, k);
+    const uint64_t occ = occ_mask(g, p0 + k);  // rows outside it are zero and not in H
     __syncthreads();  // the previous plane's LDS reads are done
     constexpr int B = 8;  // loads in flight
-    for (int i0 = tid; i0 < nin; i0 += B * nt) {
-      cpx<T> v[B];
+    auto load = [&](auto all) {
+      for (int i0 = tid; i0 < nin; i0 += B * nt) {
+        cpx<T> v[B];
 #pragma unroll
-      for (int b = 0; b < B; ++b) {
-        const int i = i0 + b * nt, c = i & (cpw - 1);
-        v[b] = i < nin && c < cols ? hk[h_slot(g, s0 + c) + ((i >> cpw_lg) << kTileLog2)] : fftc::mk((T)0, (T)0);
-      }
+        for (int b = 0; b < B; ++b) {
+          const int i = i0 + b * nt, c = i & (cpw - 1);
+          const bool on = i < nin && c < cols && (all.value || occ_row(occ, i >> cpw_lg, g));
+          v[b] = on ? hk[h_slot(g, s0 + c) + ((i >> cpw_lg) << kTileLog2)] : fftc::mk((T)0, (T)0);
+        }
 #pragma unroll
-      for (int b = 0; b < B; ++b) {
-        const int i = i0 + b * nt;
-        if (i < nin) buf[(i & (cpw - 1)) * P.stride + fftc::pad(i >> cpw_lg)] = v[b];
+        for (int b = 0; b < B; ++b) {
+          const int i = i0 + b * nt;
+          if (i < nin) buf[(i & (cpw - 1)) * P.stride + fftc::pad(i >> cpw_lg)] = v[b];
+        }
       }
-    }
+    };
+    // the test of every row costs as much as the reads it saves on a fully occupied plane
+    if (occ_full(occ, g))
+      load(std::true_type());
+    else
+      load(std::false_type());
     __syncthreads();
     mix_stages<T, +1>(buf, P, tv, 0, 1);
 #pragma unroll
@@ -349,9 +369,10 @@ __global__ void __launch_bounds__(MT) col_inv_mix_kernel(const cpx<T> *__restric
     __syncthreads();
     mix_stages<T, -1>(buf, P, tv, 0, 1);
     cpx<T> *hk = H + h_plane(g, k);
+    const uint64_t occ = occ_mask(g, p0 + k);
     for (int i = tid; i < nout; i += nt) {
       const int c = i & (cpw - 1), k2 = i >> cpw_lg;
-      if (c < cols) hk[ht_slot(g, s0 + c) + ht_row(k2)] = buf[c * P.stride + fftc::pad(k2)];
+      if (c < cols && occ_row(occ, k2, g)) hk[ht_slot(g, s0 + c) + ht_row(k2)] = buf[c * P.stride + fftc::pad(k2)];
     }
   }
 }
@@ -407,7 +428,7 @@ void mix_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx
   const int lb = mix_row_lds<T>(g, false), nt = cp.rowf.nt;
   if (g.gather) {
     cpx<T> *planes = (cpx<T> *)grid;
-    row_planes_mix_kernel<T><<<grd, nt, lb, st>>>(H, planes, tw1, g, cp.rowf, nb, g.pch_row);
+    row_planes_mix_kernel<T><<<grd, nt, lb, st>>>(H, planes, tw1, g, cp.rowf, p0, nb, g.pch_row);
     launch_gather<T>(recs, taps, off, planes, vacc, g, cp.nvalid, p0, nb, st);
     return;
   }
@@ -443,7 +464,7 @@ template <typename T> int allow_mix(const ChanPlan &cp) {
   const Geom &g = cp.g;
   const int top = MixThreads<T>::value, rows = cp.rowf.nt, cols = cp.colf.nt;
   // what the kernels assume of their launches
-  if (cp.rowf.n != g.nf1 || cp.rowf.count != g.rpw || cp.colf.n != g.nf2 || cp.colf.count != g.cpw || rows < 64 ||
+  if (cp.rowf.n != g.nf1 || cp.rowf.count != g.rpw || g.rpw > 64 || cp.colf.n != g.nf2 || cp.colf.count != g.cpw || rows < 64 ||
       rows > top || cols < 64 || cols > top || mix_cells(g.cpw, g.N2, cols) > 16 || g.pch_row < 1 || g.pch_fwd < 1 ||
       g.pch_inv < 1 || g.zrow < 1 || (g.cpw & (g.cpw - 1)) != 0) {
     set_error("mixed-radix plan of grid %d x %d does not fit its kernels", g.nf2, g.nf1);

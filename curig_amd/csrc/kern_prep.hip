@@ -224,6 +224,43 @@ __global__ void __launch_bounds__(256) bin_scatter_kernel(const double *__restri
   }
 }
 
+// Whether any of the bins [s0, s1] of layer l holds a record
+__device__ __forceinline__ bool strips_hold(const int *__restrict__ off, const Geom &g, int l, int s0, int s1) {
+  return off[l * g.ntiles + s1 + 1] > off[l * g.ntiles + s0];
+}
+
+// Geom::occ from the bin offsets (full-width row strips, LDS path): a wavefront
+// per plane, a lane per block of rows.  The records that reach rows [r0, r1] of
+// plane p have iy in [r0 - kw + 1, r1] and iw in [p - kww + 1, p], both cyclic;
+// the answer is that of their bins, so it holds every row and plane whose walk
+// (walk_table_build) finds a record.
+// An observation leaves rows of the grid empty: a 128-antenna, 5 km array on
+// 8192^2 pixels of 6 degrees reaches 63% of its rows and planes.  The row passes
+// leave the empty ones out and H without them, and the column passes neither read
+// nor write them: 32 planes of 16384^2, image rows 21.0 -> 13.5 ms and columns 14.4
+// -> 12.4, prediction rows 14.1 -> 10.7; 8192^2, 66% occupied, rows 5.05 -> 3.97
+// ms, columns 3.13 -> 2.86 per 26 planes.
+__global__ void __launch_bounds__(256) occ_kernel(const int *__restrict__ off, Geom g, uint64_t *__restrict__ occ) {
+  const int p = (int)((blockIdx.x * (long)blockDim.x + threadIdx.x) >> 6), b = threadIdx.x & 63;
+  if (p >= g.P) return;
+  const int r0 = b << g.occ_lg, r1 = min(g.nf2, r0 + (1 << g.occ_lg)) - 1;
+  bool any = false;
+  if (r0 < g.nf2) {
+    // [lo, hi] and, wrapped below row 0, [wl, nf2 - 1]
+    const int lo = r0 - g.kw + 1, wl = lo < 0 ? max(lo + g.nf2, 0) : g.nf2;
+    const int a0 = max(lo, 0) / g.T2, a1 = r1 / g.T2, b0 = wl / g.T2, b1 = (g.nf2 - 1) / g.T2;
+    // layers of planes pl .. p, and wrapped ones wp .. P - 1
+    const int pl = p - g.kww + 1, wp = pl < 0 ? max(pl + g.P, 0) : g.P;
+    for (int l = max(pl, 0) / g.Pbin; l <= p / g.Pbin; ++l)
+      any = any || strips_hold(off, g, l, a0, a1) || (wl < g.nf2 && strips_hold(off, g, l, b0, b1));
+    if (wp < g.P)
+      for (int l = wp / g.Pbin; l <= (g.P - 1) / g.Pbin; ++l)
+        any = any || strips_hold(off, g, l, a0, a1) || (wl < g.nf2 && strips_hold(off, g, l, b0, b1));
+  }
+  const uint64_t m = __ballot(any);
+  if (b == 0) occ[p] = m;
+}
+
 // --------------------------------------------------------------------------
 // launchers
 // --------------------------------------------------------------------------
@@ -273,6 +310,10 @@ void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
                                                                    (Rec<T> *)b.recs, b.perm, with_value ? 1 : 0,
                                                                    taps);
   }
+}
+
+void launch_occ(const int *off, const Geom &g, uint64_t *occ, hipStream_t st) {
+  occ_kernel<<<(g.P + 3) / 4, 256, 0, st>>>(off, g, occ);
 }
 
 template void enqueue_binning<float>(const Problem &, const ChanPlan &, const Bufs &, hipStream_t, bool);

@@ -44,7 +44,12 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
-  if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, rpw);
+  // planes whose block of rows holds no record are passed over (rpw, a power of
+  // two of at most 64, keeps to a block)
+  PlaneWalk pw(g, p0, k0, k1, row0, row0);
+  int pn = pw.next();
+  if (pn >= k1) return;
+  if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, rpw);
   for (int i = tid; i < rpw * F::kStride; i += nt) acc[i] = Cell{0, 0};
   if (kFix) {
     for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
@@ -54,11 +59,12 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
   fft.init(tw, j, nullptr);
   __syncthreads();
   int cur = 0;
-  for (int pl = k0; pl < k1; ++pl, cur ^= 1) {
+  for (int pl = pn; pl < k1; pl = pn, cur ^= 1) {
     const int p = p0 + pl, total = wt[cur].total;
-    const bool more = pl + 1 < k1;
+    pn = pw.next();
+    const bool more = pn < k1;
     WalkAhead wa;
-    if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, rpw);
+    if (tid < 64 && more) walk_issue(wa, off, g, p0 + pn, row0, rpw);
     if (kFix && total > 0) {
       bound_records<T, KWM>(wt[cur], total, recs, taps, g, p, row0, rpw, fixt, nblk);
       __syncthreads();
@@ -138,16 +144,20 @@ __global__ void __launch_bounds__(RowThreads<N>::value) row_interp_reg_kernel(
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw), *own = buf + s * F::kStride;
   const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
-  if (tid < 64) walk_table_build(wt[0], off, g, p0 + k0, row0, rpw);
+  PlaneWalk pw(g, p0, k0, k1, row0, row0);
+  int pn = pw.next();
+  if (pn >= k1) return;
+  if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, rpw);
   F fft;
   fft.init(tw, j, nullptr);
   __syncthreads();
   int cur = 0;
-  for (int pl = k0; pl < k1; ++pl, cur ^= 1) {
+  for (int pl = pn; pl < k1; pl = pn, cur ^= 1) {
     const int p = p0 + pl, total = wt[cur].total;
-    const bool more = pl + 1 < k1;
+    pn = pw.next();
+    const bool more = pn < k1;
     WalkAhead wa;
-    if (tid < 64 && more) walk_issue(wa, off, g, p + 1, row0, rpw);
+    if (tid < 64 && more) walk_issue(wa, off, g, p0 + pn, row0, rpw);
     if (total > 0) {
       cpx<T> v[16];
       load_row_elems<T, N>(v, H, g, pl, row0 + s, j);
@@ -168,7 +178,7 @@ template <typename T, int N>
 __global__ void __launch_bounds__(RowThreads<N>::value) row_planes_reg_kernel(const cpx<T> *__restrict__ H,
                                                                              cpx<T> *__restrict__ grid,
                                                                              const cpx<T> *__restrict__ tw, Geom g,
-                                                                             int nb, int pchunk) {
+                                                                             int p0, int nb, int pchunk) {
   using F = RegFft<T, N, -1>;
   constexpr int G = F::G;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -176,9 +186,10 @@ __global__ void __launch_bounds__(RowThreads<N>::value) row_planes_reg_kernel(co
   cpx<T> *own = reinterpret_cast<cpx<T> *>(smem_raw) + s * F::kStride;
   const int row = xcd_group(blockIdx.x, gridDim.x) * rpw + s;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
+  PlaneWalk pw(g, p0, k0, k1, row & ~(rpw - 1), row & ~(rpw - 1));
   F fft;
   fft.init(tw, j, nullptr);
-  for (int pl = k0; pl < k1; ++pl) {
+  for (int pl = pw.next(); pl < k1; pl = pw.next()) {
     cpx<T> v[16];
     load_row_elems<T, N>(v, H, g, pl, row, j);
     __syncthreads();  // the previous plane's LDS reads are done
@@ -246,7 +257,7 @@ void rowreg_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx<
   const int lb = rowreg_lds<T>(g, false), nt = g.rpw * g.nf1 / 16;
   with_row_len<T>(g.nf1, [&](auto N) {
     if (g.gather) {
-      row_planes_reg_kernel<T, N.value><<<grd, nt, lb, st>>>(H, (cpx<T> *)grid, tw1, g, nb, g.pch_row);
+      row_planes_reg_kernel<T, N.value><<<grd, nt, lb, st>>>(H, (cpx<T> *)grid, tw1, g, p0, nb, g.pch_row);
     } else if constexpr (N.value != 4096) {
       if (g.kw <= 8)
         row_interp_reg_kernel<T, 8, N.value><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, nb, g.pch_row);
@@ -263,7 +274,7 @@ template <typename T> int allow_rowreg(const Geom &g, bool spread) {
   int ier = kErrArg;
   const bool known = with_row_len<T>(g.nf1, [&](auto N) {
     constexpr int n = N.value;
-    if (g.rpw < 1 || nt < 64 || nt > RowThreads<n>::value || g.nf2 % g.rpw || g.pch_row < 1 || g.zrow < 1) return;
+    if (g.rpw < 1 || g.rpw > 64 || (g.rpw & (g.rpw - 1)) || nt < 64 || nt > RowThreads<n>::value || g.nf2 % g.rpw || g.pch_row < 1 || g.zrow < 1) return;
     if (spread) {
       with_acc64<T>(g.acc64, [&](auto A) {
         if constexpr (n != 4096 || A.value) {

@@ -52,6 +52,7 @@ struct Bufs {
   void *recs = nullptr, *grid = nullptr, *H = nullptr;
   void *taps = nullptr;  // LDS path: each record's kernel taps, [nrec][3][tap_width] of the precision
   double2 *acc = nullptr, *vacc = nullptr;
+  uint64_t *occ = nullptr;  // LDS path: Geom::occ of the running problem
   const void *tw1 = nullptr, *tw2 = nullptr;
   const double *hc_d = nullptr;  // piecewise-polynomial kernel coefficients, FP64 | FP32
   const float *hc_f = nullptr;
@@ -114,6 +115,7 @@ void launch_pack_columns(const Columns &c, double *uvw, int n, hipStream_t st);
 // count, scan and scatter of one problem's rows into bin order (records and permutation)
 template <typename T>
 void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipStream_t st, bool with_value);
+void launch_occ(const int *off, const Geom &g, uint64_t *occ, hipStream_t st);
 void launch_fill_zero_c128(double2 *p, long n, hipStream_t st);
 void launch_zero_rows(bool dbl, void *vis, long stride, int nrow, hipStream_t st);
 

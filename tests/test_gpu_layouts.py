@@ -188,3 +188,40 @@ def test_w_correction_against_direct_sum(eps):
     say(f"[w correction] eps {eps}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
     tol = max(3 * eps, 1e-12)
     assert e1 < tol and e2 < tol
+
+
+# records in few rows and planes: the other rows are neither written to nor read
+# from the intermediate planes, which a call on non-finite values fills first.
+# Blocks of 64 and more rows, grids below one block, records across row 0 and
+# across the last plane, batches of more planes than one mask word holds
+OCCUPIED = [("fp64", 64, 64), ("fp32", 64, 64), ("fp64", 1024, 64), ("fp32", 2048, 64), ("fp64", 64, 2048),
+            ("fp32", 64, 2048), ("fp32", 64, 4096), ("fp64", 64, 4096), ("fp32", 64, 8192), ("fp32", 8192, 64),
+            ("fp64", 8192, 64), ("fp64", 600, 90), ("fp32", 1500, 75)]
+
+
+@pytest.mark.parametrize("precision,nx,ny", OCCUPIED)
+@pytest.mark.parametrize("planes", [0, 70])
+def test_rows_without_records(precision, nx, ny, planes):
+    lib = _lib()
+    fov, eps, wmax = 2.0, 1e-6, 3000.0
+    uvw, vis, wgt, img, f0 = _case(400, nx, ny, fov, wmax, nx + ny)
+    uvw[:, 0] = np.where(np.arange(400) % 2, 0.02, 0.3) * uvw[:, 0]
+    uvw[:, 2] = np.where(np.arange(400) % 2, uvw[:, 2], 0.9 * wmax + 0.1 * uvw[:, 2])
+    image = gpu_ms2dirty if precision == "fp64" else (lambda *a: gpu_f32(True, *a))
+    predict = gpu_dirty2ms if precision == "fp64" else (lambda *a: gpu_f32(False, *a))
+    assert lib.curig_set_tuning(0, 0, planes, 0) == 0
+    try:
+        full = _case(400, nx, ny, fov, wmax, 5)[0]
+        image(full, np.full(400, np.inf + 0j), wgt, nx, ny, fov, f0, eps)
+        d = image(uvw, vis, wgt, nx, ny, fov, f0, eps)
+        predict(full, np.full((nx, ny), np.inf + 0j), wgt, nx, ny, fov, f0, eps)
+        v = predict(uvw, img, wgt, nx, ny, fov, f0, eps)
+        lib.curig_set_fft_path(1)
+        e1 = O.l2error(image(uvw, vis, wgt, nx, ny, fov, f0, eps), d)
+        e2 = O.l2error(predict(uvw, img, wgt, nx, ny, fov, f0, eps), v)
+    finally:
+        lib.curig_set_fft_path(0)
+        lib.curig_set_tuning(0, 0, 0, 0)
+    say(f"[rows without records] {precision} {nx}x{ny} planes {planes}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
+    tol = 1e-11 if precision == "fp64" else 2e-6
+    assert e1 < tol and e2 < tol
