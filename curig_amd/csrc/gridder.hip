@@ -53,7 +53,7 @@ namespace {
 // serialised on the host (g_ws_mu), and a call on another stream than the
 // previous call's waits for that call's launches on the device (ws_order).
 enum Slot {
-  S_PART, S_CNT, S_HIST, S_OFF, S_BSUM, S_BINRANK, S_RECS, S_PERM, S_GRID, S_ACC, S_VACC, S_TAB, S_FFTW,
+  S_PART, S_CNT, S_HIST, S_OFF, S_BSUM, S_BINRANK, S_RECS, S_SLOT, S_GRID, S_ACC, S_VACC, S_TAB, S_FFTW,
   S_H, S_TW, S_HC, S_TAPS, S_UVW, S_OCC,
   S_NSLOT
 };
@@ -867,8 +867,8 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule
   b.binrank = (int2 *)vp;
   CURIG_TRY(ws_get(dev, S_RECS, sizeof(Rec<T>) * nrow, &vp));
   b.recs = vp;
-  CURIG_TRY(ws_get(dev, S_PERM, sizeof(int) * nrow, &vp));
-  b.perm = (int *)vp;
+  CURIG_TRY(ws_get(dev, S_SLOT, sizeof(int) * nrow, &vp));
+  b.slot = (int *)vp;
   CURIG_TRY(ws_get(dev, S_GRID, sizeof(v2_t<T>) * grid, &vp));
   b.grid = vp;
   CURIG_TRY(ws_get(dev, S_ACC, sizeof(double2) * npix, &vp));
@@ -1075,8 +1075,6 @@ int enqueue_dirty2ms(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   Range rp("curig dirty2ms binning and prologue");
   enqueue_binning<T>(pb, cp, b, st, false);
   if (g.occ) launch_occ(b.off, g, b.occ, st);
-  // every output row is written: flagged rows get 0
-  launch_zero_rows(pb.dbl, pb.vis, pb.vis_stride, pb.nrow, st);
   const Rec<T> *recs = (const Rec<T> *)b.recs;
   v2_t<T> *grid = (v2_t<T> *)b.grid;
   double2 *gimg = b.acc;
@@ -1132,7 +1130,7 @@ int enqueue_dirty2ms(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   }
   int e2 = tm.mark();
   Range rf("curig dirty2ms finalize");
-  launch_finalize(pb.dbl, b.perm, b.vacc, (int)cp.nvalid, pb.uvw, pb.wgt, pb.wgt_stride, pb.vis, pb.vis_stride, g,
+  launch_finalize(pb.dbl, b.slot, b.vacc, pb.nrow, pb.uvw, pb.wgt, pb.wgt_stride, pb.vis, pb.vis_stride, g,
                   st);
   CURIG_HIP(hipGetLastError());
   int e3 = tm.mark();
@@ -1198,7 +1196,7 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
       << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.occ_lg << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
-  k << b.dev << b.occ << b.tabs << b.hist << b.off << b.bsum << b.perm << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc
+  k << b.dev << b.occ << b.tabs << b.hist << b.off << b.bsum << b.slot << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc
     << b.vacc << b.tw1 << b.tw2 << b.hc_d << b.hc_f;
   return k.h;
 }

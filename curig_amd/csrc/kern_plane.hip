@@ -378,14 +378,21 @@ __global__ void __launch_bounds__(256) interp_kernel(const Rec<T> *__restrict__ 
   }
 }
 
-// finalize (dirty2ms): vis_j = acc * wgt_j * e^{-i D w_j}  (ra_exec.cu:56-89)
+// finalize (dirty2ms): vis_j = acc * wgt_j * e^{-i D w_j}  (ra_exec.cu:56-89),
+// flagged rows 0.  In the order of the rows: their sums are gathered and the rest
+// is read and written in whole lines; in the records' order, with a pass of zeros
+// before it, 20M points took 0.80 + 0.02 ms (0.35 here), 2M 109 + 25 us (60 here).
 template <typename T>
-__global__ void __launch_bounds__(256) finalize_kernel(const int *__restrict__ perm, const double2 *__restrict__ vacc,
-                                                        int nrec, const double *__restrict__ uvw,
+__global__ void __launch_bounds__(256) finalize_kernel(const int *__restrict__ slot, const double2 *__restrict__ vacc,
+                                                        int nrow, const double *__restrict__ uvw,
                                                         const void *__restrict__ wgt, long ws,
                                                         void *__restrict__ vis, long vs, Geom g) {
-  for (long s = blockIdx.x * (long)blockDim.x + threadIdx.x; s < nrec; s += (long)gridDim.x * blockDim.x) {
-    long j = perm[s];
+  for (long j = blockIdx.x * (long)blockDim.x + threadIdx.x; j < nrow; j += (long)gridDim.x * blockDim.x) {
+    const int s = slot[j];
+    if (s < 0) {
+      store_c<T>(vis, j * vs, 0.0, 0.0);
+      continue;
+    }
     double we = uvw[3 * j + 2] * g.wscale;
     double sn, cs;
     sincos(-g.D * we, &sn, &cs);
@@ -585,13 +592,13 @@ void launch_prologue_cols(bool dbl_in, const void *dirty, cpx<T> *gT, const Geom
     prologue_cols_kernel<float, T><<<nblocks(npix), 256, 0, st>>>(dirty, gT, g, fk1, fk2, q);
 }
 
-void launch_finalize(bool dbl, const int *perm, const double2 *vacc, int nrec, const double *uvw, const void *wgt,
+void launch_finalize(bool dbl, const int *slot, const double2 *vacc, int nrow, const double *uvw, const void *wgt,
                      long ws, void *vis, long vs, const Geom &g, hipStream_t st) {
-  if (nrec <= 0) return;
+  if (nrow <= 0) return;
   if (dbl)
-    finalize_kernel<double><<<nblocks(nrec), 256, 0, st>>>(perm, vacc, nrec, uvw, wgt, ws, vis, vs, g);
+    finalize_kernel<double><<<nblocks(nrow), 256, 0, st>>>(slot, vacc, nrow, uvw, wgt, ws, vis, vs, g);
   else
-    finalize_kernel<float><<<nblocks(nrec), 256, 0, st>>>(perm, vacc, nrec, uvw, wgt, ws, vis, vs, g);
+    finalize_kernel<float><<<nblocks(nrow), 256, 0, st>>>(slot, vacc, nrow, uvw, wgt, ws, vis, vs, g);
 }
 
 void launch_corr_tables(const QuadRule &q, int nf1, int nf2, double *tabs, hipStream_t st) {

@@ -47,7 +47,7 @@ struct ChanPlan {
 struct Bufs {
   int dev = 0;
   double *tabs = nullptr;  // fk1 [nf1/2+1] | fk2 [nf2/2+1] | quadrature nodes | weights
-  int *hist = nullptr, *off = nullptr, *bsum = nullptr, *perm = nullptr;
+  int *hist = nullptr, *off = nullptr, *bsum = nullptr, *slot = nullptr;
   int2 *binrank = nullptr;
   void *recs = nullptr, *grid = nullptr, *H = nullptr;
   void *taps = nullptr;  // LDS path: each record's kernel taps, [nrec][3][tap_width] of the precision
@@ -112,12 +112,11 @@ constexpr int kScanTile = kScanBlock * kScanItems;
 void launch_w_minmax(int nblk, const double *uvw, int nrow, const uint8_t *flag, long fs, double *part, int *cnt,
                      hipStream_t st);
 void launch_pack_columns(const Columns &c, double *uvw, int n, hipStream_t st);
-// count, scan and scatter of one problem's rows into bin order (records and permutation)
+// count, scan and scatter of one problem's rows into bin order (records, and for dirty2ms each row's record)
 template <typename T>
 void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipStream_t st, bool with_value);
 void launch_occ(const int *off, const Geom &g, uint64_t *occ, hipStream_t st);
 void launch_fill_zero_c128(double2 *p, long n, hipStream_t st);
-void launch_zero_rows(bool dbl, void *vis, long stride, int nrow, hipStream_t st);
 
 // ---- kern_plane.hip: full-plane path (rocFFT grids), corrections, direct sums
 void launch_corr_tables(const QuadRule &q, int nf1, int nf2, double *tabs, hipStream_t st);
@@ -138,7 +137,7 @@ void launch_prologue(bool dbl_in, const void *dirty, double2 *gimg, const Geom &
 template <typename T>
 void launch_prologue_cols(bool dbl_in, const void *dirty, cpx<T> *gT, const Geom &g, const double *fk1,
                           const double *fk2, const double *q, hipStream_t st);
-void launch_finalize(bool dbl, const int *perm, const double2 *vacc, int nrec, const double *uvw, const void *wgt,
+void launch_finalize(bool dbl, const int *slot, const double2 *vacc, int nrow, const double *uvw, const void *wgt,
                      long ws, void *vis, long vs, const Geom &g, hipStream_t st);
 void launch_explicit_ms2dirty(bool dbl, const Problem &pb, const Geom &g, double fc2pi, const int64_t *pix, long npix,
                               double2 *out, hipStream_t st);

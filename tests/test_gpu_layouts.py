@@ -225,3 +225,15 @@ def test_rows_without_records(precision, nx, ny, planes):
     say(f"[rows without records] {precision} {nx}x{ny} planes {planes}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
     tol = 1e-11 if precision == "fp64" else 2e-6
     assert e1 < tol and e2 < tol
+
+
+# rows counted in LDS by chunks: several and many rows to a bin, a short last chunk
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nx,ny,nrow", [(32, 64, 40001), (64, 64, 300007), (512, 32, 270000)])
+def test_many_rows_to_a_bin(precision, nx, ny, nrow):
+    fov, eps = 2.0, 1e-5
+    uvw, vis, wgt, img, f0 = _case(nrow, nx, ny, fov, 2.0, nx + nrow)
+    e1, e2 = _both_paths(precision, uvw, vis, wgt, img, nx, ny, fov, f0, eps)
+    say(f"[many rows to a bin] {precision} {nx}x{ny} rows {nrow}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
+    tol = 1e-11 if precision == "fp64" else 2e-6
+    assert e1 < tol and e2 < tol
