@@ -414,13 +414,23 @@ static void plan_mixed(Geom &g, size_t cs, size_t lds_max) {
   g.tstride = (g.nf2 + kTile - 1) / kTile * kTile * kTile + (int)(kTilePadBytes / cs);
 }
 
+// Planes per workgroup of the row kernels that hold whole rows (nt threads): all
+// of the batch's, or fewer until there are 4096 wavefronts, which even out rows of
+// many and of few records: 512 rows of a 256^2 FP64 image, 16 planes, 4 / 2 / 1
+// planes each 83 / 64 / 60 us; 640^2, 20 planes, 5 / 2 / 1 each 283 / 260 / 247 us.
+static int row_plane_chunk(const Geom &g, int nt) {
+  const long waves = (long)((g.nf2 + g.rpw - 1) / g.rpw) * ((nt + 63) / 64);
+  const int n = (int)((4096 + waves - 1) / waves);
+  return std::max(1, (g.Pb + n - 1) / n);
+}
+
 // Planes per workgroup of the mixed-radix passes (as plan_columns).
 static void plan_mixed_chunks(Geom &g) {
   auto chunk = [&](int groups) {
     const int n = std::min((1024 + groups - 1) / groups, 8);
     return std::max(std::min(2, g.Pb), (g.Pb + n - 1) / n);
   };
-  g.pch_row = chunk((g.nf2 + g.rpw - 1) / g.rpw);
+  g.pch_row = row_plane_chunk(g, g.nt_row);
   g.pch_fwd = g.pch_inv = chunk((g.N1 + g.cpw - 1) / g.cpw);
   g.nacc = (g.Pb + g.pch_fwd - 1) / g.pch_fwd;
 }
@@ -622,10 +632,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     plan_mixed_chunks(g);
   else if (g.fft_lds)
     plan_columns(g, cs, lds_max, tn.compact != 0);
-  if (g.rowreg) {
-    const int groups = g.nf2 / g.rpw, n = std::min((1024 + groups - 1) / groups, 8);
-    g.pch_row = std::max(std::min(2, g.Pb), (g.Pb + n - 1) / n);
-  }
+  if (g.rowreg) g.pch_row = row_plane_chunk(g, g.rpw * g.nf1 / 16);
   if ((g.rowreg || g.mix) && !tn.to_vis) {
     // Few row workgroups with many records each (a small grid, one plane): they
     // are shared by zrow workgroups, at least 4096 record visits each, whose

@@ -454,10 +454,10 @@ __device__ __forceinline__ int xcd_group(int bid, int n) {
 }
 
 // Workgroup id -> work item with blocks of blk consecutive items dealt to the
-// 8 XCDs in turn (n a multiple of 8 blk): every XCD gets the same mix of the
-// items, and a block's items share one L2.
+// 8 XCDs in turn (the last n mod 8 blk in order): every XCD gets the same mix of
+// the items, and a block's items share one L2.
 __device__ __forceinline__ int xcd_interleave(int bid, int n, int blk) {
-  if (n % (8 * blk)) return xcd_group(bid, n);
+  if (bid >= n - n % (8 * blk)) return bid;
   const int x = bid & 7, k = bid >> 3;
   return ((k / blk) * 8 + x) * blk + k % blk;
 }
@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_kernel(
   __shared__ WalkTable wt;
   cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
   const int nf1 = g.nf1, m = nf1 / S, N1 = g.N1, nt = blockDim.x;
-  const int item = xcd_group(blockIdx.x, gridDim.x);
+  const int item = xcd_interleave(blockIdx.x, gridDim.x, 4 * S);
   const int row0 = item / S, h = item % S, pl = blockIdx.y, p = p0 + pl;
   if (!occ_row(occ_mask(g, p), row0, g)) return;
   const int lgm = 31 - __clz(m);

@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
   cpx<T> *ltw = reinterpret_cast<cpx<T> *>(acc + nbuf);
   float *fixt = reinterpret_cast<float *>(ltw + fftc::twiddle_entries(nf1));
   short *fixe = reinterpret_cast<short *>(fixt + rpw * nblk);
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
+  const int row0 = row_group(g) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
   // planes whose blocks of rows (two at most, rpw <= 64) hold no record are passed over
@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_interp_mix_kernel(
   __shared__ WalkTable wt[2];
   const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
+  const int row0 = row_group(g) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
   int pn = pw.next();
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_planes_mix_kernel(co
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw, nrows = min(rpw, nf2 - row0);
+  const int row0 = row_group(g) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
   for (int i = tid; i < P.count * P.stride; i += nt) buf[i] = fftc::mk((T)0, (T)0);

@@ -41,7 +41,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
   Cell *acc = reinterpret_cast<Cell *>(smem_raw), *ownc = acc + s * F::kStride;
   float *fixt = reinterpret_cast<float *>(acc + rpw * F::kStride);
   short *fixe = reinterpret_cast<short *>(fixt + rpw * nblk);
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw;
+  const int row0 = row_group(g) * rpw;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
   // planes whose block of rows holds no record are passed over (rpw, a power of
@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) row_interp_reg_kernel(
   __shared__ WalkTable wt[2];
   const int tid = threadIdx.x, rpw = g.rpw, s = tid / G, j = tid % G;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw), *own = buf + s * F::kStride;
-  const int row0 = xcd_group(blockIdx.x, gridDim.x) * rpw;
+  const int row0 = row_group(g) * rpw;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   PlaneWalk pw(g, p0, k0, k1, row0, row0);
   int pn = pw.next();
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) row_planes_reg_kernel(co
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int tid = threadIdx.x, rpw = g.rpw, s = tid / G, j = tid % G;
   cpx<T> *own = reinterpret_cast<cpx<T> *>(smem_raw) + s * F::kStride;
-  const int row = xcd_group(blockIdx.x, gridDim.x) * rpw + s;
+  const int row = row_group(g) * rpw + s;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   PlaneWalk pw(g, p0, k0, k1, row & ~(rpw - 1), row & ~(rpw - 1));
   F fft;
