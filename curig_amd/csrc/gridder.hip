@@ -1007,7 +1007,6 @@ int enqueue_ms2dirty(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   {
     Range r("curig ms2dirty binning");
     enqueue_binning<T>(pb, cp, b, st, true);
-    if (g.occ) launch_occ(b.off, g, b.occ, st);
   }
   CURIG_HIP(hipGetLastError());
   int e1 = tm.mark();
@@ -1081,7 +1080,6 @@ int enqueue_dirty2ms(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   int e0 = tm.mark();
   Range rp("curig dirty2ms binning and prologue");
   enqueue_binning<T>(pb, cp, b, st, false);
-  if (g.occ) launch_occ(b.off, g, b.occ, st);
   const Rec<T> *recs = (const Rec<T> *)b.recs;
   v2_t<T> *grid = (v2_t<T> *)b.grid;
   double2 *gimg = b.acc;

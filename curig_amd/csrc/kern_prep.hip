@@ -190,6 +190,83 @@ __global__ void __launch_bounds__(kScanBlock) scan_apply_kernel(const int *__res
   if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = total;
 }
 
+// Whether any of the bins [s0, s1] of layer l holds a record
+__device__ __forceinline__ bool strips_hold(const int *off, const Geom &g, int l, int s0, int s1) {
+  return off[l * g.ntiles + s1 + 1] > off[l * g.ntiles + s0];
+}
+
+// Geom::occ of plane p from the bin offsets (full-width row strips, LDS path), by a
+// wavefront, a lane per block of rows.  The records that reach rows [r0, r1] of
+// plane p have iy in [r0 - kw + 1, r1] and iw in [p - kww + 1, p], both cyclic;
+// the answer is that of their bins, so it holds every row and plane whose walk
+// (walk_table_build) finds a record.
+// An observation leaves rows of the grid empty: a 128-antenna, 5 km array on
+// 8192^2 pixels of 6 degrees reaches 63% of its rows and planes.  The row passes
+// leave the empty ones out and H without them, and the column passes neither read
+// nor write them: 32 planes of 16384^2, image rows 21.0 -> 13.5 ms and columns 14.4
+// -> 12.4, prediction rows 14.1 -> 10.7; 8192^2, 66% occupied, rows 5.05 -> 3.97
+// ms, columns 3.13 -> 2.86 per 26 planes.
+__device__ __forceinline__ void occ_plane(const int *off, const Geom &g, int p, uint64_t *__restrict__ occ) {
+  const int b = threadIdx.x & 63;
+  const int r0 = b << g.occ_lg, r1 = min(g.nf2, r0 + (1 << g.occ_lg)) - 1;
+  bool any = false;
+  if (r0 < g.nf2) {
+    // [lo, hi] and, wrapped below row 0, [wl, nf2 - 1]
+    const int lo = r0 - g.kw + 1, wl = lo < 0 ? max(lo + g.nf2, 0) : g.nf2;
+    const int a0 = max(lo, 0) / g.T2, a1 = r1 / g.T2, b0 = wl / g.T2, b1 = (g.nf2 - 1) / g.T2;
+    // layers of planes pl .. p, and wrapped ones wp .. P - 1
+    const int pl = p - g.kww + 1, wp = pl < 0 ? max(pl + g.P, 0) : g.P;
+    for (int l = max(pl, 0) / g.Pbin; l <= p / g.Pbin; ++l)
+      any = any || strips_hold(off, g, l, a0, a1) || (wl < g.nf2 && strips_hold(off, g, l, b0, b1));
+    if (wp < g.P)
+      for (int l = wp / g.Pbin; l <= (g.P - 1) / g.Pbin; ++l)
+        any = any || strips_hold(off, g, l, a0, a1) || (wl < g.nf2 && strips_hold(off, g, l, b0, b1));
+  }
+  const uint64_t m = __ballot(any);
+  if (b == 0) occ[p] = m;
+}
+
+__global__ void __launch_bounds__(256) occ_kernel(const int *__restrict__ off, Geom g, uint64_t *__restrict__ occ) {
+  const int p = (int)((blockIdx.x * (long)blockDim.x + threadIdx.x) >> 6);
+  if (p < g.P) occ_plane(off, g, p, occ);
+}
+
+// The scan of few bins (kSmallScan at most) and the occupied blocks, in one
+// workgroup: a small image's call is as long as its launches, and four were here
+// (256^2 image 151 -> 138 us a call, prediction 120 -> 110).
+constexpr int kSmallScan = 16384;
+__global__ void __launch_bounds__(1024) scan_small_kernel(const int *__restrict__ in, int n, int *out, int total, Geom g,
+                                                           uint64_t *__restrict__ occ) {
+  __shared__ int ws[16];
+  const int items = (n + 1023) / 1024, base = threadIdx.x * items, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int loc[kSmallScan / 1024], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kSmallScan / 1024; ++k) {
+    loc[k] = k < items && base + k < n ? in[base + k] : 0;
+    sum += loc[k];
+  }
+  int run = sum;  // inclusive over the wavefront
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int t = __shfl_up(run, d);
+    if (lane >= d) run += t;
+  }
+  if (lane == 63) ws[wave] = run;
+  __syncthreads();
+  run -= sum;
+  for (int w = 0; w < wave; ++w) run += ws[w];
+#pragma unroll
+  for (int k = 0; k < kSmallScan / 1024; ++k) {
+    if (k < items && base + k < n) out[base + k] = run;
+    run += loc[k];
+  }
+  if (threadIdx.x == 0) out[n] = total;
+  if (!occ) return;
+  __threadfence_block();
+  __syncthreads();
+  for (int p = wave; p < g.P; p += 16) occ_plane(out, g, p, occ);
+}
+
 // Scatter rows into bin order; slot[j] (dirty2ms): row j's record, or -1; the
 // value carries the weight and e^{+i D w}
 // (ms2dirty pre-stages, src/astro/ra_exec.cu:98-110).
@@ -252,43 +329,6 @@ __global__ void __launch_bounds__(256) bin_scatter_kernel(const double *__restri
   }
 }
 
-// Whether any of the bins [s0, s1] of layer l holds a record
-__device__ __forceinline__ bool strips_hold(const int *__restrict__ off, const Geom &g, int l, int s0, int s1) {
-  return off[l * g.ntiles + s1 + 1] > off[l * g.ntiles + s0];
-}
-
-// Geom::occ from the bin offsets (full-width row strips, LDS path): a wavefront
-// per plane, a lane per block of rows.  The records that reach rows [r0, r1] of
-// plane p have iy in [r0 - kw + 1, r1] and iw in [p - kww + 1, p], both cyclic;
-// the answer is that of their bins, so it holds every row and plane whose walk
-// (walk_table_build) finds a record.
-// An observation leaves rows of the grid empty: a 128-antenna, 5 km array on
-// 8192^2 pixels of 6 degrees reaches 63% of its rows and planes.  The row passes
-// leave the empty ones out and H without them, and the column passes neither read
-// nor write them: 32 planes of 16384^2, image rows 21.0 -> 13.5 ms and columns 14.4
-// -> 12.4, prediction rows 14.1 -> 10.7; 8192^2, 66% occupied, rows 5.05 -> 3.97
-// ms, columns 3.13 -> 2.86 per 26 planes.
-__global__ void __launch_bounds__(256) occ_kernel(const int *__restrict__ off, Geom g, uint64_t *__restrict__ occ) {
-  const int p = (int)((blockIdx.x * (long)blockDim.x + threadIdx.x) >> 6), b = threadIdx.x & 63;
-  if (p >= g.P) return;
-  const int r0 = b << g.occ_lg, r1 = min(g.nf2, r0 + (1 << g.occ_lg)) - 1;
-  bool any = false;
-  if (r0 < g.nf2) {
-    // [lo, hi] and, wrapped below row 0, [wl, nf2 - 1]
-    const int lo = r0 - g.kw + 1, wl = lo < 0 ? max(lo + g.nf2, 0) : g.nf2;
-    const int a0 = max(lo, 0) / g.T2, a1 = r1 / g.T2, b0 = wl / g.T2, b1 = (g.nf2 - 1) / g.T2;
-    // layers of planes pl .. p, and wrapped ones wp .. P - 1
-    const int pl = p - g.kww + 1, wp = pl < 0 ? max(pl + g.P, 0) : g.P;
-    for (int l = max(pl, 0) / g.Pbin; l <= p / g.Pbin; ++l)
-      any = any || strips_hold(off, g, l, a0, a1) || (wl < g.nf2 && strips_hold(off, g, l, b0, b1));
-    if (wp < g.P)
-      for (int l = wp / g.Pbin; l <= (g.P - 1) / g.Pbin; ++l)
-        any = any || strips_hold(off, g, l, a0, a1) || (wl < g.nf2 && strips_hold(off, g, l, b0, b1));
-  }
-  const uint64_t m = __ballot(any);
-  if (b == 0) occ[p] = m;
-}
-
 // --------------------------------------------------------------------------
 // launchers
 // --------------------------------------------------------------------------
@@ -322,9 +362,15 @@ void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
   else if (pb.nrow > 0)
     bin_count_kernel<<<nblocks(pb.nrow), 256, 0, st>>>(pb.uvw, pb.nrow, pb.flag, pb.flag_stride, g, b.hist,
                                                        b.binrank);
-  scan_reduce_kernel<<<(int)nscan, kScanBlock, 0, st>>>(b.hist, nbins, b.bsum);
-  scan_sums_kernel<<<1, 1024, 0, st>>>(b.bsum, (int)nscan);
-  scan_apply_kernel<<<(int)nscan, kScanBlock, 0, st>>>(b.hist, nbins, b.bsum, b.off, (int)cp.nvalid);
+  uint64_t *occ = g.occ ? b.occ : nullptr;
+  if (nbins <= kSmallScan) {
+    scan_small_kernel<<<1, 1024, 0, st>>>(b.hist, (int)nbins, b.off, (int)cp.nvalid, g, occ);
+  } else {
+    scan_reduce_kernel<<<(int)nscan, kScanBlock, 0, st>>>(b.hist, nbins, b.bsum);
+    scan_sums_kernel<<<1, 1024, 0, st>>>(b.bsum, (int)nscan);
+    scan_apply_kernel<<<(int)nscan, kScanBlock, 0, st>>>(b.hist, nbins, b.bsum, b.off, (int)cp.nvalid);
+    if (occ) occ_kernel<<<(g.P + 3) / 4, 256, 0, st>>>(b.off, g, occ);
+  }
   if (pb.nrow > 0) {
     T *taps = g.fft_lds ? (T *)b.taps : nullptr;
     if (tap_width(g.kw) == 8)
@@ -337,10 +383,6 @@ void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
                                                                    (Rec<T> *)b.recs, b.slot, with_value ? 1 : 0,
                                                                    taps);
   }
-}
-
-void launch_occ(const int *off, const Geom &g, uint64_t *occ, hipStream_t st) {
-  occ_kernel<<<(g.P + 3) / 4, 256, 0, st>>>(off, g, occ);
 }
 
 template void enqueue_binning<float>(const Problem &, const ChanPlan &, const Bufs &, hipStream_t, bool);

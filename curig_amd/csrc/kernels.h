@@ -115,7 +115,6 @@ void launch_pack_columns(const Columns &c, double *uvw, int n, hipStream_t st);
 // count, scan and scatter of one problem's rows into bin order (records, and for dirty2ms each row's record)
 template <typename T>
 void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipStream_t st, bool with_value);
-void launch_occ(const int *off, const Geom &g, uint64_t *occ, hipStream_t st);
 void launch_fill_zero_c128(double2 *p, long n, hipStream_t st);
 
 // ---- kern_plane.hip: full-plane path (rocFFT grids), corrections, direct sums

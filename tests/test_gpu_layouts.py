@@ -237,3 +237,16 @@ def test_many_rows_to_a_bin(precision, nx, ny, nrow):
     say(f"[many rows to a bin] {precision} {nx}x{ny} rows {nrow}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
     tol = 1e-11 if precision == "fp64" else 2e-6
     assert e1 < tol and e2 < tol
+
+
+# bin offsets in one workgroup and in three passes: a bin or a few, 1024 of them and
+# more (several to a thread), and about the most that one workgroup scans (4096
+# strips times three to eight layers)
+@pytest.mark.parametrize("nx,ny,wmax", [(8, 64, 5.0), (512, 64, 200.0), (600, 64, 500.0), (4096, 32, 10.0),
+                                        (4096, 32, 60.0), (4096, 32, 150.0), (4096, 32, 300.0)])
+def test_bin_offsets(nx, ny, wmax):
+    fov, eps = 2.0, 1e-6
+    uvw, vis, wgt, img, f0 = _case(5000, nx, ny, fov, wmax, nx + ny)
+    e1, e2 = _both_paths("fp64", uvw, vis, wgt, img, nx, ny, fov, f0, eps)
+    say(f"[bin offsets] {nx}x{ny} wmax {wmax}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")
+    assert e1 < 1e-11 and e2 < 1e-11
