@@ -157,11 +157,12 @@ int curig_gauss_legendre(int n, double *x, double *w);
  * w planes per batch (FFT batch) and w planes per bin layer.  The autotuner
  * (curig_amd.autotune) sets these. */
 int curig_set_tuning(int tile_x, int tile_y, int planes_per_batch, int planes_per_bin);
-/* FFT path of later calls: 0 = pruned LDS FFT where the grid is a power of two
- * and a row fits one workgroup's LDS (else rocFFT), 1 = always rocFFT. */
+/* FFT path of later calls: 0 = pruned LDS FFT where the kernel is at most 16 wide
+ * and rows and columns fit it (powers of two up to 16384, other axes while one
+ * workgroup's LDS holds them; else rocFFT), 1 = always rocFFT. */
 int curig_set_fft_path(int path);
 /* Multi-channel calls: 1 (default) = capture the whole per-channel sequence into
- * one hipGraph and replay it while the same call repeats (power-of-two grids);
+ * one hipGraph and replay it while the same call repeats (LDS FFT path);
  * 0 = queue the per-channel kernels directly. */
 int curig_set_graph_mode(int on);
 /* 1: time the stages of later calls with hipEvents (adds synchronisation;
