@@ -1198,10 +1198,13 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.occ_lg << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64 << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
+      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.occ_lg << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd
+      << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64
+      << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
-  k << b.dev << b.occ << b.tabs << b.hist << b.off << b.bsum << b.slot << b.binrank << b.recs << b.taps << b.grid << b.H << b.acc
+  k << b.dev << b.occ << b.tabs << b.hist << b.off << b.bsum << b.slot << b.binrank << b.recs << b.taps << b.grid
+    << b.H << b.acc
     << b.vacc << b.tw1 << b.tw2 << b.hc_d << b.hc_f;
   return k.h;
 }

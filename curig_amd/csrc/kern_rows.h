@@ -202,7 +202,8 @@ __device__ __forceinline__ void interp_records(const WalkTable &wt, int total, c
 // KWM lanes per record, lane i at tap i of each row of its support: a row's
 // cells are then one or two lines, where a thread per record touched a line per
 // lane and load (11-wide kernel, FP64, 220,000 records on a 250 x 360 grid:
-// 1,490 us in the fused row pass, 1,080 with eight lanes each at rows of their own, 560 so).  The x tap multiplies the lane's sum at the end.
+// 1,490 us in the fused row pass, 1,080 with eight lanes each at rows of their own,
+// 560 so).  The x tap multiplies the lane's sum at the end.
 template <typename T, int KWM>
 __global__ void __launch_bounds__(256) interp_gather_kernel(const Rec<T> *__restrict__ recs,
                                                             const T *__restrict__ taps, const int *__restrict__ off,
