@@ -385,7 +385,7 @@ static void plan_mixed(Geom &g, size_t cs, size_t lds_max) {
   const size_t room = lds_max > 8192 ? lds_max - 8192 : 0;  // walk tables, block table beside the rows
   const int max_threads = cs == 16 ? 512 : 1024;
   auto row_bytes = [&](int rows) {
-    return (size_t)(rows * fftm::seq_stride(g.nf1) + fftc::twiddle_entries(g.nf1)) * cs + (cs == 8 ? rows * (g.nf1 / 16 + 1) * 6 : 0);
+    return (size_t)(rows * fftm::seq_stride(g.nf1) + fftc::twiddle_entries(g.nf1)) * cs;
   };
   auto col_bytes = [&](int cols) { return (size_t)(cols * fftm::seq_stride(g.nf2) + fftc::twiddle_entries(g.nf2)) * cs; };
   if (row_bytes(1) > room || col_bytes(1) > room) return;
@@ -556,7 +556,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     // the one plane of a 20M-point 2-D transform (15,000 visits per row) took 5.7
     // ms in halves against 2.7 (ms2dirty), 6.8 against 3.4 (dirty2ms, equal near
     // 1,000 visits).
-    const bool halves = !dbl && g.nf1 == 8192 && !tn.compact && visits <= 1000;
+    const bool halves = !dbl && g.nf1 == 8192 && !tn.compact && visits <= 1000 && kRowSplit != 2;
     const int split = halves ? 2 : kRowSplit;
     const size_t rbp = (size_t)(fftc::padded_size(g.nf1 / split) + fftc::twiddle_entries(g.nf1)) * cs;
     const bool row_whole = rb + 2048 <= lds_max && rpw * g.nf1 / 16 <= max_threads;
@@ -595,16 +595,16 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     const bool rows = g.mix || (pow2(g.nf1) && !g.rsplit);
     g.gather = tn.to_vis && rows && !tn.compact &&
                nrow_valid * (double)g.kw * g.kww > 0.3 * g.P * (double)g.nf1 * g.nf2;
-    // FP32 rows with many records are summed in FP64 (twice the LDS, no bound
-    // pass): by record visits per row and plane, FP64 against integer sums, 41
-    // (1500 x 1100) 1.27 / 1.08 ms, 615 (1024^2, 33 planes) 0.76 / 0.77, 2,000
-    // (1500^2 modes, 1M points) 0.21 / 0.23, 15,000 (4096^2, 20M) 2.7 / 4.0 ms; up
-    // to 1024 cells, where a row takes little LDS anyway, 190 (256^2 image) 77 /
-    // 138 us.  The integers' bound grows with a block's records, their sum with
-    // the square root: error against 64 bits, thousands of records per block
-    // (uv data within 2.4% of a 512^2 grid), 1.4e-6 in integers, 1.3e-7 in FP64.
-    const bool few_cells = g.nf1 <= 1024;
-    const bool dense = !dbl && !tn.to_vis && rows && visits > (g.nf1 >= 4096 ? 1000 : few_cells ? 100 : 600);
+    // FP32 row sums (FP64 either way, RowAcc): complex cells, twice the LDS of a
+    // row, or one component after the other, reading every record twice.  Complex /
+    // components by record visits per row and plane: up to 1024 cells, where a row
+    // takes little LDS anyway, 65 (256^2 image) 40 / 47 us, 95 (512^2) 95 / 99, 2,600
+    // (256^2) 584 / 887; 2048 cells, 690 (1024^2) 0.71 / 0.66 ms, 1,360 1.19 / 1.16,
+    // 2,770 2.13 / 2.31; mixed radix, 43 (1500 x 1100) 1.27 / 1.11 ms, 173 1.52 /
+    // 1.43, 425 2.01 / 2.13; 4 in rows of 8000 8.3 / 5.7 ms.  Rows of 4096 and 8192
+    // beyond 1,000 run whole in complex cells, fewer in the kernels of kern_lds.h.
+    const double line = g.nf1 <= 1024 ? -1 : g.nf1 >= 4096 ? 1000 : g.mix ? 300 : 1500;
+    const bool dense = !dbl && !tn.to_vis && rows && visits > line;
     if (!g.mix && !g.rsplit && (g.nf1 <= 2048 || g.nf1 == 8192 || g.gather || dense)) {
       g.rowreg = 1;
       // 256 threads, or one row's; fewer while that leaves fewer than 1024

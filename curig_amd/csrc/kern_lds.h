@@ -323,13 +323,13 @@ __device__ __forceinline__ void fft4096_part_to_regs(cpx<T> *buf, cpx<T> *v, int
       const int e = fexp[(tid >> kFixBlkLog2) + r * (256 >> kFixBlkLog2)];
       v[r] = fftc::mk((T)ldexpf((float)x.x, -e), (T)ldexpf((float)x.y, -e));
     }
-  } else {
+  } else if (IN != 3) {  // (3: v holds the inputs, a barrier since they were read)
     const cpx<T> *b = buf + fftc::pad(tid);
 #pragma unroll
     for (int r = 0; r < 16; ++r) v[r] = b[272 * r];
   }
   fftc::dft_small<T, 16>(v, sign);
-  __syncthreads();
+  if (IN != 3) __syncthreads();
   {
     cpx<T> *b = buf + 17 * tid;  // stage 1 outputs: pad(16 j + r) = 17 j + r
 #pragma unroll
@@ -472,7 +472,13 @@ __device__ __forceinline__ int xcd_interleave(int bid, int n, int blk) {
 // of 2^kFixBlkLog2 (e_b from a bound on the block's contributions, so every
 // partial sum stays below 2^30: bound_row_part).  LDS FP32 atomics take about
 // 100 cycles per wave instruction on this GPU, integer ones about as little
-// as stores.
+// as stores.  FP32 halves of rows of 8192 sum in FP64, the real parts of all
+// records and then the imaginary ones in cells of one double (add_share): integers
+// keep 30 bits of a block's bound, which grows with its records (0.5 million
+// visibilities within 4 cells of the centre of an 8192^2 grid: error against 64
+// bits 8e-5, sums in floats 3e-6, in FP64 2.3e-7; 66% occupied 8192^2 grid, 67
+// visits per row and plane, integers 3.96 ms, FP64 4.45 ms per 26 planes; 0.7
+// visits 3.07 and 2.92 ms).
 enum { kAccNative = 0, kAccFix = 2 };
 
 // Bound pass of kAccFix for one record (index idx): adds the record's bound
@@ -569,6 +575,55 @@ __device__ __forceinline__ void spread_row_part(const Rec<T> rc, const Taps<T, K
   }
 }
 
+// A record's contribution to part h of its row and plane (spread_row_part): the
+// value at the cells ix .. ix + kw - 1 is (re, im) x[i] wh[i].
+template <typename T, int KWM> struct PartShare {
+  int ix;
+  T re, im, x[KWM];
+};
+
+// false: the record does not reach the row and plane
+template <typename T, int KWM, typename Tw>
+__device__ __forceinline__ bool part_share(PartShare<T, KWM> &c, const Rec<T> &rc, int idx, const T *__restrict__ taps,
+                                           const Tw &tv, const Geom &g, int p, int row0, int h, int sign) {
+  int k = p - rc.iw;
+  if (k < 0) k += g.P;
+  if (k >= g.kww) return false;
+  int jj = row0 - rc.iy;
+  if (jj < 0) jj += g.nf2;
+  if (jj >= g.kw) return false;
+  const T *tq = taps + (size_t)idx * (3 * KWM);
+  const T a = tq[2 * KWM + k] * tq[KWM + jj];
+  c.ix = rc.ix;
+  c.re = rc.re * a;
+  c.im = rc.im * a;
+  if (h) {
+    const cpx<T> w = tv[(h * rc.ix) & (g.nf1 - 1)];
+    const T ws = (T)sign * w.y, t = c.re * w.x - c.im * ws;
+    c.im = c.re * ws + c.im * w.x;
+    c.re = t;
+  }
+#pragma unroll
+  for (int i = 0; i < KWM; ++i) c.x[i] = tq[i];
+  return true;
+}
+
+// One component of it (IM: the imaginary one) added in FP64 to cells of one double.
+template <bool IM, typename T, int KWM>
+__device__ __forceinline__ void add_share(double *cells, const PartShare<T, KWM> &c, const cpx<T> *wh, const Geom &g, int h,
+                                          int mm) {
+#pragma unroll
+  for (int i = 0; i < KWM; ++i) {
+    if (i < g.kw) {
+      int cx = c.ix + i;
+      if (cx >= g.nf1) cx -= g.nf1;
+      const T re = c.re * c.x[i], im = c.im * c.x[i];
+      T v = IM ? im : re;
+      if (h) v = IM ? re * wh[i].y + im * wh[i].x : re * wh[i].x - im * wh[i].y;
+      atomicAdd(cells + fftc::pad(cx & mm), (double)v);
+    }
+  }
+}
 
 // ms2dirty row pass for rows too long for two workgroups per CU: one workgroup
 // per part h of a row split S ways (the row transform's outputs S k + h, see
@@ -582,18 +637,19 @@ __device__ __forceinline__ void spread_row_part(const Rec<T> rc, const Taps<T, K
 // factors are loaded once (16384^2 grids: 23.8 against 24.3 ms per 32-plane launch for
 // one workgroup per (row, part, plane)).  With S = 1 it runs whole FP32 rows
 // of 4096 (2048^2 images).  FP32 parts of 4096 accumulate the spread in block
-// floating point (kAccFix): int32 LDS atomics instead of float ones, after a
-// bound pass over the plane's records.
+// floating point (kAccFix: int32 LDS atomics instead of float ones, after a
+// bound pass over the plane's records), the halves of rows of 8192 in FP64.
 template <typename T, int E, int KWM, int S>
 __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
     const Rec<T> *__restrict__ recs, const T *__restrict__ taps, const int *__restrict__ off, cpx<T> *__restrict__ H,
     const cpx<T> *__restrict__ tw, Geom g, int p0, int nb) {
+  constexpr bool kWide = sizeof(T) == 4 && S == 2 && kRowSplit != 2;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ WalkTable wt[2];
   __shared__ cpx<T> whs[KWM];
   // kAccFix block table (FP32): the blocks' bounds, and their exponents for
   // the first FFT stage
-  constexpr bool kFixable = sizeof(T) == 4;
+  constexpr bool kFixable = sizeof(T) == 4 && !kWide;
   __shared__ float fixt[kFixable ? kFixBlks : 1];
   __shared__ short fixe[kFixable ? kFixBlks : 1];
   __shared__ int fixnan;                         // a block's bound is not finite
@@ -608,9 +664,9 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
   PlaneWalk pw(g, p0, 0, nb, row0, row0);
   int pn = pw.next();
   if (pn >= nb) return;
-  // FP32 parts of 4096 accumulate in block floating point (kAccFix), not
-  // with LDS float atomics
-  const bool regs = E == 16 && m == 4096, fix = kFixable && regs;
+  // FP32 parts of 4096 accumulate in block floating point (kAccFix) or, in
+  // halves of 8192, in FP64 by component (kWide), not with LDS float atomics
+  const bool regs = kWide || (E == 16 && m == 4096), fix = kFixable && regs;
   const int accm = fix ? kAccFix : kAccNative;
   if (kFixable && j < kFixBlks) fixt[j] = 0.f;
   if (kFixable && j == 0) fixnan = 0;
@@ -647,6 +703,39 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
     const bool more = pn < nb;
     WalkAhead wa;
     if (j < 64 && more) walk_issue(wa, off, g, p0 + pn, row0);
+    cpx<T> v[16];
+    if constexpr (kWide) {
+      double *cells = reinterpret_cast<double *>(smem_raw);
+      PartShare<T, KWM> c0;  // this thread's first record, kept for the second pass
+      const bool on0 = j < total && part_share<T, KWM>(c0, r0, idx0, taps, tv, g, p, row0, h, sign);
+      auto pass = [&](auto im) {
+        if (on0) add_share<im.value>(cells, c0, whs, g, h, m - 1);
+        for (int t = j + nt; t < total; t += nt) {
+          const int ia = walk_record(wt[cur], t);
+          PartShare<T, KWM> c;
+          if (part_share<T, KWM>(c, recs[ia], ia, taps, tv, g, p, row0, h, sign))
+            add_share<im.value>(cells, c, whs, g, h, m - 1);
+        }
+        __syncthreads();
+        int tid = threadIdx.x;
+        __asm__ volatile("" : "+v"(tid));
+        double *own = cells + fftc::pad(tid);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const T x = (T)own[272 * r];
+          own[272 * r] = 0.0;
+          if constexpr (im.value)
+            v[r].y = x;
+          else
+            v[r].x = x;
+        }
+      };
+      if (total > 0) {
+        pass(std::false_type());
+        __syncthreads();
+        pass(std::true_type());
+      }
+    }
     if (fix && total > 0) {
       // block bounds (kAccFix); a plane without records leaves the table zero
       if (j < total) bound_row_part<T, KWM>(r0, idx0, taps, g, p, row0, m - 1, fixt);
@@ -662,12 +751,12 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
         if (e == kFixNaN) fixnan = 1;
       }
     }
-    if (j < total) {
+    if (!kWide && j < total) {
       Taps<T, KWM> q0;
       load_taps<T, KWM>(taps, idx0, q0);
       spread_row_part<T, KWM>(r0, q0, ldsf, tv, whs, g, p, row0, h, m - 1, sign, accm, fixt);
     }
-    for (int t = j + nt; t < total; t += nt) {
+    for (int t = j + nt; !kWide && t < total; t += nt) {
       const int ia = walk_record(wt[cur], t);
       Taps<T, KWM> ta;
       load_taps<T, KWM>(taps, ia, ta);
@@ -692,9 +781,10 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
       // column S (j + 256 r) + h + N1 / 2 (folded by nf1), which can be an
       // image column for r < 4 and r >= 12 only; its slot steps by 64 tiles
       // per r (as in row_ifft_interp_part_kernel's inputs)
-      cpx<T> v[16];
       const bool pnan = fix && fixnan;  // read before the transform's barriers; cleared after them
-      if (fix)
+      if constexpr (kWide)
+        fft4096_part_to_regs<T, 3>(lds, v, sign, pt);
+      else if (fix)
         fft4096_part_to_regs<T, 2>(lds, v, sign, pt, fixe);
       else
         fft4096_part_to_regs<T, 0>(lds, v, sign, pt);

@@ -40,29 +40,64 @@ __device__ __forceinline__ void mix_stages(cpx<T> *buf, const fftm::Plan &P, con
   }
 }
 
-// the first stage on the spread's cells: integers scaled by block (cell k of
-// sequence q in block k >> kFixBlkLog2 of exponent fexp[q * nblk + block]), or
-// FP64 sums whose first half the transform then runs in
-template <typename T, int SIGN, bool ACC64, typename Tw>
-__device__ __forceinline__ void mix_first_cells(cpx<T> *buf, const typename RowAcc<T, ACC64>::cell *acc, const fftm::Plan &P,
-                                                const Tw &tw, const short *fexp, int nblk) {
+// f(element of the register array, offset in the buffer) for this thread's inputs
+// of the first stage, f(butterfly's first element) after each butterfly's
+template <int RR, typename F, typename B>
+__device__ __forceinline__ void mix_first_inputs(const fftm::Plan &P, int tid, F f, B each) {
+  const int nbf = P.n / RR, total = nbf * P.count;
+#pragma unroll
+  for (int b = 0; b < fftm::radix_nb(RR); ++b) {
+    const int jg = tid + b * P.nt;
+    if (jg < total) {
+      const int seq = P.count > 1 ? fftm::quot(jg, P.bf_magic[0]) : 0, j = jg - seq * nbf;
+#pragma unroll
+      for (int r = 0; r < RR; ++r) f(b * RR + r, seq * P.stride + fftc::pad(j + r * nbf));
+      each(b * RR);
+    }
+  }
+}
+
+constexpr int kMixElems = 20;  // inputs of a stage per thread at most
+
+// the real parts of this thread's inputs of the first stage, their cells cleared
+template <typename T> __device__ __forceinline__ void mix_take_real(double *cells, const fftm::Plan &P, T *re) {
+  int tid = threadIdx.x;
+  __asm__ volatile("" : "+v"(tid));
+  fftm::with_radix(P.R[0], [&](auto tag) {
+    constexpr int RR = decltype(tag)::value;
+    mix_first_inputs<RR>(
+        P, tid,
+        [&](int e, int at) {
+          re[e] = (T)cells[at];
+          cells[at] = 0.0;
+        },
+        [](int) {});
+    // ends each radix's case differently: its stores to re, merged with another's, would go to memory
+    __asm__ volatile("; %0" ::"i"(RR));
+  });
+}
+
+// the first stage on the spread's sums, in whose place (complex cells: first half)
+// the transform then runs
+template <typename T, int SIGN, typename Cell>
+__device__ __forceinline__ void mix_first_cells(cpx<T> *buf, const Cell *acc, const T *re, const fftm::Plan &P) {
   int tid = threadIdx.x;
   __asm__ volatile("" : "+v"(tid));
   fftm::with_radix(P.R[0], [&](auto tag) {
     constexpr int RR = decltype(tag)::value;
     cpx<T> v[RR * fftm::radix_nb(RR)];
-    fftm::stage_load<T, RR, SIGN>(
-        [&](int q, int k) {
-          const int at = q * P.stride + fftc::pad(k);
-          if constexpr (RowAcc<T, ACC64>::fix) {
-            const int2 x = reinterpret_cast<const int2 *>(buf)[at];
-            const int e = fexp[q * nblk + (k >> kFixBlkLog2)];
-            return fftc::mk((T)ldexpf((float)x.x, -e), (T)ldexpf((float)x.y, -e));
-          } else {
-            return fftc::mk((T)acc[at].x, (T)acc[at].y);
-          }
+    mix_first_inputs<RR>(
+        P, tid,
+        [&](int e, int at) {
+          if constexpr (std::is_same<Cell, double>::value)
+            v[e] = fftc::mk(re[e], (T)acc[at]);
+          else
+            v[e] = fftc::mk((T)acc[at].x, (T)acc[at].y);
         },
-        v, P, 0, 1, tw, tid);
+        [&](int e) {
+          fftm::dft<T, RR, SIGN>(v + e);
+          __builtin_amdgcn_sched_barrier(0);
+        });
     __syncthreads();
     fftm::stage_store<T, RR>([&](int q, int k, cpx<T> x) { buf[q * P.stride + fftc::pad(k)] = x; }, v, P, 0, 1, tid);
   });
@@ -77,17 +112,14 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
     const Rec<T> *__restrict__ recs, const T *__restrict__ taps, const int *__restrict__ off, cpx<T> *__restrict__ H,
     const cpx<T> *__restrict__ tw, Geom g, fftm::Plan P, int p0, int nb, int pchunk) {
   using Cell = typename RowAcc<T, ACC64>::cell;
-  constexpr bool kFix = RowAcc<T, ACC64>::fix;
+  constexpr bool kParts = RowAcc<T, ACC64>::parts;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ WalkTable wt[2];
-  __shared__ int fixnan;
   const int nf1 = g.nf1, nf2 = g.nf2, N1 = g.N1, nt = blockDim.x, tid = threadIdx.x, rpw = g.rpw;
-  const int nbuf = P.count * P.stride, nblk = fix_row_blocks(nf1), h1 = N1 / 2;
+  const int nbuf = P.count * P.stride, h1 = N1 / 2;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
   Cell *acc = reinterpret_cast<Cell *>(smem_raw);
   cpx<T> *ltw = reinterpret_cast<cpx<T> *>(acc + nbuf);
-  float *fixt = reinterpret_cast<float *>(ltw + fftc::twiddle_entries(nf1));
-  short *fixe = reinterpret_cast<short *>(fixt + rpw * nblk);
   const int row0 = row_group(g) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
@@ -97,11 +129,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
   if (pn >= k1) return;
   const auto tv = lds_twiddles<T>(ltw, tw, nf1);
   if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, nrows);
-  for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{0, 0};
-  if (kFix) {
-    for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
-    if (tid == 0) fixnan = 0;
-  }
+  for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{};
   __syncthreads();
   int cur = 0;
   for (int pl = pn; pl < k1; pl = pn, cur ^= 1) {
@@ -110,12 +138,16 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
     const bool more = pn < k1;
     WalkAhead wa;
     if (tid < 64 && more) walk_issue(wa, off, g, p0 + pn, row0, nrows);
-    if (kFix && total > 0) {
-      bound_records<T, KWM>(wt[cur], total, recs, taps, g, p, row0, nrows, fixt, nblk);
-      __syncthreads();
-      block_exponents(fixt, fixe, nrows * nblk, &fixnan);
+    T re[kParts ? kMixElems : 1];
+    if constexpr (kParts) {
+      if (total > 0) {
+        spread_records<kReal, T, KWM>(wt[cur], total, recs, taps, g, p, row0, nrows, acc, P.stride);
+        __syncthreads();
+        mix_take_real<T>(acc, P, re);
+        __syncthreads();
+      }
     }
-    spread_records<T, KWM, ACC64>(wt[cur], total, recs, taps, g, p, row0, nrows, acc, P.stride, fixt, nblk);
+    spread_records<kParts ? kImag : kBoth, T, KWM>(wt[cur], total, recs, taps, g, p, row0, nrows, acc, P.stride);
     if (tid < 64 && more) walk_finish(wt[cur ^ 1], wa);
     __syncthreads();  // spread done; the next plane's walk table is complete
     cpx<T> *hb = H + h_plane(g, pl) + row0 * kTile;
@@ -126,9 +158,8 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
         for (int i = occ_row(occ, row0 + r, g) ? tid : N1; i < N1; i += nt) hb[h_slot(g, i) + (r << kTileLog2)] = fftc::mk((T)0, (T)0);
       continue;
     }
-    const bool pnan = kFix && fixnan;  // cleared below, after the transform's barriers
-    if (kFix || ACC64) {
-      mix_first_cells<T, +1, ACC64>(buf, acc, P, tv, fixe, nblk);
+    if constexpr (kParts || ACC64) {
+      mix_first_cells<T, +1>(buf, acc, re, P);
       mix_stages<T, +1>(buf, P, tv, 1, P.R[0]);
     } else {
       mix_stages<T, +1>(buf, P, tv, 0, 1);
@@ -136,16 +167,10 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
     for (int r = 0; r < nrows; ++r)
       for (int i = tid; i < N1; i += nt) {
         const int k = i >= h1 ? i - h1 : nf1 + i - h1;
-        cpx<T> x = buf[r * P.stride + fftc::pad(k)];
-        if (pnan) x = fftc::mk((T)NAN, (T)NAN);
-        put_row(hb + h_slot(g, i) + (r << kTileLog2), x, add);
+        put_row(hb + h_slot(g, i) + (r << kTileLog2), buf[r * P.stride + fftc::pad(k)], add);
       }
     __syncthreads();  // every output read: clear for the next plane
-    for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{0, 0};
-    if (kFix) {
-      for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
-      if (tid == 0) fixnan = 0;
-    }
+    for (int i = tid; i < nbuf; i += nt) acc[i] = Cell{};
     __syncthreads();
   }
 }
@@ -382,9 +407,7 @@ __global__ void __launch_bounds__(MT) col_inv_mix_kernel(const cpx<T> *__restric
 // --------------------------------------------------------------------------
 template <typename T> inline int mix_row_lds(const Geom &g, bool spread) {
   const int cells = g.rpw * fftm::seq_stride(g.nf1);
-  int b = cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>)) + fftc::twiddle_entries(g.nf1) * (int)sizeof(cpx<T>);
-  if (sizeof(T) == 4 && spread && !g.acc64) b += g.rpw * fix_row_blocks(g.nf1) * 6 + 2;
-  return b;
+  return cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>)) + fftc::twiddle_entries(g.nf1) * (int)sizeof(cpx<T>);
 }
 template <typename T> inline int mix_col_lds(const Geom &g, int cpw) {
   return (int)sizeof(cpx<T>) * (cpw * fftm::seq_stride(g.nf2) + fftc::twiddle_entries(g.nf2));

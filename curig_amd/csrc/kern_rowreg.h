@@ -2,8 +2,8 @@
 // (4096 and parts of 4096: the plane-loop kernels of kern_lds.h; FP32 rows of
 // 8192 kept whole).  A workgroup holds rpw rows in LDS, N / 16 threads each
 // (RegFft), and walks a chunk of the batch's planes: the stage twiddles are set
-// up once, the spread accumulates in block floating point (FP32) and the first
-// and last stages of the transform stay in registers.
+// up once, the spread accumulates in FP64 (RowAcc) and the first and last stages
+// of the transform stay in registers.
 #pragma once
 #include "fft_reg.h"
 #include "kern_rows.h"
@@ -29,18 +29,15 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
     const Rec<T> *__restrict__ recs, const T *__restrict__ taps, const int *__restrict__ off, cpx<T> *__restrict__ H,
     const cpx<T> *__restrict__ tw, Geom g, int p0, int nb, int pchunk) {
   using F = RegFft<T, N, +1>;
-  constexpr int G = F::G, nblk = N >> kFixBlkLog2;
+  constexpr int G = F::G;
   using Cell = typename RowAcc<T, ACC64>::cell;
-  constexpr bool kFix = RowAcc<T, ACC64>::fix;
+  constexpr bool kParts = RowAcc<T, ACC64>::parts;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ WalkTable wt[2];
-  __shared__ int fixnan;
   const int tid = threadIdx.x, nt = blockDim.x, rpw = g.rpw, s = tid / G, j = tid % G, N1 = g.N1, h1 = N1 / 2;
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw), *own = buf + s * F::kStride;
-  // the cells; in FP32 with FP64 sums the transform runs in their first half
+  // the cells; in FP32 the transform runs in their place (complex cells: in their first half)
   Cell *acc = reinterpret_cast<Cell *>(smem_raw), *ownc = acc + s * F::kStride;
-  float *fixt = reinterpret_cast<float *>(acc + rpw * F::kStride);
-  short *fixe = reinterpret_cast<short *>(fixt + rpw * nblk);
   const int row0 = row_group(g) * rpw;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
@@ -50,11 +47,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
   int pn = pw.next();
   if (pn >= k1) return;
   if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, rpw);
-  for (int i = tid; i < rpw * F::kStride; i += nt) acc[i] = Cell{0, 0};
-  if (kFix) {
-    for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
-    if (tid == 0) fixnan = 0;
-  }
+  for (int i = tid; i < rpw * F::kStride; i += nt) acc[i] = Cell{};
   F fft;
   fft.init(tw, j, nullptr);
   __syncthreads();
@@ -65,34 +58,34 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
     const bool more = pn < k1;
     WalkAhead wa;
     if (tid < 64 && more) walk_issue(wa, off, g, p0 + pn, row0, rpw);
-    if (kFix && total > 0) {
-      bound_records<T, KWM>(wt[cur], total, recs, taps, g, p, row0, rpw, fixt, nblk);
-      __syncthreads();
-      block_exponents(fixt, fixe, rpw * nblk, &fixnan);
+    cpx<T> v[16];
+    if constexpr (kParts) {
+      if (total > 0) {
+        spread_records<kReal, T, KWM>(wt[cur], total, recs, taps, g, p, row0, rpw, acc, F::kStride);
+        __syncthreads();
+        Cell *in = ownc + F::pos0(j);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          v[e].x = (T)in[F::pos(e)];
+          in[F::pos(e)] = 0.0;
+        }
+        __syncthreads();
+      }
     }
-    spread_records<T, KWM, ACC64>(wt[cur], total, recs, taps, g, p, row0, rpw, acc, F::kStride, fixt, nblk);
+    spread_records<kParts ? kImag : kBoth, T, KWM>(wt[cur], total, recs, taps, g, p, row0, rpw, acc, F::kStride);
     if (tid < 64 && more) walk_finish(wt[cur ^ 1], wa);
     __syncthreads();  // spread done; the next plane's walk table is complete
-    cpx<T> v[16];
     if (total > 0) {
-      const bool pnan = kFix && fixnan;  // cleared below, after the transform's barriers
       const Cell *in = ownc + F::pos0(j);
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        if (kFix) {
-          const int2 x = reinterpret_cast<const int2 *>(in)[F::pos(e)];
-          const int b = fixe[s * nblk + ((j + G * e) >> kFixBlkLog2)];
-          v[e] = fftc::mk((T)ldexpf((float)x.x, -b), (T)ldexpf((float)x.y, -b));
-        } else {
+        if constexpr (kParts)
+          v[e].y = (T)in[F::pos(e)];
+        else
           v[e] = fftc::mk((T)in[F::pos(e)].x, (T)in[F::pos(e)].y);
-        }
       }
       __syncthreads();
       fft.template run<false>(v, own, j);
-      if (pnan) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = fftc::mk((T)NAN, (T)NAN);
-      }
     } else {
       // no visibility reaches these rows of this plane (and the LDS is still clear)
 #pragma unroll
@@ -107,11 +100,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
     if (total == 0) continue;
     __syncthreads();  // the transform's LDS reads are done: clear for the next plane
 #pragma unroll
-    for (int e = 0; e < 16; ++e) (ownc + F::pos0(j))[F::pos(e)] = Cell{0, 0};
-    if (kFix) {
-      for (int i = tid; i < rpw * nblk; i += nt) fixt[i] = 0.f;
-      if (tid == 0) fixnan = 0;
-    }
+    for (int e = 0; e < 16; ++e) (ownc + F::pos0(j))[F::pos(e)] = Cell{};
     __syncthreads();
   }
 }
@@ -225,11 +214,15 @@ template <typename T, typename F> inline bool with_row_len(int n, F f) {
   return false;
 }
 
+// whether a plan sums rows of N cells so (ACC64: Geom::acc64): FP32 rows of 2048
+// and 8192 both ways, shorter ones and 4096 in complex cells only
+template <typename T, int N, bool ACC64> constexpr bool row_acc() {
+  return sizeof(T) == 8 ? N != 4096 : ACC64 || N == 2048 || N == 8192;
+}
+
 template <typename T> inline int rowreg_lds(const Geom &g, bool spread) {
   const int cells = g.rpw * (g.nf1 + g.nf1 / 16 + 16);
-  int b = cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>));
-  if (sizeof(T) == 4 && spread && !g.acc64) b += g.rpw * (g.nf1 >> kFixBlkLog2) * 6;
-  return b;
+  return cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>));
 }
 
 template <typename T>
@@ -240,7 +233,7 @@ void rowreg_spread(const Rec<T> *recs, const T *taps, const int *off, const Geom
   if (g.zrow > 1) zero_planes<T>(H, g, nb, st);
   with_row_len<T>(g.nf1, [&](auto N) {
     with_acc64<T>(g.acc64, [&](auto A) {
-      if constexpr (N.value != 4096 || A.value) {
+      if constexpr (row_acc<T, N.value, A.value>()) {
         if (g.kw <= 8)
           spread_row_reg_kernel<T, 8, N.value, A.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb, g.pch_row);
         else
@@ -277,7 +270,7 @@ template <typename T> int allow_rowreg(const Geom &g, bool spread) {
     if (g.rpw < 1 || g.rpw > 64 || (g.rpw & (g.rpw - 1)) || nt < 64 || nt > RowThreads<n>::value || g.nf2 % g.rpw || g.pch_row < 1 || g.zrow < 1) return;
     if (spread) {
       with_acc64<T>(g.acc64, [&](auto A) {
-        if constexpr (n != 4096 || A.value) {
+        if constexpr (row_acc<T, n, A.value>()) {
           ier = allow_lds(spread_row_reg_kernel<T, 8, n, A.value>, lb);
           if (ier == kOk) ier = allow_lds(spread_row_reg_kernel<T, 16, n, A.value>, lb);
         }
