@@ -171,7 +171,8 @@ struct Tuning {
   int lds_bytes = 0;    // LDS per workgroup of the device (0: 160 KiB, gfx950)
   int kereval = 0;      // kernel evaluation: 0 exp(sqrt()), 1 piecewise polynomial (Horner)
   int to_vis = 0;       // 1: the plan of a dirty2ms call
-  int compact = 0;      // 1: layouts with the smallest working set (the no-allocation entry's fixed scratch)
+  int compact = 0;      // 1: the layouts of a path that take the least memory; 2: and no mixed-radix path (where
+                        // memory is short, and in the no-allocation entry's fixed scratch)
   size_t grid_budget_bytes = size_t(48) << 30;
 };
 

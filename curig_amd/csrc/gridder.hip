@@ -103,6 +103,15 @@ int scratch_base(int dev, char **out) {
   return kOk;
 }
 
+// CURIG_WORKSPACE_LIMIT (bytes): device memory the workspace may hold, for
+// processes that share a card; read when a buffer grows.
+bool within_limit(const Workspace &w, size_t more) {
+  const char *s = std::getenv("CURIG_WORKSPACE_LIMIT");
+  if (!s || !*s) return true;
+  for (size_t n : w.n) more += n;
+  return more <= std::strtoull(s, nullptr, 10);
+}
+
 int ws_get(int dev, Slot s, size_t bytes, void **out) {
   if (g_arena) {
     // no-allocation call: consecutive 256-byte aligned pieces of the scratch
@@ -125,7 +134,7 @@ int ws_get(int dev, Slot s, size_t bytes, void **out) {
       w.p[s] = nullptr;
       w.n[s] = 0;
     }
-    hipError_t e = hipMalloc(&w.p[s], bytes);
+    hipError_t e = within_limit(w, bytes) ? hipMalloc(&w.p[s], bytes) : hipErrorOutOfMemory;
     if (e != hipSuccess) {
       (void)hipGetLastError();
       set_error("device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
@@ -135,6 +144,19 @@ int ws_get(int dev, Slot s, size_t bytes, void **out) {
     if (s == S_TW) w.tw_key[0] = w.tw_key[1] = w.tw_key[2] = -1;
   }
   *out = w.p[s];
+  return kOk;
+}
+
+// Frees the buffers, but for keep (hipFree waits for what uses them).
+int ws_drop(int dev, Slot keep) {
+  Workspace &w = g_ws[dev];
+  for (int s = 0; s < S_NSLOT; ++s) {
+    if (s == keep || !w.p[s]) continue;
+    CURIG_HIP(hipFree(w.p[s]));
+    w.p[s] = nullptr;
+    w.n[s] = 0;
+  }
+  w.tw_key[0] = w.tw_key[1] = w.tw_key[2] = -1;
   return kOk;
 }
 
@@ -425,13 +447,14 @@ static int row_plane_chunk(const Geom &g, int nt) {
 }
 
 // Planes per workgroup of the mixed-radix passes (as plan_columns).
-static void plan_mixed_chunks(Geom &g) {
+static void plan_mixed_chunks(Geom &g, bool compact) {
   auto chunk = [&](int groups) {
     const int n = std::min((1024 + groups - 1) / groups, 8);
     return std::max(std::min(2, g.Pb), (g.Pb + n - 1) / n);
   };
   g.pch_row = row_plane_chunk(g, g.nt_row);
   g.pch_fwd = g.pch_inv = chunk((g.N1 + g.cpw - 1) / g.cpw);
+  if (compact) g.pch_fwd = g.Pb;
   g.nacc = (g.Pb + g.pch_fwd - 1) / g.pch_fwd;
 }
 
@@ -583,7 +606,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
       g.tstride = g.nf2 * kTile + (int)(kTilePadBytes / cs);
     }
   }
-  if (!g.fft_lds && tn.fft != 1 && !tn.compact && g.kw <= 16) plan_mixed(g, cs, lds_max);
+  if (!g.fft_lds && tn.fft != 1 && tn.compact < 2 && g.kw <= 16) plan_mixed(g, cs, lds_max);
   if (g.fft_lds) {
     // Dense records: dirty2ms writes the planes' rows out and gathers each
     // record's cells once.  The fused row pass visits a record in every row and
@@ -629,7 +652,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   g.Pb = std::max(1, std::min(Pb, g.P));
   g.nbatch = (g.P + g.Pb - 1) / g.Pb;
   if (g.mix)
-    plan_mixed_chunks(g);
+    plan_mixed_chunks(g, tn.compact != 0);
   else if (g.fft_lds)
     plan_columns(g, cs, lds_max, tn.compact != 0);
   if (g.rowreg) g.pch_row = row_plane_chunk(g, g.rpw * g.nf1 / 16);
@@ -1227,7 +1250,13 @@ int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const T
     packed = pbs[0];
     if (packed.nrow > 0) {
       void *vp;
-      CURIG_TRY(ws_get(dev, S_UVW, sizeof(double) * 3 * (size_t)packed.nrow, &vp));
+      const size_t bytes = sizeof(double) * 3 * (size_t)packed.nrow;
+      int ier = ws_get(dev, S_UVW, bytes, &vp);
+      if (ier == kErrAlloc && !g_arena) {
+        CURIG_TRY(ws_drop(dev, S_NSLOT));
+        ier = ws_get(dev, S_UVW, bytes, &vp);
+      }
+      CURIG_TRY(ier);
       launch_pack_columns(packed.cols, (double *)vp, packed.nrow, st);
       CURIG_HIP(hipGetLastError());
       packed.uvw = (const double *)vp;
@@ -1261,7 +1290,21 @@ int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const T
     }
     CURIG_TRY(ier);
   } else {
-    CURIG_TRY((reserve<T>(cps, pbs, rule, to_image, dev, st, b)));
+    // A plan that does not fit the device's free memory gives way to smaller ones:
+    // without the full planes of the dense dirty2ms gather and the accumulators
+    // per plane chunk (three times the plane memory at 2048^2), then without the
+    // mixed-radix path (its records' taps)
+    int ier = reserve<T>(cps, pbs, rule, to_image, dev, st, b);
+    // (first beside the buffers that earlier calls left, then without them)
+    for (int t = 0; t < 3 && ier == kErrAlloc; ++t) {
+      Tuning tn = tune ? *tune : Tuning();
+      tn.compact = t < 2 ? 1 : 2;
+      if (t > 0) CURIG_TRY(ws_drop(dev, pbs == &packed ? S_UVW : S_NSLOT));
+      CURIG_TRY(plan_all(to_image, pbs, n, st, &tn, dev, cps, rule));
+      b = Bufs();
+      ier = reserve<T>(cps, pbs, rule, to_image, dev, st, b);
+    }
+    CURIG_TRY(ier);
   }
   for (ChanPlan &cp : cps) {
     cp.g.occ = b.occ;
@@ -1386,7 +1429,7 @@ int ms2dirty_device_noalloc(const Problem &pb, hipStream_t st, const Tuning *tun
   ar.cap = kScratchBytes;
   g_arena = &ar;
   Tuning tn = tune ? *tune : Tuning();
-  tn.compact = 1;  // the layouts with the smallest working set
+  tn.compact = 2;  // the layouts with the smallest working set
   const int ier = pb.dbl ? run_locked<double>(true, &pb, 1, st, &tn, 0, nullptr, dev)
                          : run_locked<float>(true, &pb, 1, st, &tn, 0, nullptr, dev);
   g_arena = nullptr;
