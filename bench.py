@@ -194,7 +194,9 @@ def kernel_bytes(plans, nrow, precision, nx, ny):
       gridding (spread + row FFT):    24 R + (s_c + s_w) M + s_c P nf2 N1
       column FFT + w-accumulation:    s_c P nf2 N1 + 16 N (2 B - 1)
       w-fill + inverse column FFT:    s_c N B + s_c P nf2 N1
-      inverse row FFT + interpolation: s_c P nf2 N1 + (32 + 32) M
+      inverse row FFT + interpolation: s_c P nf2 N1 + (32 + 32) M, and
+                                      2 s_c P nf1 nf2 where the rows are formed
+                                      and then gathered from
     (the last: one 32-byte sorted record and one FP64 accumulator read and
     written per visibility).  The tile-spread path (rocFFT planes) writes full
     planes: 24 R + (s_c + s_w) M + s_c P nf1 nf2.
@@ -218,10 +220,39 @@ def kernel_bytes(plans, nrow, precision, nx, ny):
             out["col_fwd"] += plane + 16 * npix * (2 * s["nbatch"] - 1)
             out["col_inv"] += sc * npix * s["nbatch"] + plane
             out["row_interp"] += plane + 64 * M
+            if "gather" in plan_kernels(s, precision)["row_interp"]:
+                out["row_interp"] += 2 * sc * P * s["nf1"] * s["nf2"]
         else:
             out["grid"] += 24 * nrow + (sc + sw) * M + sc * P * s["nf1"] * s["nf2"]
         out["launches"] += s["nbatch"]
     return out
+
+
+def plan_kernels(plan, precision):
+    """Names of the kernels that one plan (plan_info's values and "nvis") runs, by
+    kernel_bytes' keys; two kernels timed together are joined with " + "."""
+    if not plan["fft_lds"]:
+        return {"grid": "spread_tile_kernel"}
+    nf1, nf2, split = plan["nf1"], plan["nf2"], plan["rsplit"] > 0
+    pow2 = not nf1 & (nf1 - 1) and not nf2 & (nf2 - 1) and 2 * plan["ny"] <= nf1 and 2 * plan["nx"] <= nf2
+    whole = "reg" if pow2 else "mix"
+    # the plan's rules: FP32 rows of 4096 leave the plane-loop kernel, and dirty2ms
+    # forms the planes' rows and gathers from them, where records are dense
+    per_plane = plan["nvis"] * plan["kw"] ** 2 / plan["nf3"]
+    dense_rows = precision == "fp32" and per_plane > 1000 * nf2
+    gather = not split and per_plane > 0.3 * nf1 * nf2
+    planes = pow2 and (split or nf1 == 4096)
+    cols = "_mix" if not pow2 else "_reg" if nf2 == 16384 else ""
+    names = {"grid": f"spread_row_{whole}_kernel", "col_fwd": f"col_fwd{cols}_kernel", "col_inv": f"col_inv{cols}_kernel",
+             "row_interp": f"row_interp_{whole}_kernel"}
+    if planes and (split or not dense_rows):
+        names["grid"] = "spread_row_part_planes_kernel"
+    if gather:
+        names["row_interp"] = f"row_planes_{whole}_kernel + interp_gather_kernel"
+    elif planes:
+        loop = nf1 // max(plan["rsplit"], 1) == 4096
+        names["row_interp"] = "row_ifft_interp_part_planes_kernel" if loop else "row_ifft_interp_part_kernel"
+    return names
 
 
 def timed_steps(run, steps, warmup, stats=True):
@@ -780,31 +811,16 @@ def main():
     for ch in range(run.nchan):
         stats_by_ch.append(dict(_lib.plan_info(cfg["vis"].shape[0], cfg["nx"], cfg["ny"], cfg["fov"],
                                                float(cfg["freqs"][ch]), cfg["eps"], 2.0, -1, float(w.min()),
-                                               float(w.max()), run.prec), nvis=cfg["vis"].shape[0]))
+                                               float(w.max()), run.prec), nvis=cfg["vis"].shape[0],
+                                nx=cfg["nx"], ny=cfg["ny"]))
     kb = kernel_bytes(stats_by_ch, cfg["vis"].shape[0], args.precision, cfg["nx"], cfg["ny"])
     launches = kb["launches"]
     mean = lambda key, d: sum(c[key] for c in calls[d]) / len(calls[d]) * 1e-3
-    lds = bool(stats_by_ch[0]["fft_lds"])
-    split = stats_by_ch[0]["rsplit"] > 0  # rows split over several workgroups
-    part = "_part" if split else ""
-    # rows of 4096 run the plane-loop row kernel whole (one part)
-    planes = split or stats_by_ch[0]["nf1"] == 4096
-    pow2 = all(stats_by_ch[0][k] & (stats_by_ch[0][k] - 1) == 0 for k in ("nf1", "nf2"))
-    whole = "reg" if pow2 else "mix"  # whole rows of other lengths
-    spread = ("spread_row_part_planes_kernel" if planes and pow2 else f"spread_row_{whole}_kernel") if lds else "spread_tile_kernel"
-    kernels = {spread: (kb["grid"], mean("t_grid", "m2d"))}
-    if lds:
-        # columns of 16384 run the register-resident column kernels
-        reg = "_reg" if stats_by_ch[0]["nf2"] == 16384 else ""
-        kernels[f"col_fwd{reg}_kernel"] = (kb["col_fwd"], mean("t_fft", "m2d"))
-        kernels[f"col_inv{reg}_kernel"] = (kb["col_inv"], mean("t_fft", "d2m"))
-        # rows and row parts of 4096 run the plane-loop interpolation kernel
-        nf1 = stats_by_ch[0]["nf1"]
-        rs = stats_by_ch[0]["rsplit"]
-        ipl = nf1 // max(rs, 1) == 4096
-        interp = f"row_ifft_interp{part}_kernel" if split else f"row_interp_{whole}_kernel"
-        kernels["row_ifft_interp_part_planes_kernel" if ipl and pow2 else interp] = (
-            kb["row_interp"], mean("t_grid", "d2m"))
+    names = plan_kernels(stats_by_ch[0], args.precision)
+    spread = names["grid"]
+    times = {"grid": ("t_grid", "m2d"), "col_fwd": ("t_fft", "m2d"), "col_inv": ("t_fft", "d2m"),
+             "row_interp": ("t_grid", "d2m")}
+    kernels = {name: (kb[k], mean(*times[k])) for k, name in names.items()}
     per_kernel = {k: {"bytes_per_launch": round(b / launches), "avg_launch_ms": round(t / launches * 1e3, 3),
                       "achieved_GBps": round(b / t / 1e9, 1), "frac": round(b / t / 1e9 / HBM_PEAK_GBS, 4)}
                   for k, (b, t) in kernels.items() if t > 0}
@@ -815,7 +831,7 @@ def main():
     kname = spread
     B, t_dom = kb["grid_full"], kernels[kname][1]
     achieved = B / t_dom / 1e9
-    interp = next((k for k in kernels if k.startswith("row_ifft_interp")), None)
+    interp = names.get("row_interp")
     mirror = None
     if interp and kernels[interp][1] > 0:
         a_i = kb["grid_full"] / kernels[interp][1] / 1e9
