@@ -114,6 +114,9 @@ struct Geom {
   int fft_lds;
   const uint64_t *occ; // [P] planes' occupied row blocks: bit b for rows b << occ_lg .. (null: all taken as
   int occ_lg;          // occupied); rows of the other blocks are neither written to nor read from H
+  int fix;             // ms2dirty: rows or row parts summed in integers (kAccFix, kern_lds.h)
+  const uint64_t *crowd;  // [P] fix: the row blocks whose cells too many records share (kFixRecords; null: none told
+  const uint64_t *plain;  // apart), and the other ones of occ
   int mix;            // LDS path on axes 2^a 3^b 5^c (mixed-radix kernels), else powers of two
   int rowreg;         // whole power-of-two rows in the kernels of kern_rowreg.h
   int acc64;          // ms2dirty, FP32, dense records: rows summed in FP64 (rowreg and mix)

@@ -153,7 +153,9 @@ __device__ __forceinline__ bool occ_full(uint64_t mask, const Geom &g) {
 // The planes k of [k0, k1) of a batch that starts at plane p0 in which the block
 // of row ra or of row rb is occupied, in order (Geom::occ, 64 planes at a time;
 // every lane of a wavefront takes part, and every wavefront finds the same).
-struct PlaneWalk {
+// CROWD: of those blocks, the ones of Geom::plain (kNotCrowded) or Geom::crowd (kCrowded).
+enum { kAllBlocks = 0, kNotCrowded = 1, kCrowded = 2 };
+template <int CROWD = kAllBlocks> struct PlaneWalk {
   const Geom &g;
   int p0, k1, ra, rb, base;
   uint64_t m = 0;
@@ -167,7 +169,8 @@ struct PlaneWalk {
       const int k = base + (threadIdx.x & 63);
       bool on = false;
       if (k < k1) {
-        const uint64_t o = occ_mask(g, p0 + k);
+        const uint64_t *mask = CROWD == kCrowded ? g.crowd : CROWD == kNotCrowded ? g.plain : g.occ;
+        const uint64_t o = mask ? mask[p0 + k] : ~uint64_t(0);
         on = occ_row(o, ra, g) || occ_row(o, rb, g);
       }
       m = __ballot(on);

@@ -556,7 +556,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
   g.rpw = g.cpw = g.nct = g.tstride = g.nslot = g.slot_lg = g.lds_row_bytes = g.lds_col_bytes = g.rsplit =
       g.lds_rowp_bytes = g.colreg = g.cpw_inv = g.pch_fwd = g.pch_inv = 0;
   g.nacc = 1;
-  g.mix = g.nt_row = g.nt_col = g.pch_row = g.gather = g.rowreg = g.acc64 = 0;
+  g.mix = g.nt_row = g.nt_col = g.pch_row = g.gather = g.rowreg = g.acc64 = g.fix = 0;
   g.zrow = 1;
   auto pow2 = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
   // record visits per grid row and plane
@@ -640,6 +640,7 @@ int plan_geometry(int nrow_valid, int nx, int ny, double fov, double freq, doubl
     }
     if (dense && (size_t)g.rpw * (g.nf1 + g.nf1 / 16 + 16) * 16 + 8192 <= lds_max) g.acc64 = 1;
   }
+  g.fix = !dbl && !tn.to_vis && g.fft_lds && !g.mix && !g.rowreg && g.rsplit != 2 && g.nf1 / std::max(g.rsplit, 1) == 4096;
   // planes per batch from the memory budget: full planes (rocFFT path) or, on
   // the LDS path, the compact plane plus the one or two column-pass buffers
   size_t per_plane = (size_t)g.nf1 * g.nf2 * cs;
@@ -986,13 +987,15 @@ int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule
     launch_corr_tables(rule, g0.nf1, g0.nf2, b.tabs, st);
     CURIG_HIP(hipGetLastError());
   }
-  b.occ = nullptr;
+  b.occ = b.crowd = nullptr;
   if (g0.fft_lds) {
     // (last: a full scratch goes without)
-    if (ws_get(dev, S_OCC, sizeof(uint64_t) * nplane, &vp) == kOk)
+    if (ws_get(dev, S_OCC, sizeof(uint64_t) * 3 * nplane, &vp) == kOk) {
       b.occ = (uint64_t *)vp;
-    else if (!g_arena)
+      b.crowd = b.occ + nplane;
+    } else if (!g_arena) {
       return kErrAlloc;
+    }
   }
   b.dev = dev;
   return kOk;
@@ -1221,12 +1224,12 @@ uint64_t graph_key(bool to_image, const Problem *pbs, int n, const std::vector<C
     k << cp.nvalid << g.N1 << g.N2 << g.nf1 << g.nf2 << g.P << g.kw << g.kww << g.hdeg << g.hcoef_d << g.hcoef_f
       << g.beta << g.c << g.dx << g.dy << g.divn << g.zout << g.C << g.D << g.gamma << g.h << g.uscale << g.vscale
       << g.wscale << g.T1 << g.T2 << g.ntx << g.nty << g.ntiles << g.Pb << g.nbatch << g.Pbin << g.nlayer
-      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.occ_lg << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd
+      << g.nquad << g.ncheb << g.zcheb << g.fft_lds << g.occ_lg << g.fix << g.rpw << g.cpw << g.cpw_inv << g.pch_fwd
       << g.pch_inv << g.nacc << g.mix << g.nt_row << g.nt_col << g.pch_row << g.gather << g.rowreg << g.acc64
       << g.zrow << g.nct << g.tstride << g.nslot << g.slot_lg << g.lds_row_bytes
       << g.lds_col_bytes << g.rsplit << g.lds_rowp_bytes << g.colreg;
   }
-  k << b.dev << b.occ << b.tabs << b.hist << b.off << b.bsum << b.slot << b.binrank << b.recs << b.taps << b.grid
+  k << b.dev << b.occ << b.crowd << b.tabs << b.hist << b.off << b.bsum << b.slot << b.binrank << b.recs << b.taps << b.grid
     << b.H << b.acc
     << b.vacc << b.tw1 << b.tw2 << b.hc_d << b.hc_f;
   return k.h;
@@ -1308,6 +1311,9 @@ int run_locked(bool to_image, const Problem *pbs, int n, hipStream_t st, const T
   }
   for (ChanPlan &cp : cps) {
     cp.g.occ = b.occ;
+    const bool crowd = cp.g.fix && cp.nvalid > kFixRecords && b.crowd;
+    cp.g.crowd = crowd ? b.crowd : nullptr;
+    cp.g.plain = crowd ? b.crowd + cp.g.P : b.occ;
     cp.g.hcoef_d = b.hc_d;
     cp.g.hcoef_f = b.hc_f;
   }

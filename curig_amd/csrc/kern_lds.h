@@ -472,13 +472,14 @@ __device__ __forceinline__ int xcd_interleave(int bid, int n, int blk) {
 // of 2^kFixBlkLog2 (e_b from a bound on the block's contributions, so every
 // partial sum stays below 2^30: bound_row_part).  LDS FP32 atomics take about
 // 100 cycles per wave instruction on this GPU, integer ones about as little
-// as stores.  FP32 halves of rows of 8192 sum in FP64, the real parts of all
-// records and then the imaginary ones in cells of one double (add_share): integers
-// keep 30 bits of a block's bound, which grows with its records (0.5 million
-// visibilities within 4 cells of the centre of an 8192^2 grid: error against 64
-// bits 8e-5, sums in floats 3e-6, in FP64 2.3e-7; 66% occupied 8192^2 grid, 67
-// visits per row and plane, integers 3.96 ms, FP64 4.45 ms per 26 planes; 0.7
-// visits 3.07 and 2.92 ms).
+// as stores.  FP32 halves of rows of 8192, and of the others the rows that many
+// records share (Geom::crowd), sum in FP64: the real parts of all records and then
+// the imaginary ones in cells of one double (add_share).  Integers keep 30 bits of a
+// block's bound, which grows with its records: 0.5 million visibilities within 4
+// cells of the centre of an 8192^2 grid, error against 64 bits 8e-5, sums in floats
+// 3e-6, in FP64 2.3e-7; halves, 67 visits per row and plane, integers 3.96 ms, FP64
+// 4.45 ms per 26 planes; 0.7 visits 3.07 and 2.92 ms; quarters of 16384 (58
+// visits) 18.5 and 22 ms, so they keep the integers where they hold.
 enum { kAccNative = 0, kAccFix = 2 };
 
 // Bound pass of kAccFix for one record (index idx): adds the record's bound
@@ -638,18 +639,17 @@ __device__ __forceinline__ void add_share(double *cells, const PartShare<T, KWM>
 // one workgroup per (row, part, plane)).  With S = 1 it runs whole FP32 rows
 // of 4096 (2048^2 images).  FP32 parts of 4096 accumulate the spread in block
 // floating point (kAccFix: int32 LDS atomics instead of float ones, after a
-// bound pass over the plane's records), the halves of rows of 8192 in FP64.
-template <typename T, int E, int KWM, int S>
+// bound pass over the plane's records), or in FP64 (WIDE).
+template <typename T, int E, int KWM, int S, bool WIDE>
 __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
     const Rec<T> *__restrict__ recs, const T *__restrict__ taps, const int *__restrict__ off, cpx<T> *__restrict__ H,
     const cpx<T> *__restrict__ tw, Geom g, int p0, int nb) {
-  constexpr bool kWide = sizeof(T) == 4 && S == 2 && kRowSplit != 2;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ WalkTable wt[2];
   __shared__ cpx<T> whs[KWM];
   // kAccFix block table (FP32): the blocks' bounds, and their exponents for
   // the first FFT stage
-  constexpr bool kFixable = sizeof(T) == 4 && !kWide;
+  constexpr bool kFixable = sizeof(T) == 4 && !WIDE;
   __shared__ float fixt[kFixable ? kFixBlks : 1];
   __shared__ short fixe[kFixable ? kFixBlks : 1];
   __shared__ int fixnan;                         // a block's bound is not finite
@@ -661,12 +661,14 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
   const int item = xcd_interleave(blockIdx.x, gridDim.x, 4 * S);
   const int row0 = item / S, h = item % S;
   // planes whose block of rows holds no record are passed over
-  PlaneWalk pw(g, p0, 0, nb, row0, row0);
+  // (rows of halves in FP64 have one kernel, the others are divided: with_spread_parts)
+  constexpr int kBlocks = S == 2 ? kAllBlocks : WIDE ? kCrowded : kNotCrowded;
+  PlaneWalk<kBlocks> pw(g, p0, 0, nb, row0, row0);
   int pn = pw.next();
   if (pn >= nb) return;
-  // FP32 parts of 4096 accumulate in block floating point (kAccFix) or, in
-  // halves of 8192, in FP64 by component (kWide), not with LDS float atomics
-  const bool regs = kWide || (E == 16 && m == 4096), fix = kFixable && regs;
+  // FP32 parts of 4096 accumulate in block floating point (kAccFix) or in FP64
+  // by component (WIDE), not with LDS float atomics
+  const bool regs = WIDE || (E == 16 && m == 4096), fix = kFixable && regs;
   const int accm = fix ? kAccFix : kAccNative;
   if (kFixable && j < kFixBlks) fixt[j] = 0.f;
   if (kFixable && j == 0) fixnan = 0;
@@ -704,7 +706,7 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
     WalkAhead wa;
     if (j < 64 && more) walk_issue(wa, off, g, p0 + pn, row0);
     cpx<T> v[16];
-    if constexpr (kWide) {
+    if constexpr (WIDE) {
       double *cells = reinterpret_cast<double *>(smem_raw);
       PartShare<T, KWM> c0;  // this thread's first record, kept for the second pass
       const bool on0 = j < total && part_share<T, KWM>(c0, r0, idx0, taps, tv, g, p, row0, h, sign);
@@ -751,12 +753,12 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
         if (e == kFixNaN) fixnan = 1;
       }
     }
-    if (!kWide && j < total) {
+    if (!WIDE && j < total) {
       Taps<T, KWM> q0;
       load_taps<T, KWM>(taps, idx0, q0);
       spread_row_part<T, KWM>(r0, q0, ldsf, tv, whs, g, p, row0, h, m - 1, sign, accm, fixt);
     }
-    for (int t = j + nt; !kWide && t < total; t += nt) {
+    for (int t = j + nt; !WIDE && t < total; t += nt) {
       const int ia = walk_record(wt[cur], t);
       Taps<T, KWM> ta;
       load_taps<T, KWM>(taps, ia, ta);
@@ -782,7 +784,7 @@ __global__ void __launch_bounds__(256) spread_row_part_planes_kernel(
       // image column for r < 4 and r >= 12 only; its slot steps by 64 tiles
       // per r (as in row_ifft_interp_part_kernel's inputs)
       const bool pnan = fix && fixnan;  // read before the transform's barriers; cleared after them
-      if constexpr (kWide)
+      if constexpr (WIDE)
         fft4096_part_to_regs<T, 3>(lds, v, sign, pt);
       else if (fix)
         fft4096_part_to_regs<T, 2>(lds, v, sign, pt, fixe);
@@ -963,7 +965,7 @@ __global__ void __launch_bounds__(256) row_ifft_interp_part_planes_kernel(
   const int nf1 = g.nf1, N1 = g.N1, nt = blockDim.x, j = threadIdx.x;
   const int item = xcd_interleave(blockIdx.x, gridDim.x, 4 * S);
   const int row0 = item / S, h = item % S;
-  PlaneWalk pw(g, p0, 0, nb, row0, row0);
+  PlaneWalk<> pw(g, p0, 0, nb, row0, row0);
   int pn = pw.next();
   if (pn >= nb) return;
   const auto tv = lds_twiddles<T>(lds + fftc::padded_size(m), tw, nf1);
@@ -1363,49 +1365,49 @@ template <typename T, typename F> inline void with_split(int S, F f) {
   f(std::integral_constant<int, kRowSplit>());
 }
 
+// f(integral_constant<int, S>, bool_constant<WIDE>) for the spread kernels that a
+// plan launches: rows of 4096 whole, split rows; in FP32 the crowded row blocks of
+// the integer sums beside the others (Geom::crowd), and halves of 8192 in FP64 only
+template <typename T, typename F> inline void with_spread_parts(const Geom &g, bool crowd, F f) {
+  using std::integral_constant;
+  auto go = [&](auto S) {
+    if constexpr (sizeof(T) == 4 && S.value == 2 && kRowSplit != 2) {
+      f(S, std::true_type());
+    } else {
+      f(S, std::false_type());
+      if constexpr (sizeof(T) == 4) {
+        if (crowd) f(S, std::true_type());
+      }
+    }
+  };
+  if (whole_row_planes<T>(g))
+    go(integral_constant<int, 1>());
+  else if (g.rsplit > 1)
+    with_split<T>(g.rsplit, go);
+}
+
 // ms2dirty, one batch on the LDS path: spread + row FFT -> H (column-tiled)
 template <typename T>
 void lds_spread_rows(const Rec<T> *recs, const T *taps, const int *off, const Geom &g, int p0, int nb, cpx<T> *H,
                      const cpx<T> *tw1, hipStream_t st) {
-  if (g.rsplit > 1) {
-    const int nt = g.nf1 / (16 * g.rsplit), grd = g.rsplit * g.nf2;
-    const int lb = g.lds_rowp_bytes;
-    with_split<T>(g.rsplit, [&](auto S) {
-      if (g.kw <= 8)
-        spread_row_part_planes_kernel<T, 16, 8, S.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
-      else
-        spread_row_part_planes_kernel<T, 16, 16, S.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
-    });
-    return;
-  }
-  if (whole_row_planes<T>(g)) {
-    // rows of 4096: one workgroup per row walks the batch's planes
-    const int lb = g.lds_row_bytes;
+  with_spread_parts<T>(g, g.crowd != nullptr, [&](auto S, auto W) {
+    const int grd = S.value * g.nf2, nt = g.nf1 / (16 * S.value), lb = g.rsplit > 1 ? g.lds_rowp_bytes : g.lds_row_bytes;
     if (g.kw <= 8)
-      spread_row_part_planes_kernel<T, 16, 8, 1><<<g.nf2, 256, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
+      spread_row_part_planes_kernel<T, 16, 8, S.value, W.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
     else
-      spread_row_part_planes_kernel<T, 16, 16, 1><<<g.nf2, 256, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
-    return;
-  }
+      spread_row_part_planes_kernel<T, 16, 16, S.value, W.value><<<grd, nt, lb, st>>>(recs, taps, off, H, tw1, g, p0, nb);
+  });
 }
 
 template <typename T>
 int allow_spread_rows(const Geom &g) {
-  if (whole_row_planes<T>(g)) {
-    const int lb = g.lds_row_bytes;
-    CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 8, 1>, lb)));
-    CURIG_TRY((allow_lds(spread_row_part_planes_kernel<T, 16, 16, 1>, lb)));
-  }
-  if (g.rsplit > 1) {
-    const int lb = g.lds_rowp_bytes;
-    int ier = kOk;
-    with_split<T>(g.rsplit, [&](auto S) {
-      ier = allow_lds(spread_row_part_planes_kernel<T, 16, 8, S.value>, lb);
-      if (ier == kOk) ier = allow_lds(spread_row_part_planes_kernel<T, 16, 16, S.value>, lb);
-    });
-    CURIG_TRY(ier);
-  }
-  return kOk;
+  const int lb = g.rsplit > 1 ? g.lds_rowp_bytes : g.lds_row_bytes;
+  int ier = kOk;
+  with_spread_parts<T>(g, g.fix != 0, [&](auto S, auto W) {
+    if (ier == kOk) ier = allow_lds(spread_row_part_planes_kernel<T, 16, 8, S.value, W.value>, lb);
+    if (ier == kOk) ier = allow_lds(spread_row_part_planes_kernel<T, 16, 16, S.value, W.value>, lb);
+  });
+  return ier;
 }
 
 // rows (rsplit 0) or row parts (rsplit kRowSplit) of 4096 points (FP64:

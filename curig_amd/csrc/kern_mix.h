@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) spread_row_mix_kernel(
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const bool add = gridDim.z > 1;
   // planes whose blocks of rows (two at most, rpw <= 64) hold no record are passed over
-  PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
+  PlaneWalk<> pw(g, p0, k0, k1, row0, row0 + nrows - 1);
   int pn = pw.next();
   if (pn >= k1) return;
   const auto tv = lds_twiddles<T>(ltw, tw, nf1);
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_interp_mix_kernel(
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw);
   const int row0 = row_group(g) * rpw, nrows = min(rpw, nf2 - row0);
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
-  PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
+  PlaneWalk<> pw(g, p0, k0, k1, row0, row0 + nrows - 1);
   int pn = pw.next();
   if (pn >= k1) return;
   const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(MixThreads<T>::value) row_planes_mix_kernel(co
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
   const auto tv = lds_twiddles<T>(buf + P.count * P.stride, tw, nf1);
   for (int i = tid; i < P.count * P.stride; i += nt) buf[i] = fftc::mk((T)0, (T)0);
-  PlaneWalk pw(g, p0, k0, k1, row0, row0 + nrows - 1);
+  PlaneWalk<> pw(g, p0, k0, k1, row0, row0 + nrows - 1);
   for (int pl = pw.next(); pl < k1; pl = pw.next()) {
     __syncthreads();  // the previous plane's rows are written
     mix_load_rows<T>(buf, H + h_plane(g, pl), g, P, row0, nrows, N1);

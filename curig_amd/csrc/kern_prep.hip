@@ -329,6 +329,65 @@ __global__ void __launch_bounds__(256) bin_scatter_kernel(const double *__restri
   }
 }
 
+// Whether the block of rows blockIdx.y of plane blockIdx.x is crowded (Geom::crowd; the
+// others that occ has are Geom::plain's): more than kFixRecords records reach a row
+// of it in one block of 16 cells (of a row part: m cells).  A sample of the records
+// that reach the block's rows is counted by cell block and by groups of eight first
+// rows; a row's records lie in two neighbouring groups, three for kernels beyond 8.
+constexpr int kCrowdSample = 1024, kCrowdGroups = (256 + 15 + 7) / 8;
+__global__ void __launch_bounds__(256) crowd_kernel(const int *__restrict__ off, const Rec<float> *__restrict__ recs,
+                                                    Geom g, int m, const uint64_t *__restrict__ occ,
+                                                    uint64_t *__restrict__ crowd, uint64_t *__restrict__ plain) {
+  __shared__ int hist[kCrowdGroups][256];
+  const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
+  if (!(occ[p] >> b & 1)) return;
+  const int r0 = b << g.occ_lg, rows = min(g.nf2 - r0, 1 << g.occ_lg), s1 = (r0 + rows - 1) / g.T2;
+  // the runs of records in bins of strips [a, s1], [w, nty - 1], planes [pl, p], [wp, P - 1] (occ_plane)
+  const int lo = r0 - g.kw + 1, a = max(lo, 0) / g.T2, w = lo < 0 ? max(lo + g.nf2, 0) / g.T2 : g.nty;
+  const int pl = p - g.kww + 1, wp = pl < 0 ? max(pl + g.P, 0) : g.P;
+  auto runs = [&](auto f) {
+    auto layer = [&](int l) {
+      const int *o = off + l * g.ntiles;
+      f(o[a], o[s1 + 1]);
+      if (w < g.nty) f(o[w], o[g.nty]);
+    };
+    for (int l = max(pl, 0) / g.Pbin; l <= p / g.Pbin; ++l) layer(l);
+    if (wp < g.P)
+      for (int l = wp / g.Pbin; l <= (g.P - 1) / g.Pbin; ++l) layer(l);
+  };
+  long n = 0;
+  runs([&](int i0, int i1) { n += i1 - i0; });
+  bool full = false;
+  if (n > kFixRecords) {
+    const int groups = (rows + g.kw + 6) >> 3, step = (int)((n + kCrowdSample - 1) / kCrowdSample);
+    for (int i = 0; i < groups; ++i) hist[i][tid] = 0;
+    __syncthreads();
+    long at = 0;  // records before the run: every step-th of all runs is taken
+    runs([&](int i0, int i1) {
+      for (long i = (at + step - 1) / step + tid; i * step < at + i1 - i0; i += blockDim.x) {
+        const Rec<float> &rc = recs[i0 + (i * step - at)];
+        const int dy = imod(rc.iy - lo, g.nf2), dz = imod(p - rc.iw, g.P), ix = rc.ix;
+        if (dy >= rows + g.kw - 1 || dz >= g.kww) continue;
+        const int c0 = (ix & (m - 1)) >> 4, c1 = ((ix + g.kw - 1) & (m - 1)) >> 4;
+        atomicAdd(&hist[dy >> 3][c0], 1);
+        if (c1 != c0) atomicAdd(&hist[dy >> 3][c1], 1);
+      }
+      at += i1 - i0;
+    });
+    __syncthreads();
+    const long most = kFixRecords / step;
+    int x = 0, y = 0;
+    for (int i = 0; i < groups; ++i) {
+      const int z = hist[i][tid];
+      full = full || (g.kw > 8 ? x : 0) + y + z > most;
+      x = y;
+      y = z;
+    }
+  }
+  full = __syncthreads_or(full);
+  if (tid == 0) atomicOr((unsigned long long *)(full ? crowd : plain) + p, 1ull << b);
+}
+
 // --------------------------------------------------------------------------
 // launchers
 // --------------------------------------------------------------------------
@@ -382,6 +441,12 @@ void enqueue_binning(const Problem &pb, const ChanPlan &cp, const Bufs &b, hipSt
                                                                    pb.wgt_stride, g, b.binrank, b.off,
                                                                    (Rec<T> *)b.recs, b.slot, with_value ? 1 : 0,
                                                                    taps);
+  }
+  if (sizeof(T) == 4 && g.crowd) {
+    fill_int_kernel<<<nblocks(4 * g.P), 256, 0, st>>>((int *)b.crowd, 4L * g.P, 0);  // and plain behind it
+    const dim3 grd(g.P, ((g.nf2 - 1) >> g.occ_lg) + 1);
+    crowd_kernel<<<grd, 256, 0, st>>>(b.off, (const Rec<float> *)b.recs, g, g.nf1 / std::max(g.rsplit, 1), occ, b.crowd,
+                                      b.crowd + g.P);
   }
 }
 

@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) spread_row_reg_kernel(
   const bool add = gridDim.z > 1;
   // planes whose block of rows holds no record are passed over (rpw, a power of
   // two of at most 64, keeps to a block)
-  PlaneWalk pw(g, p0, k0, k1, row0, row0);
+  PlaneWalk<> pw(g, p0, k0, k1, row0, row0);
   int pn = pw.next();
   if (pn >= k1) return;
   if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, rpw);
@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) row_interp_reg_kernel(
   cpx<T> *buf = reinterpret_cast<cpx<T> *>(smem_raw), *own = buf + s * F::kStride;
   const int row0 = row_group(g) * rpw;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
-  PlaneWalk pw(g, p0, k0, k1, row0, row0);
+  PlaneWalk<> pw(g, p0, k0, k1, row0, row0);
   int pn = pw.next();
   if (pn >= k1) return;
   if (tid < 64) walk_table_build(wt[0], off, g, p0 + pn, row0, rpw);
@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(RowThreads<N>::value) row_planes_reg_kernel(co
   cpx<T> *own = reinterpret_cast<cpx<T> *>(smem_raw) + s * F::kStride;
   const int row = row_group(g) * rpw + s;
   const int k0 = blockIdx.y * pchunk, k1 = min(nb, k0 + pchunk);
-  PlaneWalk pw(g, p0, k0, k1, row & ~(rpw - 1), row & ~(rpw - 1));
+  PlaneWalk<> pw(g, p0, k0, k1, row & ~(rpw - 1), row & ~(rpw - 1));
   F fft;
   fft.init(tw, j, nullptr);
   for (int pl = pw.next(); pl < k1; pl = pw.next()) {

@@ -52,7 +52,8 @@ struct Bufs {
   void *recs = nullptr, *grid = nullptr, *H = nullptr;
   void *taps = nullptr;  // LDS path: each record's kernel taps, [nrec][3][tap_width] of the precision
   double2 *acc = nullptr, *vacc = nullptr;
-  uint64_t *occ = nullptr;  // LDS path: Geom::occ of the running problem
+  // LDS path: Geom::occ, and Geom::crowd with Geom::plain behind it, of the running problem
+  uint64_t *occ = nullptr, *crowd = nullptr;
   const void *tw1 = nullptr, *tw2 = nullptr;
   const double *hc_d = nullptr;  // piecewise-polynomial kernel coefficients, FP64 | FP32
   const float *hc_f = nullptr;
@@ -78,6 +79,17 @@ inline int nblocks(long n, int bs = 256, long cap = 1 << 20) {
 
 // Bins a row workgroup of the LDS path walks at most (the plan coarsens bins to stay within it).
 constexpr int kMaxWalk = 128;
+// Records of a row and plane in one block of 16 cells up to which FP32 rows and row
+// parts of 4096 sum integers scaled by the block's bound; blocks of rows beyond it
+// (Geom::crowd) run in FP64.  The integers' error grows with the records, to 1e-9 of the
+// image for each: 1.3 million rows of noise within 4 cells of the centre of a 4096^2
+// grid, 2.5e-4 from the FP64 image in integers, 2.8e-7 so; within 200 cells, below the
+// line, 5.3e-7.  The FP64 rows take a sixth longer where they are sparse, less where the
+// integers' atomics collide: a 100 m array on 8192^2 pixels 21.2 ms per 32 planes
+// either way, 300 m 13.0 and 15.7 ms (2.4e-7 and 2.0e-7 from FP64), 500 m and more all
+// integers.  Telling the blocks apart: 2048^2 image 24 us and 5 us per 32 planes of
+// 1.28 ms, 8192^2 57 and 38 us of 13.5 ms.
+constexpr int kFixRecords = 7000;
 // Column-tile width of the LDS path's intermediate planes.
 constexpr int kTile = 1 << kTileLog2;
 

@@ -43,6 +43,57 @@ def test_crowded_uv_data(nx, ny, nrow, eps):
     assert err < BAR
 
 
+# integer sums (rows of 4096, row parts of 16384), whose crowded blocks of rows run in
+# FP64: all rows crowded, or a crowd among rows that are not; strips and layers of bins
+# of other sizes, several batches of planes
+@pytest.mark.parametrize("nx,ny,nrow,crowd,eps,tuning", [
+    (128, 2048, 60_000, 60_000, 1e-6, (0, 0, 0, 0)), (127, 2047, 40_000, 40_000, 1e-9, (0, 0, 0, 0)),
+    (64, 8192, 30_000, 30_000, 1e-6, (0, 0, 0, 0)), (63, 8191, 30_000, 30_000, 1e-9, (0, 0, 0, 0)),
+    (256, 2048, 60_000, 40_000, 1e-6, (0, 3, 5, 1)), (256, 8192, 60_000, 40_000, 1e-6, (0, 5, 0, 3)),
+    (2048, 2048, 200_000, 50_000, 1e-6, (0, 0, 0, 0))])
+def test_crowded_blocks_of_integer_rows(nx, ny, nrow, crowd, eps, tuning):
+    from curig_amd import _lib as L
+
+    fov = 2.0
+    uvw, vis, f0 = _crowded(nrow, 4, fov, nx + ny)
+    uvw[crowd:, :2] *= np.array([nx, ny]) / 4 * 0.95
+    order = np.random.default_rng(1).permutation(nrow)
+    uvw, vis = uvw[order], vis[order]
+    want = gpu_ms2dirty(uvw, vis, None, nx, ny, fov, f0, eps)
+    lib = L.load()
+    assert lib.curig_set_tuning(*tuning) == 0
+    try:
+        err = O.l2error(want, gpu_f32(True, uvw, vis, None, nx, ny, fov, f0, eps))
+    finally:
+        lib.curig_set_tuning(0, 0, 0, 0)
+    say(f"[crowded blocks] {nx}x{ny} rows {nrow} crowd {crowd} eps {eps} tuning {tuning}: {err:.2e}")
+    assert err < BAR
+
+
+def test_crowded_channels_replayed():
+    """One channel of two crowded (the other's rows flagged), replayed as a graph."""
+    import torch
+
+    from curig_amd import _lib as L
+
+    nx, ny, nrow, fov, eps = 128, 2048, 60_000, 2.0, 1e-6
+    uvw, vis, f0 = _crowded(nrow, 4, fov, 5)
+    uvw[50_000:, :2] *= np.array([nx, ny]) / 4 * 0.9
+    freq, ms = np.array([f0, 1.02 * f0]), np.stack([vis, vis[::-1]], axis=1)
+    flag = np.zeros((nrow, 2), dtype=np.uint8)
+    flag[:50_000, 1] = 1
+    d_uvw, d_ms, d_flag = torch.from_numpy(uvw).cuda(), torch.from_numpy(np.ascontiguousarray(ms)).cuda(), torch.from_numpy(flag).cuda()
+    want = [gpu_ms2dirty(uvw[flag[:, c] == 0], ms[flag[:, c] == 0, c], None, nx, ny, fov, freq[c], eps) for c in range(2)]
+    for _ in range(3):
+        out = torch.full((2, nx, ny), float("nan"), dtype=torch.complex64, device="cuda")
+        L.check(L.load().curig_ms2dirty_multi_dev(nrow, 2, nx, ny, fov, freq, d_uvw.data_ptr(), d_ms.data_ptr(), None,
+                                                  d_flag.data_ptr(), out.data_ptr(), 1, eps, 2.0, -1, 1,
+                                                  torch.cuda.current_stream().cuda_stream))
+        errs = [O.l2error(w, g) for w, g in zip(want, out.cpu().numpy())]
+        say(f"[crowded channels] {errs}")
+        assert max(errs) < BAR
+
+
 def test_crowded_uv_data_without_allocation():
     """Whole rows of 8192 in components: the entry point of the smallest working set only."""
     import torch
