@@ -110,7 +110,7 @@ struct Geom {
   int ncheb;          // terms of its Chebyshev series, which holds for |z| <= zcheb; 0: none; -1: none,
                       // and the correction tables computed on the host
   double zcheb;
-  // pruned LDS FFT path (power-of-two grids); fft_lds == 0 selects rocFFT
+  // pruned LDS FFT path (powers of two, and mixed radix: mix); fft_lds == 0 selects rocFFT
   int fft_lds;
   const uint64_t *occ; // [P] planes' occupied row blocks: bit b for rows b << occ_lg .. (null: all taken as
   int occ_lg;          // occupied); rows of the other blocks are neither written to nor read from H

@@ -4,23 +4,25 @@
 //   ms2dirty  prep: w range -> plan; bin rows by (w-plane batch, grid tile of the
 //             kernel's first cell); counting sort into 32/56-byte records
 //             for each batch of Pb w planes:
-//               power-of-two grids (LDS path): spread + row FFT -> column-tiled
-//               planes; column FFT fused with the w-accumulation (FP64)
+//               LDS path (axes that are powers of two or 2^a 3^b 5^c and fit a
+//               workgroup): spread + row FFT -> column-tiled planes; column FFT
+//               fused with the w-accumulation (FP64)
 //               other grids: tile-owner spread into whole planes, rocFFT,
 //               w-accumulation
 //             epilogue: ES / w corrections, / n
 //   dirty2ms  prologue: corrections, / n; for each batch: w-fill + inverse
 //             column FFT, inverse row FFT fused with the interpolation into
-//             FP64 per-row accumulators (other grids: w-fill, rocFFT,
-//             interpolation); finalize: weight and e^{-i D w}, scatter to row order.
+//             FP64 per-row accumulators, or written out as rows that dense
+//             records are gathered from (other grids: w-fill, rocFFT,
+//             interpolation); finalize: weight and e^{-i D w}, in row order.
 //
 // Mathematically this is the reference's operator (src/astro/ra_exec.cu:141-436):
 // same grid sizes, w-plane count and scaling (set_nhg_type3), kernel and
 // correction factors; the full nf3 x nf2 x nf1 grid of the reference is never
 // materialised (only Pb planes at a time), and the kernel is normalised to peak 1
 // (its Fourier-series factors carry the same normalisation, so it cancels).
-// The kernels live in kern_prep.hip, kern_plane.hip and kern_lds_*.hip; this
-// file queues them through the launchers of kernels.h.
+// The kernels live in kern_prep.hip, kern_plane.hip and kern_{lds,rowreg,mix}_*.hip;
+// this file queues them through the launchers of kernels.h.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -332,9 +334,9 @@ static void plan_columns(Geom &g, size_t cs, size_t lds_max, bool compact) {
     // the inverse pass in short launches' worth of planes: its workgroups, one
     // column each, share lines of H in fours, and the further they drift apart
     // over the planes the more partial lines the L2 writes back (8192^2, 32
-    // planes: 19.9 ms walking all planes, 17.7, 13.9 and 16.1 ms in chunks of 8,
-    // 4 and 2; a chunk's setup costs about one plane; FP64 stores whole 64-byte
-    // pieces)
+    // planes, 63% of the rows occupied: 15.4 ms walking all planes, 13.7 in chunks
+    // of 8 and of 4; all rows: 22.0, 19.4 and 16.6 ms; chunks of 2 lose, a chunk's
+    // setup costs about one plane; FP64 stores whole 64-byte pieces)
     if (cs == 8) g.pch_inv = std::min(4, g.Pb);
     g.lds_col_bytes = (int)colreg_lds_bytes(cs);
     return;
@@ -393,9 +395,10 @@ static int mixed_threads(int n, int count, int max_threads, int min_threads) {
 // Against the full-plane path (tile spread, rocFFT, w-sum over whole planes):
 // 1500 x 1100 FP32 ms2dirty 19.6 -> 10.5 ms, 3000 x 2500 FP64 dirty2ms 185 ->
 // 47 ms, 512^2 FP64 at upsampling 1.25 (both directions, host arrays) 4.0 -> 2.3
-// ms, so the full planes remain for axes that do not fit (FP64 beyond about 9000
-// points), kernels wider than 16, and grids of few rows (a one-dimensional
-// transform's 2 kw rows: the row workgroups would hold all its points).
+// ms, so the full planes remain for axes beyond 16 points for each thread of the
+// largest workgroup (FP64 8192 points, FP32 16384), kernels wider than 16, and grids
+// of few rows (a one-dimensional transform's 2 kw rows: the row workgroups would hold
+// all its points).
 static void plan_mixed(Geom &g, size_t cs, size_t lds_max) {
   // FP32 with the image beyond half the grid keeps the full planes: its
   // corrections amplify rounding up to 1e-4 of the result, and another
@@ -862,9 +865,10 @@ int batch_fft(int dev, const Geom &g, int nb, int sign, void *grid, hipStream_t 
   return kOk;
 }
 
-// Phase 2 (one wait): allocate the working set for all problems, upload the
-// correction tables and twiddles, create FFT plans and kernel attributes, so
-// that phase 3 queues kernels only.
+// Phase 2: allocate the working set for all problems, compute the correction
+// tables, create FFT plans and kernel attributes, so that phase 3 queues kernels
+// only (a wait where the sizes change and twiddles are uploaded, and for tables and
+// polynomials from the host).
 template <typename T>
 int reserve(const std::vector<ChanPlan> &cps, const Problem *pbs, const QuadRule &rule, bool to_image, int dev,
             hipStream_t st, Bufs &b) {

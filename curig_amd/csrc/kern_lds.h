@@ -1,7 +1,9 @@
-// Pruned LDS FFT path (power-of-two grids): the row and column kernels of
-// both directions, included by one source per precision and kernel group
-// (kern_lds_{spread,interp,cols}_{f32,f64}.hip), each of which instantiates
-// its launchers.
+// Pruned LDS FFT path, power-of-two grids: the kernels of long rows (4096 points
+// and row parts) and of columns of 16384, and what all row and column kernels of
+// the path share (other rows: kern_rowreg.h, columns: kern_cols.h, mixed-radix
+// axes: kern_mix.h).  Included by one source per precision and kernel group
+// (kern_lds_{spread,interp,cols}_{f32,f64}.hip), each of which instantiates its
+// launchers.
 #pragma once
 #include <type_traits>
 
@@ -11,7 +13,7 @@
 namespace curig {
 
 // --------------------------------------------------------------------------
-// pruned LDS FFT path (power-of-two grids)
+// pruned LDS FFT path
 //
 // ms2dirty per batch of planes: (1) one workgroup per grid row of a plane
 // spreads the row's visibilities into LDS, runs the row FFT (length nf1) and
@@ -1411,10 +1413,14 @@ int allow_spread_rows(const Geom &g) {
 }
 
 // rows (rsplit 0) or row parts (rsplit kRowSplit) of 4096 points (FP64:
-// 173 VGPRs at the two workgroups per CU that its LDS allows)
+// up to 223 VGPRs at the two workgroups per CU that its LDS allows)
 template <typename T> inline bool interp_planes(const Geom &g) {
   return (g.rsplit == 0 && g.rpw == 1 && g.nf1 == 4096) || (g.rsplit > 1 && g.nf1 / g.rsplit == 4096);
 }
+
+// whether plans have parts of other lengths (FP32: quarters of 16384 and halves of
+// 8192 are 4096, other builds' parts are not)
+template <typename T> constexpr bool other_parts() { return sizeof(T) == 8 || kRowSplit != 4; }
 
 // dirty2ms, one batch on the LDS path: inverse row FFT fused with the interpolation
 template <typename T>
@@ -1438,15 +1444,15 @@ void lds_row_interp(const Rec<T> *recs, const T *taps, const int *off, const cpx
       with_split<T>(g.rsplit, go);
     return;
   }
-  if (g.rsplit > 1) {
-    // parts of other lengths (FP64 rows of 8192): kRowSplit ways
+  // parts of other lengths (FP64 rows of 8192): kRowSplit ways
+  if constexpr (other_parts<T>()) {
+    if (g.rsplit <= 1) return;
     const dim3 grd(kRowSplit * g.nf2, nb);
     const int nt = g.nf1 / (16 * kRowSplit), lb = g.lds_rowp_bytes;
     if (g.kw <= 8)
       row_ifft_interp_part_kernel<T, 16, 8, kRowSplit><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, -1);
     else
       row_ifft_interp_part_kernel<T, 16, 16, kRowSplit><<<grd, nt, lb, st>>>(H, recs, taps, off, vacc, tw1, g, p0, -1);
-    return;
   }
 }
 
@@ -1465,7 +1471,8 @@ int allow_row_interp(const Geom &g) {
     else
       with_split<T>(g.rsplit, go);
     CURIG_TRY(ier);
-  } else if (g.rsplit > 1) {
+  } else if constexpr (other_parts<T>()) {
+    if (g.rsplit <= 1) return kOk;
     CURIG_TRY((allow_lds(row_ifft_interp_part_kernel<T, 16, 8, kRowSplit>, g.lds_rowp_bytes)));
     CURIG_TRY((allow_lds(row_ifft_interp_part_kernel<T, 16, 16, kRowSplit>, g.lds_rowp_bytes)));
   }

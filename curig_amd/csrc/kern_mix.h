@@ -415,16 +415,19 @@ template <typename T> inline int mix_col_lds(const Geom &g, int cpw) {
 // f(cells per thread 8 or 16, threads at most 512 or 1024)
 template <typename T, typename F> inline void with_cells(int cells, int nt, F f) {
   using std::integral_constant;
-  if (sizeof(T) == 4 && nt > 512) {
-    if (cells <= 8)
-      f(integral_constant<int, 8>(), integral_constant<int, 1024>());
-    else
-      f(integral_constant<int, 16>(), integral_constant<int, 1024>());
-  } else if (cells <= 8) {
-    f(integral_constant<int, 8>(), integral_constant<int, 512>());
-  } else {
-    f(integral_constant<int, 16>(), integral_constant<int, 512>());
+  if constexpr (sizeof(T) == 4) {
+    if (nt > 512) {
+      if (cells <= 8)
+        f(integral_constant<int, 8>(), integral_constant<int, 1024>());
+      else
+        f(integral_constant<int, 16>(), integral_constant<int, 1024>());
+      return;
+    }
   }
+  if (cells <= 8)
+    f(integral_constant<int, 8>(), integral_constant<int, 512>());
+  else
+    f(integral_constant<int, 16>(), integral_constant<int, 512>());
 }
 inline int mix_cells(int cpw, int N2, int nt) { return (cpw * N2 + nt - 1) / nt; }
 

@@ -1,7 +1,7 @@
-// Full-plane path (grids that are not powers of two: tile-owner spread into
-// whole planes, rocFFT, w-accumulation / w-fill, interpolation), the
-// correction epilogue / prologues shared with the LDS path, the finalize
-// scatter and the FP64 direct sums.
+// Full-plane path (grids that the LDS path does not take: tile-owner spread into
+// whole planes, rocFFT, w-accumulation / w-fill, interpolation), the correction
+// tables, epilogue and prologues shared with the LDS path, the finalize pass and the
+// FP64 direct sums.
 #include "dev_common.h"
 
 namespace curig {

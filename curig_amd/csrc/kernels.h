@@ -46,7 +46,7 @@ struct ChanPlan {
 // Device pointers of one call's working set (slots of the per-device workspace).
 struct Bufs {
   int dev = 0;
-  double *tabs = nullptr;  // fk1 [nf1/2+1] | fk2 [nf2/2+1] | quadrature nodes | weights
+  double *tabs = nullptr;  // fk1 [nf1/2+1] | fk2 [nf2/2+1] | quadrature nodes | weights | Chebyshev coefficients
   int *hist = nullptr, *off = nullptr, *bsum = nullptr, *slot = nullptr;
   int2 *binrank = nullptr;
   void *recs = nullptr, *grid = nullptr, *H = nullptr;

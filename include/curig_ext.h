@@ -153,7 +153,7 @@ int curig_kernel_horner(double epsilon, double sigma, int precision, int *deg, d
 int curig_gauss_legendre(int n, double *x, double *w);
 
 /* Tuning of later calls (0 = default): tile width / height of the bins (for
- * power-of-two grids only the height is used: bins are full-width row strips),
+ * the LDS FFT path only the height is used: bins are full-width row strips),
  * w planes per batch (FFT batch) and w planes per bin layer.  The autotuner
  * (curig_amd.autotune) sets these. */
 int curig_set_tuning(int tile_x, int tile_y, int planes_per_batch, int planes_per_bin);
