@@ -407,7 +407,8 @@ __global__ void __launch_bounds__(MT) col_inv_mix_kernel(const cpx<T> *__restric
 // --------------------------------------------------------------------------
 template <typename T> inline int mix_row_lds(const Geom &g, bool spread) {
   const int cells = g.rpw * fftm::seq_stride(g.nf1);
-  return cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>)) + fftc::twiddle_entries(g.nf1) * (int)sizeof(cpx<T>);
+  return cells * (int)(spread && g.acc64 ? sizeof(double2) : sizeof(cpx<T>)) +
+         fftc::twiddle_entries(g.nf1) * (int)sizeof(cpx<T>);
 }
 template <typename T> inline int mix_col_lds(const Geom &g, int cpw) {
   return (int)sizeof(cpx<T>) * (cpw * fftm::seq_stride(g.nf2) + fftc::twiddle_entries(g.nf2));

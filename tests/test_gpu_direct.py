@@ -66,8 +66,9 @@ def test_rows_of_8192_by_density(nx, ny, nrow, eps, visits, rsplit):
 
 def test_mixed_radix_rows_without_records_in_fp64():
     """Five visibilities and mixed-radix grids of an upsampling of 2, at FP64's own bar."""
-    for nx, ny, nrow, eps, wmax in ((300, 250, 5, 1e-6, 2000.0), (75, 1125, 3000, 1e-6, 300.0), (3000, 40, 3000, 1e-6, 200.0),
-                                    (100, 100, 3000, 1e-6, 9000.0)):
+    eps = 1e-6
+    for nx, ny, nrow, wmax in ((300, 250, 5, 2000.0), (75, 1125, 3000, 300.0), (3000, 40, 3000, 200.0),
+                               (100, 100, 3000, 9000.0)):
         uvw, vis, wgt, img, f0 = _case(nrow, nx, ny, 2.0, wmax, 3)
         e1, e2 = _both_paths("fp64", uvw, vis, wgt, img, nx, ny, 2.0, f0, eps)
         say(f"[mixed radix, FP64] {nx}x{ny} rows {nrow}: ms2dirty {e1:.2e}, dirty2ms {e2:.2e}")

@@ -82,7 +82,7 @@ def test_crowded_channels_replayed():
     freq, ms = np.array([f0, 1.02 * f0]), np.stack([vis, vis[::-1]], axis=1)
     flag = np.zeros((nrow, 2), dtype=np.uint8)
     flag[:50_000, 1] = 1
-    d_uvw, d_ms, d_flag = torch.from_numpy(uvw).cuda(), torch.from_numpy(np.ascontiguousarray(ms)).cuda(), torch.from_numpy(flag).cuda()
+    d_uvw, d_ms, d_flag = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (uvw, ms, flag))
     want = [gpu_ms2dirty(uvw[flag[:, c] == 0], ms[flag[:, c] == 0, c], None, nx, ny, fov, freq[c], eps) for c in range(2)]
     for _ in range(3):
         out = torch.full((2, nx, ny), float("nan"), dtype=torch.complex64, device="cuda")
